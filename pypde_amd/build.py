@@ -18,6 +18,8 @@ ROCM = os.environ.get("ROCM_PATH", "/opt/rocm")
 
 EMBED = [("PRELUDE_SRC", os.path.join(PKG, "systems", "pde_prelude.h")),
          ("COMMON_SRC", os.path.join(CSRC, "kernels", "ader_common.h")),
+         ("WIDE_SRC", os.path.join(CSRC, "kernels", "ader_wide.h")),
+         ("WIDE_PRED_SRC", os.path.join(CSRC, "kernels", "ader_wide_predictor.h")),
          ("KERNELS_SRC", os.path.join(CSRC, "kernels", "ader_kernels.h")),
          ("STEP_SRC", os.path.join(CSRC, "kernels", "ader_step.h")),
          ("MLP_SRC", os.path.join(CSRC, "kernels", "mlp_train.h")),

@@ -269,8 +269,43 @@ DEV void cell_deriv(const double (&w)[ND][V], int idx, double rdx, double* out) 
 // eigenvalue work per lane.  Both lanes form the cell's (l_0 / dX_0) + (l_1 /
 // dX_1) from the pair's two terms.  The host launches DT_LANES * nwc threads.
 constexpr bool DT_PAIR = (D == 2) && (V <= 5) && !PDE_SECOND;
-constexpr int DT_LANES = DT_PAIR ? 2 : 1;
+constexpr int DT_LANES = V > 8 ? 64 : DT_PAIR ? 2 : 1;
 
+#if PDE_V > 8
+// One wavefront per w-cell: the cell's mean (lane v takes variable v), then
+// one eigenvalue problem per direction over the wavefront.
+DEV void dt_body(const double* __restrict__ wh, StepState* st, const Geom& g, const Blk& b) {
+  __shared__ WideMat wm[WIDE_WAVES];
+  const int lane = threadIdx.x & 63;
+  WideMat& W = wm[threadIdx.x >> 6];
+  const long c = (long)b.x * WIDE_WAVES + (threadIdx.x >> 6);
+  double sum = 0.0;
+  if (c < g.nwc) {
+    if (lane < V) {
+      double acc = T_WP[0] * wh[(long)lane * g.nwc + c];
+#pragma unroll
+      for (int idx = 1; idx < ND; idx++)
+        acc = dfma(T_WP[idx], wh[(long)(idx * V + lane) * g.nwc + c], acc);
+      W.P[0][lane] = acc;
+    }
+    wide_sync();
+    double q[V], dq[D * V], f0[V];
+#pragma unroll
+    for (int v = 0; v < V; v++) q[v] = W.P[0][v];
+#pragma unroll
+    for (int i = 0; i < D * V; i++) dq[i] = 0.0;
+    static_for<0, D>([&](auto dc) {
+      constexpr int d = decltype(dc)::value;
+      const double lam = wide_max_abs_eigs(W, q, dq, d, lane, f0);
+      sum = sum + lam / g.dX[d];
+    });
+    if (!(sum > 0.0)) sum = 0.0;
+  }
+  if (lane == 0 && sum > 0.0)
+    atomicMax(&st->pstat[b.x & 63][8], (unsigned long long)__double_as_longlong(sum));
+  if (last_workgroup(&st->dt_ticket, b.n)) dt_finalize(st);
+}
+#else
 DEV void dt_body(const double* __restrict__ wh, StepState* st, const Geom& g, const Blk& b) {
   const long item = (long)b.x * 256 + threadIdx.x;
   const long c = DT_PAIR ? (item >> 1) : item;
@@ -343,6 +378,7 @@ DEV void dt_body(const double* __restrict__ wh, StepState* st, const Geom& g, co
   // the last workgroup to finish takes dt from the 64 slots
   if (last_workgroup(&st->dt_ticket, b.n)) dt_finalize(st);
 }
+#endif
 
 extern "C" __global__ void __launch_bounds__(256)
 k_dt(const double* __restrict__ wh, StepState* st, Geom g) {
@@ -380,6 +416,22 @@ DEV void dt_finalize(StepState* st) {
 extern "C" __global__ void __launch_bounds__(256)
 k_eig_batch(const double* __restrict__ A, const double* __restrict__ x, double* __restrict__ out,
             long n, int which) {
+#if PDE_V > 8
+  // a workgroup's 256 matrices, 64 in turn per wavefront (which is 0: Roe and
+  // Osher stop at V = 8)
+  __shared__ WideMat wm[WIDE_WAVES];
+  const int lane = threadIdx.x & 63;
+  const long i0 = (long)blockIdx.x * 256 + (threadIdx.x & ~63u);
+  for (long k = i0; k < i0 + 64 && k < n; k++) {
+    double col[V];
+#pragma unroll
+    for (int r = 0; r < V; r++) col[r] = lane < V ? A[k * V * V + r * V + lane] : 0.0;
+    const double lam = wide_max_abs_eig(wm[threadIdx.x >> 6], col, lane);
+    if (lane == 0) out[k] = lam;
+  }
+  (void)x;
+  (void)which;
+#else
   const long i = (long)blockIdx.x * 256 + threadIdx.x;
   if (i >= n) return;
   double H[V * V];
@@ -398,5 +450,6 @@ k_eig_batch(const double* __restrict__ A, const double* __restrict__ x, double* 
   for (int v = 0; v < V; v++) out[i * V + v] = y[v];
 #else
   (void)x;
+#endif
 #endif
 }

@@ -598,6 +598,7 @@ DEV bool newton_node(const NodeCtx& c, const double (&q)[N][V], double (&G)[N][V
 }
 #endif
 
+#if PDE_V <= 8  // above, ader_wide_predictor.h
 // Persistent, work-queued: each wavefront claims cells from st->qhead (reset
 // by k_dt's last workgroup every step), iterates its CPW slots, and as soon as a slot's
 // cell has converged writes that cell's outputs and refills the slot with the
@@ -1236,6 +1237,8 @@ k_predictor_static2(const double* __restrict__ wh, const double* __restrict__ gu
                         hw_blk());
 }
 
+#endif  // PDE_V <= 8
+
 #if PDE_MIXED
 // ---------------------------------------------- mixed precision: FP32 phase
 // The predictor's space-time iteration with its contractions (spatial
@@ -1482,6 +1485,85 @@ DEV void face_cells(const Geom& g, long f, long* wl, long* wr) {
 // (fluxes.cpp:72-101), Roe or Osher (fluxes.cpp:20-70), the viscous term
 // (fluxes.cpp:96-100) and the non-conservative path integral Bint
 // (fluxes.cpp:103-116), from the two cells' face traces.
+#if PDE_V > 8
+// Above V = 8 (Rusanov, first-order F): one face point per workgroup of two
+// wavefronts, one for each side's wave speed and F.
+template <int d, int BS>
+DEV void flux_dir(const double* __restrict__ tr, double* __restrict__ ff, double* __restrict__ fb,
+                  const StepState* st, const Geom& g, const double* __restrict__ trd,
+                  const Blk& b) {
+  static_assert(BS == 128, "one wavefront per side");
+  (void)st;
+  (void)trd;
+  const long nf = g.nf[d];
+  const long item = b.x;
+  const long f = item % nf;
+  const int j = (int)((item / nf) % ND1);
+  const int t = (int)(item / (nf * ND1));
+  long wl, wr;
+  face_cells<d>(g, f, &wl, &wr);
+  const int lane = threadIdx.x & 63, side = threadIdx.x >> 6;
+  const double* const trL = tr + (long)((((d * 2 + 1) * N + t) * ND1 + j) * V) * g.nwc + wl;
+  const double* const trR = tr + (long)((((d * 2 + 0) * N + t) * ND1 + j) * V) * g.nwc + wr;
+  const long o = (long)((t * ND1 + j) * V) * nf + f;
+  __shared__ WideMat wm[2];
+#if PDE_USE_F
+  {
+    __shared__ double fs[2][V], lam[2];
+    double q[V], dq[D * V], f0[V];
+    const double* const src = side ? trR : trL;
+#pragma unroll
+    for (int v = 0; v < V; v++) q[v] = src[(long)v * g.nwc];
+#pragma unroll
+    for (int i = 0; i < D * V; i++) dq[i] = 0.0;
+    const double l = wide_max_abs_eigs(wm[side], q, dq, d, lane, f0);
+    if (lane == 0) {
+      lam[side] = l;
+#pragma unroll
+      for (int v = 0; v < V; v++) fs[side][v] = f0[v];
+    }
+    __syncthreads();
+    if (threadIdx.x < V) {
+      const int v = threadIdx.x;
+      const double s = dmax(lam[0], lam[1]);
+      ff[o + (long)v * nf] =
+          s * (trL[(long)v * g.nwc] - trR[(long)v * g.nwc]) + (fs[0][v] + fs[1][v]);
+    }
+  }
+#endif
+#if PDE_USE_B
+  if (side == 0) {
+    // lane v forms row v of the path average of B (written by lane 0 over wm)
+    // and its product with Dq
+    double Dq[V], qL[V], Mx[V], q[V];
+    double* const bm = &wm[0].P[0][0];
+    const int row = lane < V ? lane : 0;
+#pragma unroll
+    for (int v = 0; v < V; v++) {
+      qL[v] = trL[(long)v * g.nwc];
+      Dq[v] = trR[(long)v * g.nwc] - qL[v];
+    }
+#pragma unroll
+    for (int i = 0; i < N; i++) {
+#pragma unroll
+      for (int v = 0; v < V; v++) q[v] = dfma(T_X[i], Dq[v], qL[v]);
+      wide_sync();
+      if (lane == 0) B(bm, q, d);
+      wide_sync();
+#pragma unroll
+      for (int k = 0; k < V; k++) {
+        const double e = bm[row * V + k];
+        Mx[k] = (i == 0) ? T_W[0] * e : dfma(T_W[i], e, Mx[k]);
+      }
+    }
+    double acc = Mx[0] * Dq[0];
+#pragma unroll
+    for (int k = 1; k < V; k++) acc = dfma(Mx[k], Dq[k], acc);
+    if (lane < V) fb[o + (long)lane * nf] = acc;
+  }
+#endif
+}
+#else
 template <int d, int BS = 256>
 DEV void flux_dir(const double* __restrict__ tr, double* __restrict__ ff, double* __restrict__ fb,
                   const StepState* st, const Geom& g, const double* __restrict__ trd,
@@ -1618,8 +1700,11 @@ DEV void flux_dir(const double* __restrict__ tr, double* __restrict__ ff, double
 #endif
 }
 
+#endif
+
 // Workgroup sizes 256 (k_flux0, k_flux1), 128 and 64 (..._128, ..._64): the
 // autotuner picks one per problem; every face point's arithmetic is the same.
+// Above V = 8 only k_flux0 and k_flux1 exist, of 128 threads.
 #define PYPDE_FLUX_KERNEL(NAME, DIR, BS)                                                       \
   extern "C" __global__ void __launch_bounds__(BS)                                             \
   NAME(const double* __restrict__ tr, double* __restrict__ ff, double* __restrict__ fb,        \
@@ -1627,13 +1712,18 @@ DEV void flux_dir(const double* __restrict__ tr, double* __restrict__ ff, double
     if (st->done) return;                                                                      \
     flux_dir<DIR, BS>(tr, ff, fb, st, g, trd, hw_blk());                                       \
   }
-PYPDE_FLUX_KERNEL(k_flux0, 0, 256)
+constexpr int FLUX_BS0 = V > 8 ? 128 : 256;
+PYPDE_FLUX_KERNEL(k_flux0, 0, FLUX_BS0)
+#if PDE_D >= 2
+PYPDE_FLUX_KERNEL(k_flux1, 1, FLUX_BS0)
+#endif
+#if PDE_V <= 8
 PYPDE_FLUX_KERNEL(k_flux0_128, 0, 128)
 PYPDE_FLUX_KERNEL(k_flux0_64, 0, 64)
 #if PDE_D >= 2
-PYPDE_FLUX_KERNEL(k_flux1, 1, 256)
 PYPDE_FLUX_KERNEL(k_flux1_128, 1, 128)
 PYPDE_FLUX_KERNEL(k_flux1_64, 1, 64)
+#endif
 #endif
 
 // ------------------------------------------------------------- corrector
@@ -2203,6 +2293,7 @@ k_dt_b(const Member* ms, const BlkMap* map, int nm) {
   dt_body(M.wh, M.st, M.g, b);
 }
 
+#if PDE_V <= 8
 extern "C" __global__ void __launch_bounds__(64)
 k_predictor_static_b(const Member* ms, const BlkMap* map, int nm, double newton_tol,
                      int newton_maxit) {
@@ -2246,6 +2337,7 @@ k_predictor_hot_b(const Member* ms, const BlkMap* map, int nm, double newton_tol
 }
 
 #endif
+#endif  // PDE_V <= 8
 
 #define PYPDE_FLUX_BATCH(NAME, DIR, BS)                                                        \
   extern "C" __global__ void __launch_bounds__(BS)                                             \
@@ -2254,13 +2346,17 @@ k_predictor_hot_b(const Member* ms, const BlkMap* map, int nm, double newton_tol
     if (M.st->done) return;                                                                    \
     flux_dir<DIR, BS>(M.tr, M.ff[DIR], M.fb[DIR], M.st, M.g, M.trd, b);                        \
   }
-PYPDE_FLUX_BATCH(k_flux0_b, 0, 256)
+PYPDE_FLUX_BATCH(k_flux0_b, 0, FLUX_BS0)
+#if PDE_D >= 2
+PYPDE_FLUX_BATCH(k_flux1_b, 1, FLUX_BS0)
+#endif
+#if PDE_V <= 8
 PYPDE_FLUX_BATCH(k_flux0_128_b, 0, 128)
 PYPDE_FLUX_BATCH(k_flux0_64_b, 0, 64)
 #if PDE_D >= 2
-PYPDE_FLUX_BATCH(k_flux1_b, 1, 256)
 PYPDE_FLUX_BATCH(k_flux1_128_b, 1, 128)
 PYPDE_FLUX_BATCH(k_flux1_64_b, 1, 64)
+#endif
 #endif
 
 extern "C" __global__ void __launch_bounds__(256)

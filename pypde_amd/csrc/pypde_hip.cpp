@@ -31,9 +31,10 @@
 
 namespace {
 
-#include "kernels_embed.inc"  // PRELUDE_SRC, COMMON_SRC, KERNELS_SRC, STEP_SRC
+#include "kernels_embed.inc"  // PRELUDE_SRC, COMMON_SRC, WIDE_SRC, KERNELS_SRC, STEP_SRC
 
 constexpr int MAXV = 17;
+constexpr int WIDE_V = 8;  // above this V the kernels of ader_wide.h and ader_wide_predictor.h
 thread_local std::string g_err;
 
 int fail(int code, const char* fmt, ...) {
@@ -169,7 +170,9 @@ std::string full_source(const Spec& s, const pypde::Tables& T) {
   if (s.mixed)  // the same physics once more, in FP32, for the mixed predictor's first phase
     o << REAL32_SRC << "\nnamespace f32 {\n#define double R\n#line 1 \"system (FP32)\"\n" << s.src
       << "\n#undef double\n}  // namespace f32\n";
+  if (s.V > WIDE_V) o << WIDE_SRC << "\n";
   o << KERNELS_SRC << "\n" << STEP_SRC << "\n";
+  if (s.V > WIDE_V) o << WIDE_PRED_SRC << "\n";
   return o.str();
 }
 
@@ -355,7 +358,7 @@ struct pypde_ctx {
   Spec spec;
   pypde_options opts;
   Geom g;
-  int D, N, V, ND, NT, CPW;
+  int D, N, V, ND, NT, CPW;  // CPW: cells per predictor workgroup (one wavefront)
   hipModule_t mod = nullptr;
   uint64_t code_key = 0;  // the code object's cache key (kernel source and options)
   hipFunction_t fn[K_COUNT] = {};
@@ -438,6 +441,9 @@ int load_module(pypde_ctx* c, const std::vector<char>& code, uint64_t key, hipMo
   for (int k = 0; k < K_COUNT; k++) {
     fn[k] = nullptr;
     bool optional = ((k == K_FLUX1 || k == K_FLUX1_128 || k == K_FLUX1_64) && c->D < 2) ||
+                    ((k == K_FLUX0_128 || k == K_FLUX0_64 || k == K_FLUX1_128 ||
+                      k == K_FLUX1_64) && c->V > WIDE_V) ||
+                    ((k == K_PRED || k == K_PRED_STATIC2) && c->V > WIDE_V) ||
                     k == K_MLPGUESS || k == K_MLPPACK || (k == K_PRED32 && !c->spec.mixed) ||
                     k == K_PRED_COLD || k == K_PRED_HOT || k == K_PRED_COLD3 || k >= K_B_WENO;
     if (hipModuleGetFunction(&fn[k], *mod, kernel_names[k]) != hipSuccess) {
@@ -458,6 +464,15 @@ int launch(pypde_ctx* c, int k, dim3 grid, dim3 block, std::vector<void*>& args)
 }
 
 long cdiv(long a, long b) { return (a + b - 1) / b; }
+
+// Face-flux launch of one direction: variants and threads per workgroup, and
+// workgroups for `items` face points (above WIDE_V one face point per
+// workgroup of 128 threads).
+int flux_variants(int V) { return V > WIDE_V ? 1 : N_FLUX_V; }
+int flux_threads(int V, int variant) { return V > WIDE_V ? 128 : FLUX_BS[variant]; }
+long flux_blocks(int V, int variant, long items) {
+  return V > WIDE_V ? items : cdiv(items, FLUX_BS[variant]);
+}
 
 // Callers built against the older, shorter pypde_stats leave out the node
 // counters; struct_size says which layout the caller has.
@@ -549,7 +564,7 @@ int enqueue_step(pypde_ctx* c, bool guess_now, std::vector<hipEvent_t>* evs) {
     float tol32 = (float)c->opts.mixed_tol;
     int maxit32 = c->opts.mixed_maxit;
     std::vector<void*> a = {&w, &gin, &gout, &st, &g, &tol32, &maxit32};
-    if ((rc = launch(c, K_PRED32, dim3((unsigned)cdiv(g.nwc, c->CPW)), dim3(64), a))) return rc;
+    if ((rc = launch(c, K_PRED32, dim3((unsigned)cdiv(g.nwc, 64 / c->ND)), dim3(64), a))) return rc;
   }
   mark();
   {
@@ -584,8 +599,9 @@ int enqueue_step(pypde_ctx* c, bool guess_now, std::vector<hipEvent_t>* evs) {
     const double* td = c->trd;
     std::vector<void*> a = {&t, &f, &b, &st, &g, &td};
     long items = g.nf[d] * c->N * (c->ND / c->N);
-    const int bs = FLUX_BS[c->tune.flux];
-    if ((rc = launch(c, FLUX_KID[d][c->tune.flux], dim3((unsigned)cdiv(items, bs)), dim3(bs), a)))
+    if ((rc = launch(c, FLUX_KID[d][c->tune.flux],
+                     dim3((unsigned)flux_blocks(c->V, c->tune.flux, items)),
+                     dim3(flux_threads(c->V, c->tune.flux)), a)))
       return rc;
     mark();
   }
@@ -790,8 +806,9 @@ static pypde_ctx* create_ctx(const char* src, bool useF, bool useB, bool useS, c
   c->ND = 1;
   for (int d = 0; d < ndim; d++) c->ND *= N;
   c->NT = c->ND * N;
-  c->CPW = 64 / c->ND;
-  c->dt_lanes = (ndim == 2 && V <= 5 && !secondOrder) ? 2 : 1;  // DT_PAIR in ader_kernels.h
+  c->CPW = V > WIDE_V ? 1 : 64 / c->ND;
+  // DT_LANES in ader_kernels.h
+  c->dt_lanes = V > WIDE_V ? 64 : (ndim == 2 && V <= 5 && !secondOrder) ? 2 : 1;
   c->device = opts.device;
   // Predictor schedule: the autotuner picks among the static one (one
   // wavefront per group of CPW cells), the persistent work-queued kernel and
@@ -802,6 +819,11 @@ static pypde_ctx* create_ctx(const char* src, bool useF, bool useB, bool useS, c
     c->pred_w2 = strcmp(e, "static2") == 0;
     c->pred_split = strcmp(e, "split") == 0;
     c->pred_fixed = true;
+  }
+  // above WIDE_V there is one predictor kernel
+  if (V > WIDE_V) {
+    c->pred_static = c->pred_fixed = true;
+    c->pred_w2 = c->pred_split = false;
   }
   Geom& g = c->g;
   memset(&g, 0, sizeof g);
@@ -940,7 +962,7 @@ uint64_t tune_key(pypde_ctx* c) {
 
 void apply_tuning(pypde_ctx* c, const std::vector<int>& v) {
   c->tune.weno = (c->D == 2 && v[0] >= 0 && v[0] < N_WENO_V) ? v[0] : 0;
-  c->tune.flux = (v[1] >= 0 && v[1] < N_FLUX_V) ? v[1] : 0;
+  c->tune.flux = (v[1] >= 0 && v[1] < flux_variants(c->V)) ? v[1] : 0;
   c->tune.update = (v[2] >= 0 && v[2] < N_UPD_V) ? v[2] : 0;
   if (!c->pred_fixed) {
     c->pred_static = v[3] != 1;
@@ -1018,14 +1040,15 @@ int autotune(pypde_ctx* c) {
   c->ret = nullptr;
   const int nw = c->D == 2 ? N_WENO_V : 1;
   const int np = c->pred_fixed ? 1 : (c->fn[K_PRED_COLD] && c->hot ? N_PRED_V : 2);
-  const int ntrial = std::max(std::max(nw, N_FLUX_V), std::max(N_UPD_V, np));
+  const int nfl = flux_variants(c->V);
+  const int ntrial = std::max(std::max(nw, nfl), std::max(N_UPD_V, np));
   const int reps = 2;
   std::vector<std::vector<hipEvent_t>> evs(1 + reps * ntrial);
   int rc = 0;
   for (size_t k = 0; k < evs.size() && !rc; k++) {
     const int tk = k == 0 ? 0 : (int)((k - 1) % ntrial);
     c->tune.weno = tk % nw;
-    c->tune.flux = tk % N_FLUX_V;
+    c->tune.flux = tk % nfl;
     c->tune.update = tk % N_UPD_V;
     if (!c->pred_fixed) {
       c->pred_static = (tk % np) != 1;
@@ -1061,7 +1084,7 @@ int autotune(pypde_ctx* c) {
     const int tk = (int)((k - 1) % ntrial);
     tw[tk % nw] = std::min(tw[tk % nw], span(evs[k], 0, 1));
     tp[tk % np] = std::min(tp[tk % np], span(evs[k], 3, 4));
-    tf[tk % N_FLUX_V] = std::min(tf[tk % N_FLUX_V], span(evs[k], 4, 6));
+    tf[tk % nfl] = std::min(tf[tk % nfl], span(evs[k], 4, 6));
     tu[tk % N_UPD_V] = std::min(tu[tk % N_UPD_V], span(evs[k], 6, 7));
   }
   for (auto& e : evs)
@@ -1078,7 +1101,7 @@ int autotune(pypde_ctx* c) {
       if (t[i] < t[b]) b = i;
     return b;
   };
-  std::vector<int> v = {best(tw, nw), best(tf, N_FLUX_V), best(tu, N_UPD_V),
+  std::vector<int> v = {best(tw, nw), best(tf, nfl), best(tu, N_UPD_V),
                         c->pred_fixed ? (c->pred_static ? 0 : 1) : best(tp, np)};
   apply_tuning(c, v);
   c->tune.source = 1;
@@ -1371,7 +1394,7 @@ static int batch_setup(pypde_ensemble* e, long cap) {
           case BS_FLUX0:
           case BS_FLUX1: {
             const int d = s - BS_FLUX0;
-            gx = d < D ? cdiv(g.nf[d] * N * (ND / N), FLUX_BS[gr.flux]) : 0;
+            gx = d < D ? flux_blocks(V, gr.flux, g.nf[d] * N * (ND / N)) : 0;
             break;
           }
           default: {
@@ -1453,7 +1476,8 @@ static int enqueue_group_step(pypde_ensemble* e, const EnsGroup& gr) {
     return rc;
   }
   for (int d = 0; d < c->D; d++)
-    if ((rc = go(B_FLUX_KID[d][gr.flux], BS_FLUX0 + d, FLUX_BS[gr.flux], false))) return rc;
+    if ((rc = go(B_FLUX_KID[d][gr.flux], BS_FLUX0 + d, flux_threads(c->V, gr.flux), false)))
+      return rc;
   return go(B_UPD_KID[gr.update], BS_UPDATE, 256, false);
 }
 

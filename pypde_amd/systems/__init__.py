@@ -72,12 +72,19 @@ def standard_configs(full=False):
         s = SYSTEMS[name]
         out.append(dict(src=source(name), useF=s["F"], useB=s["B"], useS=s["S"], ndim=ndim, N=N,
                         V=s["V"], stiff=stiff, use_M=s["M"], flux=0, ensemble=True))
-    # 17-variable GPR (1D, order 2, the reference's B.dQ evaluation); each takes
-    # a few minutes to compile
+    # 17-variable GPR (1D, order 2, the reference's B.dQ evaluation)
     for stiff in ((False, True) if full else ()):
         s = SYSTEMS["gpr"]
         out.append(dict(src=source("gpr"), useF=True, useB=True, useS=True, ndim=1, N=2, V=17,
                         stiff=stiff, use_M=False, flux=0, b_quirk=1))
+    # ... and the other orders and dimensions its tests run, and its ensemble members
+    for ndim, N, stiff, quirk, ens in ((1, 1, True, 0, False), (1, 4, True, 0, False),
+                                       (2, 2, True, 0, False), (2, 3, False, 1, False),
+                                       (2, 6, False, 0, False), (1, 2, True, 0, False),
+                                       (1, 2, True, 0, True)) if full else ():
+        s = SYSTEMS["gpr"]
+        out.append(dict(src=source("gpr"), useF=True, useB=True, useS=True, ndim=ndim, N=N, V=17,
+                        stiff=stiff, use_M=False, flux=0, b_quirk=quirk, ensemble=ens))
     return out
 
 
