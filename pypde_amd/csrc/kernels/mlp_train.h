@@ -23,48 +23,82 @@ __device__ __forceinline__ float bf16_to_f(short h) {
   return __uint_as_float(((unsigned int)(unsigned short)h) << 16);
 }
 
+// Four floats p[0], p[ld], p[2 ld], p[3 ld] as BF16, entries from `left` on
+// read as 0 (left <= 0: none is read).  vec: ld = 1 and p is 16-byte aligned.
+__device__ __forceinline__ bf16x4 load4(const float* __restrict__ p, long ld, int left, bool vec) {
+  float x[4];
+  if (vec && left >= 4) {
+    const float4 q = *(const float4*)p;
+    x[0] = q.x, x[1] = q.y, x[2] = q.z, x[3] = q.w;
+  } else {
+#pragma unroll
+    for (int i = 0; i < 4; i++) x[i] = i < left ? p[i * ld] : 0.0f;
+  }
+  bf16x4 r;
+#pragma unroll
+  for (int i = 0; i < 4; i++) r[i] = to_bf16(x[i]);
+  return r;
+}
+__device__ __forceinline__ bf16x4 round4(float4 q) {
+  const bf16x4 r = {to_bf16(q.x), to_bf16(q.y), to_bf16(q.z), to_bf16(q.w)};
+  return r;
+}
+// Whether groups of four along a row of X (leading dimension ld) are aligned.
+__device__ __forceinline__ bool vector_rows(const float* X, int ld) {
+  return (ld & 3) == 0 && ((unsigned long long)X & 15ull) == 0;
+}
+
 // C = alpha op(A) op(B) + beta C;  op(A): M x K, op(B): K x N.
 // A(m, k) = transA ? A[k * lda + m] : A[m * lda + k];  likewise B.
-// Workgroup of 4 waves computes a 64 x 64 tile; K in chunks of 32 via LDS.
+// A workgroup of 4 waves computes a 64 x 64 tile.  The network's products have
+// K = 46..135 and a batch of columns, so what bounds them is the latency of
+// one panel after another: K goes in chunks of 128, a thread's sixteen loads
+// of four values all in flight, and both operands lie in LDS with k
+// contiguous, so that a fragment is one 8-byte read (135 x 4096 x 128: 14.9 ->
+// 7.7 us against chunks of 32 and B fragments gathered from four rows).
+constexpr int GEMM_KC = 128;
 extern "C" __global__ void __launch_bounds__(256)
 k_gemm_bf16(const float* __restrict__ A, int lda, int transA, const float* __restrict__ B, int ldb,
             int transB, float* __restrict__ C, int ldc, int M, int N, int K, float alpha,
             float beta) {
-  __shared__ short As[64][32 + 4];
-  __shared__ short Bs[32][64 + 4];
+  __shared__ __align__(16) short As[64][GEMM_KC + 8];
+  __shared__ __align__(16) short Bs[64][GEMM_KC + 8];
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int m0 = blockIdx.y * 64, n0 = blockIdx.x * 64;
   const int wr = (wave >> 1) * 32, wc = (wave & 1) * 32;
+  // op(X)'s panel, row index r0.. (op(A)'s rows, op(B)'s columns), as [row][k]
+  auto stage = [&](const float* __restrict__ X, int ld, bool kfast, int r0, int rows, int k0,
+                   short (*S)[GEMM_KC + 8]) {
+    constexpr int G = GEMM_KC / 4;
+    const bool vec = kfast && vector_rows(X, ld);
+#pragma unroll
+    for (int i = 0; i < 64 * G / 256; i++) {
+      const int e = tid + 256 * i;
+      // neighbouring threads read neighbouring addresses
+      const int r = kfast ? e / G : e % 64, k = 4 * (kfast ? e % G : e / 64);
+      const int gr = r0 + r, gk = k0 + k;
+      bf16x4 v = {0, 0, 0, 0};
+      if (gr < rows && gk < K)
+        v = load4(kfast ? X + (long)gr * ld + gk : X + (long)gk * ld + gr, kfast ? 1 : ld, K - gk,
+                  vec);
+      *(bf16x4*)&S[r][k] = v;
+    }
+  };
   f32x16 acc;
 #pragma unroll
   for (int j = 0; j < 16; j++) acc[j] = 0.0f;
-  for (int k0 = 0; k0 < K; k0 += 32) {
-    for (int e = tid; e < 64 * 32; e += 256) {
-      int r = e / 32, k = e % 32;
-      int gm = m0 + r, gk = k0 + k;
-      float a = 0.0f;
-      if (gm < M && gk < K) a = transA ? A[(long)gk * lda + gm] : A[(long)gm * lda + gk];
-      As[r][k] = to_bf16(a);
-    }
-    for (int e = tid; e < 32 * 64; e += 256) {
-      int k = e / 64, c = e % 64;
-      int gk = k0 + k, gn = n0 + c;
-      float b = 0.0f;
-      if (gk < K && gn < N) b = transB ? B[(long)gn * ldb + gk] : B[(long)gk * ldb + gn];
-      Bs[k][c] = to_bf16(b);
-    }
+  for (int k0 = 0; k0 < K; k0 += GEMM_KC) {
+    if (k0) __syncthreads();
+    stage(A, lda, !transA, m0, M, k0, As);
+    stage(B, ldb, transB != 0, n0, N, k0, Bs);
     __syncthreads();
-#pragma unroll
-    for (int kk = 0; kk < 4; kk++) {
-      bf16x4 a, b;
-#pragma unroll
-      for (int i = 0; i < 4; i++) {
-        a[i] = As[wr + (lane & 31)][kk * 8 + 4 * (lane >> 5) + i];
-        b[i] = Bs[kk * 8 + 4 * (lane >> 5) + i][wc + (lane & 31)];
-      }
+    const int kc = K - k0 < GEMM_KC ? (K - k0 + 7) / 8 : GEMM_KC / 8;
+#pragma unroll 4
+    for (int kk = 0; kk < kc; kk++) {
+      const bf16x4 a = *(const bf16x4*)&As[wr + (lane & 31)][kk * 8 + 4 * (lane >> 5)];
+      const bf16x4 b = *(const bf16x4*)&Bs[wc + (lane & 31)][kk * 8 + 4 * (lane >> 5)];
       acc = __builtin_amdgcn_mfma_f32_32x32x8bf16_1k(a, b, acc, 0, 0, 0);
     }
-    __syncthreads();
   }
 #pragma unroll
   for (int j = 0; j < 16; j++) {
@@ -74,6 +108,76 @@ k_gemm_bf16(const float* __restrict__ A, int lda, int transA, const float* __res
       float v = alpha * acc[j];
       if (beta != 0.0f) v += beta * C[(long)r * ldc + c];
       C[(long)r * ldc + c] = v;
+    }
+  }
+}
+
+// C = alpha A B^T + beta C for a long K and a small C (weight gradients: K is
+// the batch): with 64 x 64 tiles such a product fills two to six workgroups
+// that walk the batch serially.  Here a workgroup of 16 waves computes a 16 x
+// 16 tile, each wave taking one sixteenth of K straight from memory (k is
+// contiguous in both operands) in chunks of 32, and the 16 partial tiles are
+// summed in wave order, so results do not depend on timing.  Bound by each
+// compute unit's line lookups (a load touches 16 rows); the workgroups start
+// at different chunks, so that a power-of-two batch's rows do not meet in one
+// L2 channel.  135 x 128 x 4096: 345 -> 16.5 us, x 16384: 2021 -> 59 us.
+typedef float f32x4 __attribute__((ext_vector_type(4)));
+constexpr int TALL_WAVES = 16;
+extern "C" __global__ void __launch_bounds__(64 * TALL_WAVES)
+k_gemm_bf16_tall(const float* __restrict__ A, int lda, const float* __restrict__ B, int ldb,
+                 float* __restrict__ C, int ldc, int M, int N, int K, float alpha, float beta) {
+  __shared__ float part[TALL_WAVES][16][17];
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int m0 = blockIdx.y * 16, n0 = blockIdx.x * 16;
+  // rows past the edge repeat the last one; their results are not stored
+  const int ra = m0 + (lane & 15) < M ? m0 + (lane & 15) : M - 1;
+  const int rb = n0 + (lane & 15) < N ? n0 + (lane & 15) : N - 1;
+  const float* const pa = A + (long)ra * lda;
+  const float* const pb = B + (long)rb * ldb;
+  const bool vec = vector_rows(A, lda) && vector_rows(B, ldb);
+  // 16x16x16: a[i] = A[l % 16][4 (l / 16) + i], c[j] = C[4 (l / 16) + j][l % 16]
+  f32x4 acc = {0.0f, 0.0f, 0.0f, 0.0f};
+  const int chunks = (K + 32 * TALL_WAVES - 1) / (32 * TALL_WAVES);  // per wave
+  int c = (int)((blockIdx.x + blockIdx.y * gridDim.x) % chunks);
+#pragma unroll 4
+  for (int i = 0; i < chunks; i++) {
+    const int k0 = 32 * (wave * chunks + c);
+    c = c + 1 < chunks ? c + 1 : 0;
+    if (vec && k0 + 32 <= K) {
+      float4 x[2][2];
+#pragma unroll
+      for (int h = 0; h < 2; h++) {
+        const int k = k0 + 16 * h + 4 * (lane >> 4);
+        x[0][h] = *(const float4*)(pa + k);
+        x[1][h] = *(const float4*)(pb + k);
+      }
+#pragma unroll
+      for (int h = 0; h < 2; h++)
+        acc = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(round4(x[0][h]), round4(x[1][h]), acc, 0,
+                                                        0, 0);
+    } else {
+#pragma unroll
+      for (int h = 0; h < 2; h++) {
+        const int k = k0 + 16 * h + 4 * (lane >> 4);
+        acc = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(load4(pa + k, 1, K - k, false),
+                                                        load4(pb + k, 1, K - k, false), acc, 0, 0,
+                                                        0);
+      }
+    }
+  }
+#pragma unroll
+  for (int j = 0; j < 4; j++) part[wave][4 * (lane >> 4) + j][lane & 15] = acc[j];
+  __syncthreads();
+  if (threadIdx.x < 256) {
+    const int r = threadIdx.x >> 4, c = threadIdx.x & 15;
+    float v = part[0][r][c];
+#pragma unroll
+    for (int w = 1; w < TALL_WAVES; w++) v += part[w][r][c];
+    if (m0 + r < M && n0 + c < N) {
+      float* const o = C + (long)(m0 + r) * ldc + n0 + c;
+      v = alpha * v;
+      if (beta != 0.0f) v += beta * *o;
+      *o = v;
     }
   }
 }
@@ -121,18 +225,19 @@ k_rowsum(const float* __restrict__ dZ, float* __restrict__ db, int rows, int col
 }
 
 // mean-squared error over rows x cols: dY = 2 (Y - T) / (rows cols), loss
-// accumulated (sum of squares / (rows cols)) into *loss.
+// accumulated (sum of squares / (rows cols)) into *loss.  At most 256
+// workgroups stride over the array: their atomics on the one address are what
+// bounds a launch with one per 256 entries (135 x 4096: 30.6 -> 8.2 us).
 extern "C" __global__ void __launch_bounds__(256)
 k_mse(const float* __restrict__ Y, const float* __restrict__ T, float* __restrict__ dY,
       float* __restrict__ loss, int rows, int cols) {
   __shared__ float red[256];
   long n = (long)rows * cols;
-  long i = (long)blockIdx.x * 256 + threadIdx.x;
   float e = 0.0f;
-  if (i < n) {
+  for (long i = (long)blockIdx.x * 256 + threadIdx.x; i < n; i += 256l * gridDim.x) {
     float d = Y[i] - T[i];
     dY[i] = 2.0f * d / (float)n;
-    e = d * d / (float)n;
+    e += d * d / (float)n;
   }
   red[threadIdx.x] = e;
   __syncthreads();

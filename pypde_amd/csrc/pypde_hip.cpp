@@ -1812,8 +1812,10 @@ int pypde_geometry(pypde_ctx* c, long* nwc, int* n_in, int* n_out) {
 
 // ---------------------------------------------------------------- training
 static hipModule_t g_mlp_mod[16];
-static hipFunction_t g_mlp_fn[16][6];
-static const char* mlp_names[6] = {"k_gemm_bf16", "k_bias_act", "k_act_grad", "k_rowsum", "k_mse", "k_adam"};
+constexpr int N_MLP = 7;
+static hipFunction_t g_mlp_fn[16][N_MLP];
+static const char* mlp_names[N_MLP] = {"k_gemm_bf16", "k_bias_act", "k_act_grad", "k_rowsum",
+                                       "k_mse", "k_adam", "k_gemm_bf16_tall"};
 
 static int mlp_fn(int k, hipFunction_t* f) {
   int dev = 0;
@@ -1826,7 +1828,7 @@ static int mlp_fn(int k, hipFunction_t* f) {
     int rc = rtc_compile(MLP_SRC, "pypde_mlp.hip", &code);
     if (rc) return rc;
     HIPCHK(hipModuleLoadData(&g_mlp_mod[dev], code.data()));
-    for (int i = 0; i < 6; i++) HIPCHK(hipModuleGetFunction(&g_mlp_fn[dev][i], g_mlp_mod[dev], mlp_names[i]));
+    for (int i = 0; i < N_MLP; i++) HIPCHK(hipModuleGetFunction(&g_mlp_fn[dev][i], g_mlp_mod[dev], mlp_names[i]));
   }
   *f = g_mlp_fn[dev][k];
   return 0;
@@ -1887,6 +1889,15 @@ int pypde_mlp_compile(void) {
 int pypde_mlp_gemm(const float* A, int lda, int transA, const float* B, int ldb, int transB,
                    float* C, int ldc, int M, int N, int K, float alpha, float beta, void* stream) {
   if (M <= 0 || N <= 0 || K <= 0) return fail(PYPDE_ERR_ARG, "gemm sizes");
+  // a long K over a C of few 64 x 64 tiles (weight gradients): split over the
+  // waves of 16 x 16 tiles.  The 64 x 64 kernel walks K serially in as many
+  // workgroups as C has tiles; measured, split against that, in us: 135 x 128
+  // at K = 256 4.7 against 10.8, 1024 x 512 (128 tiles) at K = 256 11.7 against
+  // 11.1, at K = 1024 32 against 48; below 256 one or two chunks need no split
+  if (!transA && transB && K >= 256 && cdiv(M, 64) * cdiv(N, 64) <= 128) {
+    void* a[] = {&A, &lda, &B, &ldb, &C, &ldc, &M, &N, &K, &alpha, &beta};
+    return mlp_launch(6, dim3((unsigned)cdiv(N, 16), (unsigned)cdiv(M, 16)), dim3(1024), a, stream);
+  }
   void* a[] = {&A, &lda, &transA, &B, &ldb, &transB, &C, &ldc, &M, &N, &K, &alpha, &beta};
   return mlp_launch(0, dim3((unsigned)cdiv(N, 64), (unsigned)cdiv(M, 64)), dim3(256), a, stream);
 }
@@ -1909,7 +1920,8 @@ int pypde_mlp_rowsum(const float* dZ, float* db, int rows, int cols, void* strea
 int pypde_mlp_mse(const float* Y, const float* T, float* dY, float* loss, int rows, int cols,
                   void* stream) {
   void* a[] = {&Y, &T, &dY, &loss, &rows, &cols};
-  return mlp_launch(4, dim3((unsigned)cdiv((long)rows * cols, 256)), dim3(256), a, stream);
+  return mlp_launch(4, dim3((unsigned)std::min(256l, cdiv((long)rows * cols, 256))), dim3(256), a,
+                    stream);
 }
 
 int pypde_mlp_adam(float* w, const float* g, float* m, float* v, long n, float lr, float b1,
