@@ -56,6 +56,7 @@ def build_lib():
            "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",
            "-I", os.path.join(ROOT, "include"), "-I", CSRC, "-I", GEN,
            os.path.join(CSRC, "pypde_hip.cpp"), os.path.join(CSRC, "tables.cpp"),
+           os.path.join(CSRC, "transfer.cpp"), "-pthread",
            "-o", LIB + ".tmp", "-lhiprtc", "-lamdhip64", "-ldl"]
     subprocess.run(cmd, check=True)
     os.replace(LIB + ".tmp", LIB)

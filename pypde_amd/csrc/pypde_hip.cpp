@@ -15,6 +15,7 @@
 
 #include <algorithm>
 #include <chrono>
+#include <climits>
 #include <cmath>
 #include <cstdarg>
 #include <cstdio>
@@ -28,12 +29,14 @@
 #include <vector>
 
 #include "tables.h"
+#include "transfer.h"
 
 namespace {
 
 #include "kernels_embed.inc"  // PRELUDE_SRC, COMMON_SRC, WIDE_SRC, KERNELS_SRC, STEP_SRC
 
 constexpr int MAXV = 17;
+constexpr int P2R_CELLS = 64;  // cells per workgroup of k_planes_to_rows
 constexpr int WIDE_V = 8;  // above this V the kernels of ader_wide.h and ader_wide_predictor.h
 thread_local std::string g_err;
 
@@ -401,56 +404,113 @@ struct pypde_ctx {
 namespace {
 
 // Loaded code objects, one per (device, code-object key), shared by every
-// context of the same specification (ensemble members, repeated solves) and
-// unloaded when the last one is destroyed.
+// context of the same specification (ensemble members, repeated solves).  Up
+// to MAX_IDLE_MODS that no context uses stay loaded for the next one (a load
+// takes 0.8 ms, most of a small solve's set-up); past that the least recently
+// used is unloaded.
+constexpr size_t MAX_IDLE_MODS = 8;
 struct ModEntry {
   hipModule_t mod;
   int refs;
+  unsigned long used;
+  hipFunction_t fn[K_COUNT];
 };
 std::map<std::pair<int, uint64_t>, ModEntry> g_mods;
+std::map<std::string, uint64_t> g_spec_keys;  // specification -> code-object key
+unsigned long g_mod_clock = 0;
 std::mutex g_mod_mu;
+
+// Unloads idle modules, least recently used first, down to `keep` (g_mod_mu held).
+void trim_modules(size_t keep) {
+  while (true) {
+    size_t idle = 0;
+    auto oldest = g_mods.end();
+    for (auto it = g_mods.begin(); it != g_mods.end(); ++it)
+      if (it->second.refs == 0) {
+        idle++;
+        if (oldest == g_mods.end() || it->second.used < oldest->second.used) oldest = it;
+      }
+    if (idle <= keep) return;
+    (void)hipModuleUnload(oldest->second.mod);
+    g_mods.erase(oldest);
+  }
+}
 
 void release_module(int device, hipModule_t mod) {
   if (!mod) return;
   std::lock_guard<std::mutex> lk(g_mod_mu);
-  for (auto it = g_mods.begin(); it != g_mods.end(); ++it)
-    if (it->first.first == device && it->second.mod == mod) {
-      if (--it->second.refs == 0) {
-        (void)hipModuleUnload(mod);
-        g_mods.erase(it);
-      }
+  for (auto& e : g_mods)
+    if (e.first.first == device && e.second.mod == mod) {
+      if (--e.second.refs == 0) trim_modules(MAX_IDLE_MODS);
       return;
     }
-  (void)hipModuleUnload(mod);
 }
 
-int load_module(pypde_ctx* c, const std::vector<char>& code, uint64_t key, hipModule_t* mod,
-                hipFunction_t* fn) {
-  {
+// Everything the generated source depends on.
+std::string spec_id(const Spec& s) {
+  std::ostringstream o;
+  o << s.D << ' ' << s.N << ' ' << s.V << ' ' << s.useF << s.useB << s.useS << s.useM << s.stiff
+    << s.guess << s.second << s.mixed << s.batch << ' ' << s.b_quirk << ' ' << s.flux << '\n'
+    << s.src;
+  return o.str();
+}
+
+// The code object of `spec` loaded on `device` (the current one) and its
+// kernels: a loaded one where there is one, else compiled or fetched.
+int load_module(const Spec& spec, int device, hipModule_t* mod, hipFunction_t* fn,
+                uint64_t* key_out) {
+  // asked to compile or to write the source out: not from memory
+  const char* re = getenv("PYPDE_HIP_RECOMPILE");
+  const bool resident_ok = !(re && *re && *re != '0') && !getenv("PYPDE_HIP_DUMP_SRC");
+  const std::string id = spec_id(spec);
+  auto take = [&](uint64_t key) {
+    auto it = g_mods.find({device, key});
+    if (it == g_mods.end()) return false;
+    it->second.refs++;
+    it->second.used = ++g_mod_clock;
+    *mod = it->second.mod;
+    memcpy(fn, it->second.fn, sizeof it->second.fn);
+    *key_out = key;
+    return true;
+  };
+  if (resident_ok) {
     std::lock_guard<std::mutex> lk(g_mod_mu);
-    auto it = g_mods.find({c->device, key});
-    if (it != g_mods.end()) {
-      it->second.refs++;
-      *mod = it->second.mod;
-    } else {
-      if (hipModuleLoadData(mod, code.data()) != hipSuccess)
-        return fail(PYPDE_ERR_HIP, "hipModuleLoadData failed");
-      g_mods[{c->device, key}] = {*mod, 1};
-    }
+    auto k = g_spec_keys.find(id);
+    if (k != g_spec_keys.end() && take(k->second)) return 0;
   }
+  std::vector<char> code;
+  uint64_t key = 0;
+  if (int rc = compile_code(spec, &code, &key)) return rc;
+  std::lock_guard<std::mutex> lk(g_mod_mu);
+  if (g_spec_keys.size() >= 64) g_spec_keys.clear();
+  g_spec_keys[id] = key;
+  if (take(key)) return 0;
+  ModEntry e;
+  e.refs = 1;
+  e.used = ++g_mod_clock;
+  if (hipModuleLoadData(&e.mod, code.data()) != hipSuccess)
+    return fail(PYPDE_ERR_HIP, "hipModuleLoadData failed");
   for (int k = 0; k < K_COUNT; k++) {
-    fn[k] = nullptr;
-    bool optional = ((k == K_FLUX1 || k == K_FLUX1_128 || k == K_FLUX1_64) && c->D < 2) ||
+    e.fn[k] = nullptr;
+    bool optional = ((k == K_FLUX1 || k == K_FLUX1_128 || k == K_FLUX1_64) && spec.D < 2) ||
                     ((k == K_FLUX0_128 || k == K_FLUX0_64 || k == K_FLUX1_128 ||
-                      k == K_FLUX1_64) && c->V > WIDE_V) ||
-                    ((k == K_PRED || k == K_PRED_STATIC2) && c->V > WIDE_V) ||
-                    k == K_MLPGUESS || k == K_MLPPACK || (k == K_PRED32 && !c->spec.mixed) ||
+                      k == K_FLUX1_64) && spec.V > WIDE_V) ||
+                    ((k == K_PRED || k == K_PRED_STATIC2) && spec.V > WIDE_V) ||
+                    k == K_MLPGUESS || k == K_MLPPACK || (k == K_PRED32 && !spec.mixed) ||
                     k == K_PRED_COLD || k == K_PRED_HOT || k == K_PRED_COLD3 || k >= K_B_WENO;
-    if (hipModuleGetFunction(&fn[k], *mod, kernel_names[k]) != hipSuccess) {
-      fn[k] = nullptr;
-      if (!optional) return fail(PYPDE_ERR_HIP, "kernel %s missing", kernel_names[k]);
+    if (hipModuleGetFunction(&e.fn[k], e.mod, kernel_names[k]) != hipSuccess) {
+      e.fn[k] = nullptr;
+      (void)hipGetLastError();
+      if (!optional) {
+        (void)hipModuleUnload(e.mod);
+        return fail(PYPDE_ERR_HIP, "kernel %s missing", kernel_names[k]);
+      }
     }
   }
+  g_mods[{device, key}] = e;
+  *mod = e.mod;
+  memcpy(fn, e.fn, sizeof e.fn);
+  *key_out = key;
   return 0;
 }
 
@@ -737,7 +797,7 @@ void pypde_destroy(pypde_ctx* c) {
   if (c->qh) (void)hipFree(c->qh);
   release_module(c->device, c->mod);
   release_module(c->device, c->mod_guess);
-  if (c->stream) (void)hipStreamDestroy(c->stream);
+  if (c->stream) pypde::give_stream(c->device, c->stream);
   delete c;
 }
 
@@ -793,12 +853,8 @@ static pypde_ctx* create_ctx(const char* src, bool useF, bool useB, bool useS, c
       return nullptr;
     }
   }
-  std::vector<char> code;
-  uint64_t code_key = 0;
-  if ((rc = compile_code(s, &code, &code_key))) return nullptr;
   pypde_ctx* c = new pypde_ctx();
   c->spec = s;
-  c->code_key = code_key;
   c->opts = opts;
   c->D = ndim;
   c->N = N;
@@ -860,14 +916,17 @@ static pypde_ctx* create_ctx(const char* src, bool useF, bool useB, bool useS, c
     pypde_destroy(c);
     return (pypde_ctx*)nullptr;
   };
-  if (hipSetDevice(c->device) != hipSuccess)
+  if (hipSetDevice(c->device) != hipSuccess) {
+    std::vector<char> code;  // a source that does not compile is reported as that
+    if (int r = compile_code(s, &code)) return bail(r);
     return bail(fail(PYPDE_ERR_HIP, "hipSetDevice(%d) failed: no usable GPU", c->device));
+  }
   if (hipDeviceGetAttribute(&c->n_cu, hipDeviceAttributeMultiprocessorCount, c->device) !=
       hipSuccess)
     c->n_cu = 0;
-  if (load_module(c, code, code_key, &c->mod, c->fn_plain)) return bail(PYPDE_ERR_HIP);
+  if (int r = load_module(s, c->device, &c->mod, c->fn_plain, &c->code_key)) return bail(r);
   memcpy(c->fn, c->fn_plain, sizeof c->fn);
-  if (hipStreamCreate(&c->stream) != hipSuccess)
+  if (pypde::take_stream(c->device, &c->stream) != hipSuccess)
     return bail(fail(PYPDE_ERR_HIP, "hipStreamCreate failed"));
   size_t NTR = 2 * (size_t)ndim * N * (c->ND / N) * V;
   auto alloc = [&](double** p, size_t n) {
@@ -915,7 +974,7 @@ pypde_ctx* pypde_create(const char* src, bool useF, bool useB, bool useS, int* n
 int pypde_set_state(pypde_ctx* c, const double* u) {
   HIPCHK(hipSetDevice(c->device));
   size_t n = c->g.ncell * c->V;
-  HIPCHK(hipMemcpyAsync(c->tmp, u, n * sizeof(double), hipMemcpyHostToDevice, c->stream));
+  HIPCHK(pypde::copy_to_device(c->tmp, u, n * sizeof(double), c->device, c->stream));
   std::vector<void*> a = {&c->tmp, &c->u, &c->g.ncell};
   int rc = launch(c, K_A2S, dim3((unsigned)cdiv(n, 256)), dim3(256), a);
   if (rc) return rc;
@@ -929,8 +988,7 @@ int pypde_get_state(pypde_ctx* c, double* u) {
   std::vector<void*> a = {&c->u, &c->tmp, &c->g.ncell};
   int rc = launch(c, K_S2A, dim3((unsigned)cdiv(n, 256)), dim3(256), a);
   if (rc) return rc;
-  HIPCHK(hipMemcpyAsync(u, c->tmp, n * sizeof(double), hipMemcpyDeviceToHost, c->stream));
-  HIPCHK(hipStreamSynchronize(c->stream));
+  HIPCHK(pypde::copy_to_host(u, c->tmp, n * sizeof(double), c->device, c->stream));
   return 0;
 }
 
@@ -1155,6 +1213,14 @@ static int capture_steps(const std::vector<pypde_ctx*>& cs, hipGraphExec_t* exec
   return rc;
 }
 
+// Steps to t_f at the last step's dt, at least 1: what lies past the end of a
+// run is queued for nothing (a finished run's kernels return at once, but each
+// still takes 1-2 us).
+static int steps_left(const StepState& s) {
+  const double n = std::ceil((s.tf - s.t) / s.dt);
+  return n >= 1.0 ? (int)std::min(n, 1e6) : (s.dt > 0.0 ? 1 : INT_MAX);
+}
+
 static int run_loop(pypde_ctx* c, long max_steps, pypde_stats* stats, bool first_guess) {
   if (int r = autotune(c)) return r;
   auto t0 = std::chrono::steady_clock::now();
@@ -1166,11 +1232,9 @@ static int run_loop(pypde_ctx* c, long max_steps, pypde_stats* stats, bool first
   int rc = 0;
   while (true) {
     // never queue past a step cap: the launch count equals the step count
-    if (max_steps > 0) {
-      long left = max_steps - (long)c->host_st.count;
-      if (left < chunk) chunk = (int)std::max(1L, left);
-    }
-    for (int i = 0; i < chunk && !rc; i++) {
+    int n = std::min(chunk, steps_left(c->host_st));
+    if (max_steps > 0) n = (int)std::max(1L, std::min((long)n, max_steps - (long)c->host_st.count));
+    for (int i = 0; i < n && !rc; i++) {
       if (graph && !guess_now) {
         if (!exec && (rc = capture_steps({c}, &exec))) break;
         if (hipGraphLaunch(exec, c->stream) != hipSuccess) rc = fail(PYPDE_ERR_HIP, "graph launch failed");
@@ -1182,11 +1246,12 @@ static int run_loop(pypde_ctx* c, long max_steps, pypde_stats* stats, bool first
     }
     if (rc) break;
     const long long count_before = c->host_st.count;
-    HIPCHK(hipMemcpyAsync(&c->host_st, c->st, sizeof(StepState), hipMemcpyDeviceToHost, c->stream));
-    HIPCHK(hipStreamSynchronize(c->stream));
+    // (the spread statistics are zero between steps and stay on the device)
+    HIPCHK(pypde::copy_to_host(&c->host_st, c->st, offsetof(StepState, pstat), c->device,
+                               c->stream));
     if (c->host_st.done) break;
     if (c->host_st.count == count_before) {
-      rc = fail(PYPDE_ERR_HIP, "no progress in %d steps", chunk);
+      rc = fail(PYPDE_ERR_HIP, "no progress in %d steps", n);
       break;
     }
     if (chunk < 64) chunk *= 2;
@@ -1261,7 +1326,8 @@ int pypde_run(pypde_ctx* c, double tf, long max_steps, int ndt, double* ret, pyp
     if (r2) return r2;
     HIPCHK(hipMemcpyAsync(c->ret + (rows - 1) * row, c->tmp, row * sizeof(double),
                           hipMemcpyDeviceToDevice, c->stream));
-    if (ret) HIPCHK(hipMemcpyAsync(ret, c->ret, rows * row * sizeof(double), hipMemcpyDeviceToHost, c->stream));
+    if (ret)
+      HIPCHK(pypde::copy_to_host(ret, c->ret, rows * row * sizeof(double), c->device, c->stream));
     HIPCHK(hipStreamSynchronize(c->stream));
   }
   return rc;
@@ -1691,11 +1757,8 @@ int pypde_set_guess_model(pypde_ctx* c, const pypde_mlp* m) {
   if (!c->mod_guess) {
     Spec s = c->spec;
     s.guess = true;
-    std::vector<char> code;
     uint64_t key = 0;
-    int rc = compile_code(s, &code, &key);
-    if (rc) return rc;
-    if ((rc = load_module(c, code, key, &c->mod_guess, c->fn_guess))) return rc;
+    if (int rc = load_module(s, c->device, &c->mod_guess, c->fn_guess, &key)) return rc;
   }
   if (!c->gbuf) HIPCHK(hipMalloc((void**)&c->gbuf, c->g.nwc * c->NT * c->V * sizeof(double)));
   // pack the weights once: BF16 fragments in the inference kernel's order
@@ -1874,6 +1937,14 @@ int pypde_dev_sync(void) {
   return 0;
 }
 
+void pypde_release_idle(void) {
+  {
+    std::lock_guard<std::mutex> lk(g_mod_mu);
+    trim_modules(0);
+  }
+  pypde::release_idle_transfer();
+}
+
 int pypde_device_count(void) {
   int n = 0;
   if (hipGetDeviceCount(&n) != hipSuccess) return 0;
@@ -1944,34 +2015,41 @@ int weno_solver(double* ret, double* u, int* nX, int ndim, int N, int V) {
     nin *= nX[d];
     nout *= no[d];
   }
-  std::vector<char> code;
-  if ((rc = compile_code(s, &code))) return rc;
-  HIPCHK(hipSetDevice(0));
-  // the module and device buffers are released on every return path
+  if (hipSetDevice(0) != hipSuccess) {
+    std::vector<char> code;
+    if ((rc = compile_code(s, &code))) return rc;
+    return fail(PYPDE_ERR_HIP, "hipSetDevice(0) failed: no usable GPU");
+  }
+  // the module, stream and device buffers are released on every return path
   struct Release {
     hipModule_t mod = nullptr;
+    hipStream_t stream = nullptr;
     double *du = nullptr, *dus = nullptr, *dw = nullptr;
     ~Release() {
+      if (stream) (void)hipStreamSynchronize(stream);
       for (double* p : {du, dus, dw})
         if (p) (void)hipFree(p);
-      if (mod) (void)hipModuleUnload(mod);
+      release_module(0, mod);
+      if (stream) pypde::give_stream(0, stream);
     }
   } rel;
-  HIPCHK(hipModuleLoadData(&rel.mod, code.data()));
-  hipModule_t mod = rel.mod;
-  hipFunction_t fw, fa;
-  HIPCHK(hipModuleGetFunction(&fw, mod, "k_weno"));
-  HIPCHK(hipModuleGetFunction(&fa, mod, "k_aos_to_soa"));
+  hipFunction_t fn[K_COUNT];
+  uint64_t key = 0;
+  if ((rc = load_module(s, 0, &rel.mod, fn, &key))) return rc;
+  HIPCHK(pypde::take_stream(0, &rel.stream));
+  hipStream_t st0 = rel.stream;
   int ND = 1;
   for (int d = 0; d < ndim; d++) ND *= N;
+  // du holds the input, then the rows of the result
   double *&du = rel.du, *&dus = rel.dus, *&dw = rel.dw;
-  HIPCHK(hipMalloc((void**)&du, nin * V * sizeof(double)));
+  HIPCHK(hipMalloc((void**)&du, std::max(nin, nout * ND) * V * sizeof(double)));
   HIPCHK(hipMalloc((void**)&dus, nin * V * sizeof(double)));
   HIPCHK(hipMalloc((void**)&dw, nout * ND * V * sizeof(double)));
-  HIPCHK(hipMemcpy(du, u, nin * V * sizeof(double), hipMemcpyHostToDevice));
+  HIPCHK(pypde::copy_to_device(du, u, nin * V * sizeof(double), 0, st0));
   {
     void* a[] = {&du, &dus, &nin};
-    HIPCHK(hipModuleLaunchKernel(fa, (unsigned)cdiv(nin * V, 256), 1, 1, 256, 1, 1, 0, nullptr, a, nullptr));
+    HIPCHK(hipModuleLaunchKernel(fn[K_A2S], (unsigned)cdiv(nin * V, 256), 1, 1, 256, 1, 1, 0, st0,
+                                 a, nullptr));
   }
   Geom g;
   memset(&g, 0, sizeof g);
@@ -1982,13 +2060,15 @@ int weno_solver(double* ret, double* u, int* nX, int ndim, int N, int V) {
     unsigned gx = ndim == 1 ? (unsigned)cdiv(no[0], 256) : (unsigned)cdiv(no[1], 32);
     unsigned gy = ndim == 1 ? 1 : (unsigned)cdiv(no[0], 8);
     unsigned gz = ndim == 1 ? 1 : (unsigned)V;  // 2D: one variable per workgroup
-    HIPCHK(hipModuleLaunchKernel(fw, gx, gy, gz, 256, 1, 1, 0, nullptr, a, nullptr));
+    HIPCHK(hipModuleLaunchKernel(fn[K_WENO], gx, gy, gz, 256, 1, 1, 0, st0, a, nullptr));
   }
-  std::vector<double> h(nout * ND * V);
-  HIPCHK(hipMemcpy(h.data(), dw, h.size() * sizeof(double), hipMemcpyDeviceToHost));
   // planes [node*V+v][cell] -> reference layout [cell][node][v]
-  for (long cc = 0; cc < nout; cc++)
-    for (int p = 0; p < ND * V; p++) ret[cc * ND * V + p] = h[(size_t)p * nout + cc];
+  {
+    void* a[] = {&dw, &du, &nout};
+    HIPCHK(hipModuleLaunchKernel(fn[K_P2R], (unsigned)cdiv(nout, P2R_CELLS), 1, 1, 256, 1, 1, 0,
+                                 st0, a, nullptr));
+  }
+  HIPCHK(pypde::copy_to_host(ret, du, nout * ND * V * sizeof(double), 0, st0));
   return 0;
 }
 
@@ -2092,7 +2172,7 @@ int weno_solver_noalloc(pypde_ctx* c, double* ret, const double* u, const int* n
   }
   {
     void* a[] = {&s_out, &ret, &nout};
-    if ((rc = go(K_P2R, (unsigned)cdiv(nout * c->ND * V, 256), 1, 1, a))) return rc;
+    if ((rc = go(K_P2R, (unsigned)cdiv(nout, P2R_CELLS), 1, 1, a))) return rc;
   }
   if (!stream) HIPCHK(hipStreamSynchronize(s));
   return 0;
