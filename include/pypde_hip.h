@@ -66,9 +66,10 @@ typedef struct {
   int nan_step;             /* first step with NaNs (0: none) */
   double ms_loop;           /* wall time of the step loop */
   double ms_kernel[8];      /* profile: summed time per kernel (weno, dt, learned guess,
-                               predictor, flux0, flux1, update; the last slot is kept
-                               for layout and holds only the cost of one event pair,
-                               the step's bookkeeping running inside dt and update) */
+                               predictor, flux, -, update, -; the slots marked - are kept
+                               for layout and hold only the cost of one event pair: the
+                               flux launch takes every direction, the step's bookkeeping
+                               runs inside dt and update) */
   long pred_node_full;      /* stiff predictor: per-node Newton corrections that solved
                                with the source Jacobian, summed over nodes and steps */
   long pred_node_short;     /* ... and those that took the A = 0 shortcut (max |dt dS/dQ|
@@ -172,7 +173,8 @@ int pypde_harvest_step(pypde_ctx *c, float *X, float *Y, long ldx, long col0, py
  * (state restored afterwards) and keeps the fastest, or reuses the choice
  * recorded for the same problem in <code-object cache>/tuning.txt.
  * choices[5]: WENO tile (0 8x32, 1 4x64, 2 16x16, 3 16x32), flux workgroup (0
- * 256, 1 128, 2 64), corrector (0 one thread per cell, 1..4 one variable and
+ * 128 and 1 64 threads of one face point each, 2 a point's eigenvalue problems
+ * split over several wavefronts), corrector (0 one thread per cell, 1..4 one variable and
  * 1, 2, 4, 8 x-rows per thread), predictor (0 static, 1 work queue, 2 the
  * stiff predictor's cold/hot split, 3 the same with the cold pass built for
  * three wavefronts per SIMD), source (0 defaults, 1 measured, 2 tuning table,

@@ -269,7 +269,11 @@ DEV void cell_deriv(const double (&w)[ND][V], int idx, double rdx, double* out) 
 // eigenvalue work per lane.  Both lanes form the cell's (l_0 / dX_0) + (l_1 /
 // dX_1) from the pair's two terms.  The host launches DT_LANES * nwc threads.
 constexpr bool DT_PAIR = (D == 2) && (V <= 5) && !PDE_SECOND;
-constexpr int DT_LANES = V > 8 ? 64 : DT_PAIR ? 2 : 1;
+// With a viscous F a w-cell has 2 D eigenvalue problems, each of which costs as
+// much as a whole first-order cell: a wavefront takes one of them for 64
+// cells and the sums go through LDS (64 x 64 cells, 69 wavefronts one after
+// the other's problems otherwise: 22 -> 10.7 us).
+constexpr int DT_LANES = V > 8 ? 64 : PDE_SECOND ? 2 * D : DT_PAIR ? 2 : 1;
 
 #if PDE_V > 8
 // One wavefront per w-cell: the cell's mean (lane v takes variable v), then
@@ -303,6 +307,57 @@ DEV void dt_body(const double* __restrict__ wh, StepState* st, const Geom& g, co
   }
   if (lane == 0 && sum > 0.0)
     atomicMax(&st->pstat[b.x & 63][8], (unsigned long long)__double_as_longlong(sum));
+  if (last_workgroup(&st->dt_ticket, b.n)) dt_finalize(st);
+}
+#elif PDE_SECOND
+DEV void dt_body(const double* __restrict__ wh, StepState* st, const Geom& g, const Blk& b) {
+  constexpr int CELLS = 256 / DT_LANES;  // a multiple of 64: `part` is the same in a wavefront
+  __shared__ double lam[DT_LANES][CELLS];
+  const int part = threadIdx.x / CELLS, k = threadIdx.x % CELLS;
+  const long c = (long)b.x * CELLS + k;
+  if (c < g.nwc) {
+    double w[ND][V];
+#pragma unroll
+    for (int idx = 0; idx < ND; idx++)
+#pragma unroll
+      for (int v = 0; v < V; v++) w[idx][v] = wh[(long)(idx * V + v) * g.nwc + c];
+    double q[V], dq[D * V];
+#pragma unroll
+    for (int v = 0; v < V; v++) {
+      double acc = T_WP[0] * w[0][v];
+#pragma unroll
+      for (int idx = 1; idx < ND; idx++) acc = dfma(T_WP[idx], w[idx][v], acc);
+      q[v] = acc;
+    }
+    static_for<0, D>([&](auto dc) {
+      constexpr int d = decltype(dc)::value;
+      double acc[V], tmp[V];
+#pragma unroll
+      for (int idx = 0; idx < ND; idx++) {
+        cell_deriv<d>(w, idx, 1.0 / g.dX[d], tmp);
+#pragma unroll
+        for (int v = 0; v < V; v++) acc[v] = (idx == 0) ? T_WP[0] * tmp[v] : dfma(T_WP[idx], tmp[v], acc[v]);
+      }
+#pragma unroll
+      for (int v = 0; v < V; v++) dq[d * V + v] = acc[v];
+    });
+    static_for<0, D>([&](auto dc) {
+      constexpr int d = decltype(dc)::value;
+      double f0[V];
+      if (part == 2 * d) lam[2 * d][k] = max_abs_eigs(q, dq, d, f0);
+      if (part == 2 * d + 1) lam[2 * d + 1][k] = max_abs_eigs_second_order<d>(q, dq, g.dX[d]);
+    });
+  }
+  __syncthreads();
+  double sum = 0.0;
+  if (part == 0 && c < g.nwc) {
+#pragma unroll
+    for (int d = 0; d < D; d++) sum = sum + (lam[2 * d][k] + lam[2 * d + 1][k]) / g.dX[d];
+    if (!(sum > 0.0)) sum = 0.0;
+  }
+  const double m = wave_max(sum);
+  if ((threadIdx.x & 63) == 0 && m > 0.0)
+    atomicMax(&st->pstat[b.x & 63][8], (unsigned long long)__double_as_longlong(m));
   if (last_workgroup(&st->dt_ticket, b.n)) dt_finalize(st);
 }
 #else
@@ -349,26 +404,13 @@ DEV void dt_body(const double* __restrict__ wh, StepState* st, const Geom& g, co
       for (int idx = 1; idx < ND; idx++) acc = dfma(T_WP[idx], w[idx][v], acc);
       q[v] = acc;
     }
-    static_for<0, D>([&](auto dc) {
-      constexpr int d = decltype(dc)::value;
-      double acc[V], tmp[V];
+    // a first-order F takes no gradient
 #pragma unroll
-      for (int idx = 0; idx < ND; idx++) {
-        cell_deriv<d>(w, idx, 1.0 / g.dX[d], tmp);
-#pragma unroll
-        for (int v = 0; v < V; v++) acc[v] = (idx == 0) ? T_WP[0] * tmp[v] : dfma(T_WP[idx], tmp[v], acc[v]);
-      }
-#pragma unroll
-      for (int v = 0; v < V; v++) dq[d * V + v] = acc[v];
-    });
+    for (int i = 0; i < D * V; i++) dq[i] = 0.0;
     static_for<0, D>([&](auto dc) {
       constexpr int d = decltype(dc)::value;
       double f0[V];
-      double lam = max_abs_eigs(q, dq, d, f0);
-#if PDE_SECOND
-      lam = lam + max_abs_eigs_second_order<d>(q, dq, g.dX[d]);
-#endif
-      sum = sum + lam / g.dX[d];
+      sum = sum + max_abs_eigs(q, dq, d, f0) / g.dX[d];
     });
     if (!(sum > 0.0)) sum = 0.0;
   }

@@ -1465,6 +1465,10 @@ k_predictor_f32(const double* __restrict__ wh, const double* __restrict__ gin,
 // ------------------------------------------------------------ face flux
 // Rusanov flux and B path integral at every face point (fluxes.cpp:72-116).
 // Faces along d: (nx_d + 1) x prod_{e != d} nx_e, all touching an interior cell.
+struct FaceOut {
+  double* ff[2];
+  double* fb[2];
+};
 template <int d>
 DEV void face_cells(const Geom& g, long f, long* wl, long* wr) {
   if constexpr (D == 1) {
@@ -1481,22 +1485,14 @@ DEV void face_cells(const Geom& g, long f, long* wl, long* wr) {
   }
 }
 
-// Numerical flux at one face point along axis d (fv.cpp:124-198): Rusanov
-// (fluxes.cpp:72-101), Roe or Osher (fluxes.cpp:20-70), the viscous term
-// (fluxes.cpp:96-100) and the non-conservative path integral Bint
-// (fluxes.cpp:103-116), from the two cells' face traces.
 #if PDE_V > 8
 // Above V = 8 (Rusanov, first-order F): one face point per workgroup of two
 // wavefronts, one for each side's wave speed and F.
-template <int d, int BS>
-DEV void flux_dir(const double* __restrict__ tr, double* __restrict__ ff, double* __restrict__ fb,
-                  const StepState* st, const Geom& g, const double* __restrict__ trd,
-                  const Blk& b) {
-  static_assert(BS == 128, "one wavefront per side");
-  (void)st;
-  (void)trd;
+template <int d>
+DEV void flux_wide(const double* __restrict__ tr, double* __restrict__ ff, double* __restrict__ fb,
+                   const Geom& g, long blk) {
   const long nf = g.nf[d];
-  const long item = b.x;
+  const long item = blk;
   const long f = item % nf;
   const int j = (int)((item / nf) % ND1);
   const int t = (int)(item / (nf * ND1));
@@ -1563,65 +1559,110 @@ DEV void flux_dir(const double* __restrict__ tr, double* __restrict__ ff, double
   }
 #endif
 }
-#else
-template <int d, int BS = 256>
-DEV void flux_dir(const double* __restrict__ tr, double* __restrict__ ff, double* __restrict__ fb,
-                  const StepState* st, const Geom& g, const double* __restrict__ trd,
-                  const Blk& b) {
-  const long nf = g.nf[d];
+#else  // PDE_V <= 8
+// Face f, time node t and transverse node j of flux item `item` of direction
+// d, and its two w-cells; false past the last item.
+struct FaceItem {
   long f, wl, wr;
   int j, t;
+};
+template <int d>
+DEV bool face_item(const Geom& g, unsigned int blk, int threads, int tid, FaceItem* it) {
+  const long nf = g.nf[d];
   if (g.idx32) {
     // 32-bit indices, divisions by nf and by the faces per row as
     // multiply-shifts (nf N ND1 and nwc below 2^31)
-    const unsigned item = b.x * (unsigned)BS + threadIdx.x;
-    if (item >= (unsigned)nf * (unsigned)(N * ND1)) return;
+    const unsigned item = blk * (unsigned)threads + (unsigned)tid;
+    if (item >= (unsigned)nf * (unsigned)(N * ND1)) return false;
     const unsigned rest = udiv(item, g.fmul[d], g.fsh[d]);
     const unsigned f32 = item - rest * (unsigned)nf;
-    j = (int)(rest % ND1);
-    t = (int)(rest / ND1);
-    f = f32;
+    it->j = (int)(rest % ND1);
+    it->t = (int)(rest / ND1);
+    it->f = f32;
     if constexpr (D == 1) {
-      wl = f32;
-      wr = f32 + 1;
+      it->wl = f32;
+      it->wr = f32 + 1;
     } else {
       const unsigned row = d == 0 ? (unsigned)g.nx[1] : (unsigned)g.nx[1] + 1;
       const unsigned f0 = udiv(f32, g.rmul[d], g.rsh[d]), f1 = f32 - f0 * row;
       const unsigned nw1 = (unsigned)g.nw[1];
       const unsigned l = d == 0 ? f0 * nw1 + (f1 + 1) : (f0 + 1) * nw1 + f1;
-      wl = l;
-      wr = d == 0 ? l + nw1 : l + 1;
+      it->wl = l;
+      it->wr = d == 0 ? l + nw1 : l + 1;
     }
   } else {
-    const long item = (long)b.x * BS + threadIdx.x;
-    if (item >= nf * N * ND1) return;
-    f = item % nf;
-    j = (int)((item / nf) % ND1);
-    t = (int)(item / (nf * ND1));
-    face_cells<d>(g, f, &wl, &wr);
+    const long item = (long)blk * threads + tid;
+    if (item >= nf * N * ND1) return false;
+    it->f = item % nf;
+    it->j = (int)((item / nf) % ND1);
+    it->t = (int)(item / (nf * ND1));
+    face_cells<d>(g, it->f, &it->wl, &it->wr);
   }
-  double qL[V], qR[V];
+  return true;
+}
+
+// Face traces (and, for a viscous F, gradients; zero otherwise, as the
+// reference passes unused dQ) of one side of a face point: side 0 left, 1 right.
+template <int d>
+DEV void face_state(const double* __restrict__ tr, const double* __restrict__ trd, const Geom& g,
+                    const FaceItem& it, int side, double* q, double* dq) {
+  const long w = side ? it.wr : it.wl;
+  const int e = side ? 0 : 1;
+#pragma unroll
+  for (int v = 0; v < V; v++)
+    q[v] = tr[(long)((((d * 2 + e) * N + it.t) * ND1 + it.j) * V + v) * g.nwc + w];
+#pragma unroll
+  for (int i = 0; i < D * V; i++) {
+#if PDE_SECOND
+    dq[i] = trd[(long)((((d * 2 + e) * N + it.t) * ND1 + it.j) * D * V + i) * g.nwc + w];
+#else
+    dq[i] = 0.0;
+#endif
+  }
+}
+
+#if PDE_USE_B
+// Non-conservative path integral (fluxes.cpp:103-116).
+template <int d>
+DEV void face_b(const double* qL, const double* qR, double* __restrict__ fb, long o, long nf) {
+  double Dq[V], Mx[V * V], b[V * V], q[V];
+#pragma unroll
+  for (int v = 0; v < V; v++) Dq[v] = qR[v] - qL[v];
+#pragma unroll
+  for (int i = 0; i < N; i++) {
+#pragma unroll
+    for (int v = 0; v < V; v++) q[v] = dfma(T_X[i], Dq[v], qL[v]);
+    B(b, q, d);
+#pragma unroll
+    for (int k = 0; k < V * V; k++) Mx[k] = (i == 0) ? T_W[0] * b[k] : dfma(T_W[i], b[k], Mx[k]);
+  }
 #pragma unroll
   for (int v = 0; v < V; v++) {
-    qL[v] = tr[(long)((((d * 2 + 1) * N + t) * ND1 + j) * V + v) * g.nwc + wl];
-    qR[v] = tr[(long)((((d * 2 + 0) * N + t) * ND1 + j) * V + v) * g.nwc + wr];
+    double acc = Mx[v * V] * Dq[0];
+#pragma unroll
+    for (int k = 1; k < V; k++) acc = dfma(Mx[v * V + k], Dq[k], acc);
+    fb[o + (long)v * nf] = acc;
   }
-  const long o = (long)((t * ND1 + j) * V) * nf + f;
+}
+#endif
+
+// Numerical flux at one face point along axis d (fv.cpp:124-198): Rusanov
+// (fluxes.cpp:72-101), Roe or Osher (fluxes.cpp:20-70), the viscous term
+// (fluxes.cpp:96-100) and the non-conservative path integral, one thread per
+// face point.
+template <int d, int BS>
+DEV void flux_point(const double* __restrict__ tr, double* __restrict__ ff,
+                    double* __restrict__ fb, const Geom& g, const double* __restrict__ trd,
+                    unsigned int blk) {
+  FaceItem it;
+  if (!face_item<d>(g, blk, BS, threadIdx.x, &it)) return;
+  const long nf = g.nf[d];
+  double qL[V], qR[V], dqL[D * V], dqR[D * V];
+  face_state<d>(tr, trd, g, it, 0, qL, dqL);
+  face_state<d>(tr, trd, g, it, 1, qR, dqR);
+  const long o = (long)((it.t * ND1 + it.j) * V) * nf + it.f;
 #if PDE_USE_F
   {
-    // face gradients (viscous F only; zero otherwise, as the reference passes
-    // unused dQ)
-    double dqL[D * V], dqR[D * V];
-#pragma unroll
-    for (int i = 0; i < D * V; i++) {
-#if PDE_SECOND
-      dqL[i] = trd[(long)((((d * 2 + 1) * N + t) * ND1 + j) * D * V + i) * g.nwc + wl];
-      dqR[i] = trd[(long)((((d * 2 + 0) * N + t) * ND1 + j) * D * V + i) * g.nwc + wr];
-#else
-      dqL[i] = 0.0;
-      dqR[i] = 0.0;
-#endif
-    }
     double fl[V], fr[V], fv[V];
 #if PDE_FLUX == 0
     // Rusanov: max(lam(qL), lam(qR)) (qL - qR) + F(qL) + F(qR)  (fluxes.cpp:72-101)
@@ -1677,53 +1718,180 @@ DEV void flux_dir(const double* __restrict__ tr, double* __restrict__ ff, double
   }
 #endif
 #if PDE_USE_B
-  {
-    double Dq[V], Mx[V * V], b[V * V], q[V];
-#pragma unroll
-    for (int v = 0; v < V; v++) Dq[v] = qR[v] - qL[v];
-#pragma unroll
-    for (int i = 0; i < N; i++) {
-#pragma unroll
-      for (int v = 0; v < V; v++) q[v] = dfma(T_X[i], Dq[v], qL[v]);
-      B(b, q, d);
-#pragma unroll
-      for (int k = 0; k < V * V; k++) Mx[k] = (i == 0) ? T_W[0] * b[k] : dfma(T_W[i], b[k], Mx[k]);
-    }
-#pragma unroll
-    for (int v = 0; v < V; v++) {
-      double acc = Mx[v * V] * Dq[0];
-#pragma unroll
-      for (int k = 1; k < V; k++) acc = dfma(Mx[v * V + k], Dq[k], acc);
-      fb[o + (long)v * nf] = acc;
-    }
-  }
+  face_b<d>(qL, qR, fb, o, nf);
 #endif
 }
 
-#endif
+#if PDE_USE_F
+// The same with a face point's independent eigenvalue problems in as many
+// wavefronts: 64 face points per workgroup of FLUX_SPLIT wavefronts, which
+// hand their results to the first through LDS.  Rusanov: one wavefront per
+// side; Osher: one per path point; a viscous F: one more per side.  A serial
+// chain 1 / FLUX_SPLIT as long and as many more wavefronts: what small grids
+// (few wavefronts, or a nearly empty last round of them) are bound by; the
+// same arithmetic on large ones, where the autotuner weighs it against one
+// thread per point.  Viscous flow on 64 x 64 cells: 20.8 us against 28.6 (both
+// directions); Osher on 128 x 128 155 against 131, Rusanov on 317 x 203 72
+// against 64: full rounds of wavefronts gain nothing from shorter ones.
+constexpr int FLUX_PARTS = PDE_FLUX == 0 ? 2 : PDE_FLUX == 1 ? 1 : N;  // first-order part
+constexpr int FLUX_SPLIT = FLUX_PARTS + (PDE_SECOND ? 2 : 0);
+struct FluxShared {
+  double part[FLUX_PARTS][V][64];  // the right side's F, or |A(q_i)| (qL - qR)
+  double lam[FLUX_SPLIT][64];      // wave speeds
+};
 
-// Workgroup sizes 256 (k_flux0, k_flux1), 128 and 64 (..._128, ..._64): the
-// autotuner picks one per problem; every face point's arithmetic is the same.
-// Above V = 8 only k_flux0 and k_flux1 exist, of 128 threads.
-#define PYPDE_FLUX_KERNEL(NAME, DIR, BS)                                                       \
-  extern "C" __global__ void __launch_bounds__(BS)                                             \
-  NAME(const double* __restrict__ tr, double* __restrict__ ff, double* __restrict__ fb,        \
-       const StepState* st, Geom g, const double* __restrict__ trd) {                          \
-    if (st->done) return;                                                                      \
-    flux_dir<DIR, BS>(tr, ff, fb, st, g, trd, hw_blk());                                       \
+template <int d>
+DEV void flux_split(FluxShared& sm, const double* __restrict__ tr, double* __restrict__ ff,
+                    double* __restrict__ fb, const Geom& g, const double* __restrict__ trd,
+                    unsigned int blk) {
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  FaceItem it;
+  const bool ok = face_item<d>(g, blk, 64, lane, &it);
+  const long nf = g.nf[d];
+  double qL[V], qR[V], dqL[D * V], dqR[D * V], fl[V];
+  if (ok) {
+#if PDE_SECOND
+    if (wave >= FLUX_PARTS) {
+      face_state<d>(tr, trd, g, it, wave - FLUX_PARTS, qL, dqL);
+      sm.lam[wave][lane] = max_abs_eigs_second_order<d>(qL, dqL, g.dX[d]);
+    } else
+#endif
+    {
+#if PDE_FLUX == 0
+      face_state<d>(tr, trd, g, it, wave, qL, dqL);
+      sm.lam[wave][lane] = max_abs_eigs(qL, dqL, d, fl);
+      if (wave == 1) {
+#pragma unroll
+        for (int v = 0; v < V; v++) sm.part[1][v][lane] = fl[v];
+      }
+#else
+      face_state<d>(tr, trd, g, it, 0, qL, dqL);
+      face_state<d>(tr, trd, g, it, 1, qR, dqR);
+      double Dq[V], q[V], A[V * V], ftmp[V], y[V], dqp[D * V];
+#if PDE_FLUX == 1
+      double Mx[V * V];
+#endif
+#pragma unroll
+      for (int v = 0; v < V; v++) Dq[v] = qL[v] - qR[v];
+#pragma unroll
+      for (int i = 0; i < N; i++) {
+        if (PDE_FLUX == 2 && i != wave) continue;
+#pragma unroll
+        for (int v = 0; v < V; v++) q[v] = dfma(T_X[i], Dq[v], qR[v]);
+#pragma unroll
+        for (int k = 0; k < D * V; k++) dqp[k] = dfma(T_X[i], dqL[k] - dqR[k], dqR[k]);
+#if PDE_FLUX == 1
+        system_matrix(q, dqp, d, A, ftmp);
+#pragma unroll
+        for (int k = 0; k < V * V; k++)
+          Mx[k] = (i == 0) ? T_W[0] * A[k] : dfma(T_W[i], A[k], Mx[k]);
+#endif
+      }
+#if PDE_FLUX == 1
+      abs_apply(Mx, Dq, y);
+#else
+      system_matrix(q, dqp, d, A, ftmp);
+      abs_apply(A, Dq, y);
+#endif
+#pragma unroll
+      for (int v = 0; v < V; v++) sm.part[wave][v][lane] = y[v];
+#endif
+    }
   }
-constexpr int FLUX_BS0 = V > 8 ? 128 : 256;
-PYPDE_FLUX_KERNEL(k_flux0, 0, FLUX_BS0)
-#if PDE_D >= 2
-PYPDE_FLUX_KERNEL(k_flux1, 1, FLUX_BS0)
+  __syncthreads();
+  if (!ok) return;
+  const long o = (long)((it.t * ND1 + it.j) * V) * nf + it.f;
+  if (wave == 0) {
+    double fv[V];
+#if PDE_FLUX == 0
+    face_state<d>(tr, trd, g, it, 1, qR, dqR);
+    const double s = dmax(sm.lam[0][lane], sm.lam[1][lane]);
+#pragma unroll
+    for (int v = 0; v < V; v++) fv[v] = s * (qL[v] - qR[v]) + (fl[v] + sm.part[1][v][lane]);
+#else
+    double fr[V];
+    F(fl, qL, dqL, d);
+    F(fr, qR, dqR, d);
+#pragma unroll
+    for (int v = 0; v < V; v++) {
+      double sum = PDE_FLUX == 1 ? sm.part[0][v][lane] : T_W[0] * sm.part[0][v][lane];
+#pragma unroll
+      for (int i = 1; i < FLUX_PARTS; i++) sum = dfma(T_W[i], sm.part[i][v][lane], sum);
+      fv[v] = sum + (fl[v] + fr[v]);
+    }
 #endif
+#if PDE_SECOND
+    const double s2 = dmax(sm.lam[FLUX_PARTS][lane], sm.lam[FLUX_SPLIT - 1][lane]);
+#pragma unroll
+    for (int v = 0; v < V; v++) fv[v] = fv[v] + s2 * (qL[v] - qR[v]);
+#endif
+#pragma unroll
+    for (int v = 0; v < V; v++) ff[o + (long)v * nf] = fv[v];
+  }
+#if PDE_USE_B
+  if (wave == FLUX_SPLIT - 1) {
+    face_state<d>(tr, trd, g, it, 0, qL, dqL);
+    face_state<d>(tr, trd, g, it, 1, qR, dqR);
+    face_b<d>(qL, qR, fb, o, nf);
+  }
+#endif
+}
+#else
+constexpr int FLUX_SPLIT = 1;
+#endif
+#endif  // PDE_V <= 8
+
+// Every direction's faces in one launch: the workgroups of direction 0, then
+// those of direction 1 (flux_blocks on the host); one nearly empty last round
+// of wavefronts instead of one per direction (Osher on 128 x 128: 168 -> 131
+// us; the 1024 x 256 channel 334 -> 314; 2048 x 2048 at order 2 1845 -> 1789).  MODE 0: one thread per face
+// point, BS threads per workgroup; 1: split over FLUX_SPLIT wavefronts per 64
+// points.  Above V = 8 a workgroup takes one face point.
+template <int MODE, int BS>
+DEV void flux_all(const double* __restrict__ tr, const FaceOut& out, const Geom& g,
+                  const double* __restrict__ trd, const Blk& b) {
+  constexpr int POINTS = V > 8 ? 1 : MODE ? 64 : BS;
+  const unsigned int nb0 =
+      D == 1 ? ~0u : (unsigned int)((g.nf[0] * (N * ND1) + POINTS - 1) / POINTS);
+#if PDE_V > 8
+  (void)trd;
+  if (b.x < nb0) flux_wide<0>(tr, out.ff[0], out.fb[0], g, b.x);
+#if PDE_D >= 2
+  else flux_wide<1>(tr, out.ff[1], out.fb[1], g, b.x - nb0);
+#endif
+#else
+#if PDE_USE_F
+  if constexpr (MODE == 1) {
+    __shared__ FluxShared sm;
+    if (b.x < nb0) flux_split<0>(sm, tr, out.ff[0], out.fb[0], g, trd, b.x);
+#if PDE_D >= 2
+    else flux_split<1>(sm, tr, out.ff[1], out.fb[1], g, trd, b.x - nb0);
+#endif
+    return;
+  }
+#endif
+  if (b.x < nb0) flux_point<0, POINTS>(tr, out.ff[0], out.fb[0], g, trd, b.x);
+#if PDE_D >= 2
+  else flux_point<1, POINTS>(tr, out.ff[1], out.fb[1], g, trd, b.x - nb0);
+#endif
+#endif
+}
+
+// k_flux: 128 threads (one face point each; above V = 8 one point together),
+// k_flux_64: 64 threads, k_flux_split: FLUX_SPLIT wavefronts per 64 points.
+// The autotuner picks one per problem; every face point's arithmetic is the
+// same.
+#define PYPDE_FLUX_KERNEL(NAME, MODE, BS)                                                      \
+  extern "C" __global__ void __launch_bounds__(BS)                                             \
+  NAME(const double* __restrict__ tr, FaceOut out, const StepState* st, Geom g,                \
+       const double* __restrict__ trd) {                                                       \
+    if (st->done) return;                                                                      \
+    flux_all<MODE, BS>(tr, out, g, trd, hw_blk());                                             \
+  }
+PYPDE_FLUX_KERNEL(k_flux, 0, 128)
 #if PDE_V <= 8
-PYPDE_FLUX_KERNEL(k_flux0_128, 0, 128)
-PYPDE_FLUX_KERNEL(k_flux0_64, 0, 64)
-#if PDE_D >= 2
-PYPDE_FLUX_KERNEL(k_flux1_128, 1, 128)
-PYPDE_FLUX_KERNEL(k_flux1_64, 1, 64)
-#endif
+PYPDE_FLUX_KERNEL(k_flux_64, 0, 64)
+PYPDE_FLUX_KERNEL(k_flux_split, 1, 64 * FLUX_SPLIT)
 #endif
 
 // ------------------------------------------------------------- corrector
@@ -2349,24 +2517,18 @@ k_predictor_hot_b(const Member* ms, const BlkMap* map, int nm, double newton_tol
 #endif
 #endif  // PDE_V <= 8
 
-#define PYPDE_FLUX_BATCH(NAME, DIR, BS)                                                        \
+#define PYPDE_FLUX_BATCH(NAME, MODE, BS)                                                       \
   extern "C" __global__ void __launch_bounds__(BS)                                             \
   NAME(const Member* ms, const BlkMap* map, int nm) {                                          \
     PYPDE_BATCH_MEMBER                                                                         \
     if (M.st->done) return;                                                                    \
-    flux_dir<DIR, BS>(M.tr, M.ff[DIR], M.fb[DIR], M.st, M.g, M.trd, b);                        \
+    const FaceOut out = {{M.ff[0], M.ff[1]}, {M.fb[0], M.fb[1]}};                              \
+    flux_all<MODE, BS>(M.tr, out, M.g, M.trd, b);                                              \
   }
-PYPDE_FLUX_BATCH(k_flux0_b, 0, FLUX_BS0)
-#if PDE_D >= 2
-PYPDE_FLUX_BATCH(k_flux1_b, 1, FLUX_BS0)
-#endif
+PYPDE_FLUX_BATCH(k_flux_b, 0, 128)
 #if PDE_V <= 8
-PYPDE_FLUX_BATCH(k_flux0_128_b, 0, 128)
-PYPDE_FLUX_BATCH(k_flux0_64_b, 0, 64)
-#if PDE_D >= 2
-PYPDE_FLUX_BATCH(k_flux1_128_b, 1, 128)
-PYPDE_FLUX_BATCH(k_flux1_64_b, 1, 64)
-#endif
+PYPDE_FLUX_BATCH(k_flux_64_b, 0, 64)
+PYPDE_FLUX_BATCH(k_flux_split_b, 1, 64 * FLUX_SPLIT)
 #endif
 
 extern "C" __global__ void __launch_bounds__(256)

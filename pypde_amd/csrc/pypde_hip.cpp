@@ -110,6 +110,10 @@ struct FaceBufs {
   const double* ff[2];
   const double* fb[2];
 };
+struct FaceOut {
+  double* ff[2];
+  double* fb[2];
+};
 
 // Must match Member / BlkMap of the batched ensemble kernels (ader_step.h).
 struct Member {
@@ -303,30 +307,29 @@ int check_spec(const Spec& s, bool secondOrder, int FLUX) {
   return 0;
 }
 
-enum { K_WENO, K_DT, K_PRED, K_FLUX0, K_FLUX1, K_UPDATE, K_A2S, K_S2A,
+enum { K_WENO, K_DT, K_PRED, K_FLUX, K_UPDATE, K_A2S, K_S2A,
        K_HARVEST, K_MLPGUESS, K_PRED_STATIC, K_PRED_STATIC2, K_EIG, K_P2R, K_PRED32,
-       K_WENO_4x64, K_WENO_16x16, K_WENO_16x32, K_FLUX0_128, K_FLUX0_64, K_FLUX1_128, K_FLUX1_64,
+       K_WENO_4x64, K_WENO_16x16, K_WENO_16x32, K_FLUX_64, K_FLUX_SPLIT,
        K_UPD1, K_UPD2, K_UPD4, K_UPD8, K_PRED_COLD, K_PRED_HOT, K_MLPPACK, K_PRED_COLD3,
        // batched ensemble kernels (modules built with PDE_BATCH only)
        K_B_WENO, K_B_WENO_4x64, K_B_WENO_16x16, K_B_WENO_16x32, K_B_DT, K_B_PRED_STATIC,
-       K_B_PRED_STATIC2, K_B_PRED_COLD, K_B_PRED_COLD3, K_B_PRED_HOT, K_B_FLUX0, K_B_FLUX0_128,
-       K_B_FLUX0_64, K_B_FLUX1, K_B_FLUX1_128, K_B_FLUX1_64, K_B_UPDATE, K_B_UPD1, K_B_UPD2,
+       K_B_PRED_STATIC2, K_B_PRED_COLD, K_B_PRED_COLD3, K_B_PRED_HOT, K_B_FLUX, K_B_FLUX_64,
+       K_B_FLUX_SPLIT, K_B_UPDATE, K_B_UPD1, K_B_UPD2,
        K_B_UPD4, K_B_UPD8, K_COUNT };
 const char* kernel_names[K_COUNT] = {"k_weno",   "k_dt",    "k_predictor",
-                                     "k_flux0",  "k_flux1", "k_update",
+                                     "k_flux", "k_update",
                                      "k_aos_to_soa", "k_soa_to_aos", "k_harvest", "k_mlp_guess",
                                      "k_predictor_static", "k_predictor_static2", "k_eig_batch",
                                      "k_planes_to_rows", "k_predictor_f32",
                                      "k_weno_4x64", "k_weno_16x16", "k_weno_16x32",
-                                     "k_flux0_128", "k_flux0_64", "k_flux1_128", "k_flux1_64",
+                                     "k_flux_64", "k_flux_split",
                                      "k_update_r1", "k_update_r2", "k_update_r4", "k_update_r8",
                                      "k_predictor_cold", "k_predictor_hot", "k_mlp_pack",
                                      "k_predictor_cold3",
                                      "k_weno_b", "k_weno_4x64_b", "k_weno_16x16_b", "k_weno_16x32_b",
                                      "k_dt_b", "k_predictor_static_b", "k_predictor_static2_b",
                                      "k_predictor_cold_b", "k_predictor_cold3_b", "k_predictor_hot_b",
-                                     "k_flux0_b", "k_flux0_128_b", "k_flux0_64_b",
-                                     "k_flux1_b", "k_flux1_128_b", "k_flux1_64_b",
+                                     "k_flux_b", "k_flux_64_b", "k_flux_split_b",
                                      "k_update_b", "k_update_r1_b", "k_update_r2_b", "k_update_r4_b",
                                      "k_update_r8_b"};
 
@@ -339,14 +342,11 @@ const char* kernel_names[K_COUNT] = {"k_weno",   "k_dt",    "k_predictor",
 constexpr int N_WENO_V = 4, N_FLUX_V = 3, N_UPD_V = 5, N_PRED_V = 4;
 const int WENO_TILE[N_WENO_V][2] = {{8, 32}, {4, 64}, {16, 16}, {16, 32}};
 const int WENO_KID[N_WENO_V] = {K_WENO, K_WENO_4x64, K_WENO_16x16, K_WENO_16x32};
-const int FLUX_BS[N_FLUX_V] = {256, 128, 64};
-const int FLUX_KID[2][N_FLUX_V] = {{K_FLUX0, K_FLUX0_128, K_FLUX0_64},
-                                   {K_FLUX1, K_FLUX1_128, K_FLUX1_64}};
+const int FLUX_KID[N_FLUX_V] = {K_FLUX, K_FLUX_64, K_FLUX_SPLIT};
 const int UPD_KID[N_UPD_V] = {K_UPDATE, K_UPD1, K_UPD2, K_UPD4, K_UPD8};
 const int UPD_ROWS[N_UPD_V] = {0, 1, 2, 4, 8};
 const int B_WENO_KID[N_WENO_V] = {K_B_WENO, K_B_WENO_4x64, K_B_WENO_16x16, K_B_WENO_16x32};
-const int B_FLUX_KID[2][N_FLUX_V] = {{K_B_FLUX0, K_B_FLUX0_128, K_B_FLUX0_64},
-                                     {K_B_FLUX1, K_B_FLUX1_128, K_B_FLUX1_64}};
+const int B_FLUX_KID[N_FLUX_V] = {K_B_FLUX, K_B_FLUX_64, K_B_FLUX_SPLIT};
 const int B_UPD_KID[N_UPD_V] = {K_B_UPDATE, K_B_UPD1, K_B_UPD2, K_B_UPD4, K_B_UPD8};
 
 struct MLPW {
@@ -492,10 +492,8 @@ int load_module(const Spec& spec, int device, hipModule_t* mod, hipFunction_t* f
     return fail(PYPDE_ERR_HIP, "hipModuleLoadData failed");
   for (int k = 0; k < K_COUNT; k++) {
     e.fn[k] = nullptr;
-    bool optional = ((k == K_FLUX1 || k == K_FLUX1_128 || k == K_FLUX1_64) && spec.D < 2) ||
-                    ((k == K_FLUX0_128 || k == K_FLUX0_64 || k == K_FLUX1_128 ||
-                      k == K_FLUX1_64) && spec.V > WIDE_V) ||
-                    ((k == K_PRED || k == K_PRED_STATIC2) && spec.V > WIDE_V) ||
+    bool optional = ((k == K_FLUX_64 || k == K_FLUX_SPLIT || k == K_PRED ||
+                      k == K_PRED_STATIC2) && spec.V > WIDE_V) ||
                     k == K_MLPGUESS || k == K_MLPPACK || (k == K_PRED32 && !spec.mixed) ||
                     k == K_PRED_COLD || k == K_PRED_HOT || k == K_PRED_COLD3 || k >= K_B_WENO;
     if (hipModuleGetFunction(&e.fn[k], e.mod, kernel_names[k]) != hipSuccess) {
@@ -525,13 +523,23 @@ int launch(pypde_ctx* c, int k, dim3 grid, dim3 block, std::vector<void*>& args)
 
 long cdiv(long a, long b) { return (a + b - 1) / b; }
 
-// Face-flux launch of one direction: variants and threads per workgroup, and
-// workgroups for `items` face points (above WIDE_V one face point per
-// workgroup of 128 threads).
+// Face-flux launches (FLUX_SPLIT and flux_all in ader_step.h): variants,
+// threads per workgroup, and workgroups over every direction's faces.
 int flux_variants(int V) { return V > WIDE_V ? 1 : N_FLUX_V; }
-int flux_threads(int V, int variant) { return V > WIDE_V ? 128 : FLUX_BS[variant]; }
-long flux_blocks(int V, int variant, long items) {
-  return V > WIDE_V ? items : cdiv(items, FLUX_BS[variant]);
+int flux_threads(const Spec& s, int variant) {
+  if (s.V > WIDE_V || variant == 0) return 128;
+  if (variant == 1) return 64;
+  const int parts = !s.useF ? 1 : s.flux == 0 ? 2 : s.flux == 1 ? 1 : s.N;
+  return 64 * (parts + (s.useF && s.second ? 2 : 0));
+}
+long flux_blocks(const Spec& s, int variant, const Geom& g) {
+  const long points = s.V > WIDE_V ? 1 : variant == 0 ? 128 : 64;
+  long blocks = 0;
+  for (int d = 0; d < s.D; d++) {
+    const long items = g.nf[d] * s.N * (s.D == 2 ? s.N : 1);
+    blocks += cdiv(items, points);
+  }
+  return blocks;
 }
 
 // Callers built against the older, shorter pypde_stats leave out the node
@@ -652,20 +660,19 @@ int enqueue_step(pypde_ctx* c, bool guess_now, std::vector<hipEvent_t>* evs) {
     }
   }
   mark();
-  for (int d = 0; d < c->D; d++) {
+  {
     const double* t = c->tr;
-    double *f = c->ff[d], *b = c->fb[d];
+    FaceOut out = {{c->ff[0], c->ff[1]}, {c->fb[0], c->fb[1]}};
     const StepState* st = c->st;
     const double* td = c->trd;
-    std::vector<void*> a = {&t, &f, &b, &st, &g, &td};
-    long items = g.nf[d] * c->N * (c->ND / c->N);
-    if ((rc = launch(c, FLUX_KID[d][c->tune.flux],
-                     dim3((unsigned)flux_blocks(c->V, c->tune.flux, items)),
-                     dim3(flux_threads(c->V, c->tune.flux)), a)))
+    std::vector<void*> a = {&t, &out, &st, &g, &td};
+    if ((rc = launch(c, FLUX_KID[c->tune.flux],
+                     dim3((unsigned)flux_blocks(c->spec, c->tune.flux, g)),
+                     dim3(flux_threads(c->spec, c->tune.flux)), a)))
       return rc;
-    mark();
   }
-  if (c->D == 1) mark();
+  mark();
+  mark();  // both directions run in the one launch: the second flux slot times nothing
   {
     double* uu = c->u;
     const double* v = c->vol;
@@ -864,7 +871,7 @@ static pypde_ctx* create_ctx(const char* src, bool useF, bool useB, bool useS, c
   c->NT = c->ND * N;
   c->CPW = V > WIDE_V ? 1 : 64 / c->ND;
   // DT_LANES in ader_kernels.h
-  c->dt_lanes = V > WIDE_V ? 64 : (ndim == 2 && V <= 5 && !secondOrder) ? 2 : 1;
+  c->dt_lanes = V > WIDE_V ? 64 : secondOrder ? 2 * ndim : (ndim == 2 && V <= 5) ? 2 : 1;
   c->device = opts.device;
   // Predictor schedule: the autotuner picks among the static one (one
   // wavefront per group of CPW cells), the persistent work-queued kernel and
@@ -1354,7 +1361,7 @@ int pypde_step(pypde_ctx* c, long steps, double tf, pypde_stats* stats) {
 
 // ------------------------------------------------------------ ensembles
 // Stages of a batched ensemble step, each one launch per group of members.
-enum { BS_WENO, BS_DT, BS_PRED, BS_FLUX0, BS_FLUX1, BS_UPDATE, BS_COUNT };
+enum { BS_WENO, BS_DT, BS_PRED, BS_FLUX, BS_UPDATE, BS_COUNT };
 
 // Members advanced by the same launches: entries [first, first + count) of
 // the member table, workgroup maps at map (BS_COUNT x (count + 1) entries),
@@ -1410,7 +1417,7 @@ static int batch_setup(pypde_ensemble* e, long cap) {
   std::stable_sort(order.begin(), order.end(),
                    [&](int a, int b) { return e->m[a]->g.nwc > e->m[b]->g.nwc; });
   const pypde_ctx* c0 = e->m[0];
-  const int D = c0->D, N = c0->N, V = c0->V, ND = c0->ND, CPW = c0->CPW;
+  const int D = c0->D, V = c0->V, CPW = c0->CPW;
   e->groups.clear();
   long cells = 0;
   for (int k = 0; k < nm; k++) {
@@ -1457,12 +1464,7 @@ static int batch_setup(pypde_ensemble* e, long cap) {
             break;
           case BS_DT: gx = cdiv(g.nwc * mc->dt_lanes, 256); break;
           case BS_PRED: gx = cdiv(g.nwc, CPW); break;
-          case BS_FLUX0:
-          case BS_FLUX1: {
-            const int d = s - BS_FLUX0;
-            gx = d < D ? flux_blocks(V, gr.flux, g.nf[d] * N * (ND / N)) : 0;
-            break;
-          }
+          case BS_FLUX: gx = flux_blocks(c0->spec, gr.flux, g); break;
           default: {
             const int R = UPD_ROWS[gr.update];
             gx = cdiv(R == 0 ? g.ncell : (long)V * cdiv(g.nx[0], R) * g.nx[1], 256);
@@ -1541,9 +1543,7 @@ static int enqueue_group_step(pypde_ensemble* e, const EnsGroup& gr) {
   } else if ((rc = go(gr.pred == 1 ? K_B_PRED_STATIC2 : K_B_PRED_STATIC, BS_PRED, 64, true))) {
     return rc;
   }
-  for (int d = 0; d < c->D; d++)
-    if ((rc = go(B_FLUX_KID[d][gr.flux], BS_FLUX0 + d, flux_threads(c->V, gr.flux), false)))
-      return rc;
+  if ((rc = go(B_FLUX_KID[gr.flux], BS_FLUX, flux_threads(c->spec, gr.flux), false))) return rc;
   return go(B_UPD_KID[gr.update], BS_UPDATE, 256, false);
 }
 

@@ -181,7 +181,7 @@ class Solver:
         ms = np.zeros(4)
         _capi.check(_capi.lib().pypde_get_tuning(self.h, _capi.ip(ch), _capi.dp(ms)), "tuning")
         weno = ["8x32", "4x64", "16x16", "16x32"][ch[0]]
-        flux = [256, 128, 64][ch[1]]
+        flux = [128, 64, "split"][ch[1]]
         upd = ["cell", "rows1", "rows2", "rows4", "rows8"][ch[2]]
         pred = ["static", "queue", "split", "split3"][ch[3]]
         src = ["defaults", "measured", "table", "forced"][ch[4]]
