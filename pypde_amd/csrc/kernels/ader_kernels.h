@@ -4,8 +4,9 @@
 // Device data layout (structure of arrays, cell index fastest):
 //   u   [V][ncell]                          interior state
 //   wh  [N^D * V][nwc]                      reconstruction, plane = node*V + v
-//   tr  [2*D*N*N^(D-1)*V][nwc]              face traces of the predictor,
-//                                           plane = (((d*2+e)*N+t)*N^(D-1)+j)*V+v
+//   tr  [2*D*N*N^(D-1)][ntb][V][TCW]        face traces of the predictor, plane
+//                                           ((d*2+e)*N+t)*N^(D-1)+j; TCW cells per
+//                                           block (trace_at)
 //   vol [V][nwc]                            volume (source / B) integral
 //   ff, fb [N*N^(D-1)*V][nf_d] per d        face flux / B path integral
 // nwc = prod(nx_d + 2) reconstructed cells (one ghost layer, iterator.cpp:76).
@@ -28,7 +29,20 @@ struct Geom {
   // item index and every w-cell index is below 2^31.
   unsigned fmul[2], fsh[2], rmul[2], rsh[2];
   int idx32;
+  long ntb;  // trace blocks: ceil(nwc / TCW)
 };
+
+// Face traces in blocks of the TCW cells one predictor wavefront holds, their
+// variables together: a wavefront writes whole cache lines (V TCW doubles a
+// block: 128 bytes at order 4 with four variables, where rows of 4 cells in
+// planes of one variable were 32-byte pieces that four wavefronts had to
+// complete), and what a face point reads of a block, its V variables, lies in
+// the same lines (2048 x 2048 at order 2, predictor 848 -> 729 us: it writes
+// 2.1 GB of traces, which is what bounds it).
+constexpr int TCW = V > 8 ? 1 : 64 / ND;
+DEV long trace_at(const Geom& g, int plane, long block, int slot) {
+  return ((long)plane * g.ntb + block) * (V * TCW) + slot;  // + v * TCW
+}
 
 // n / d for n < 2^31 from d's multiplier m = ceil(2^sh / d), sh = 31 +
 // ceil(log2 d): with n = q d + r, n m / 2^sh = q + (r + n e / 2^sh) / d, e =
@@ -45,7 +59,6 @@ struct StepState {
   unsigned int nan_flag, pad2;
   unsigned long long pred_iters, pred_cells, pred_capped, pred_fallbacks;
   unsigned int pred_maxit, pad3;
-  unsigned long long qhead;     // predictor work queue: next unclaimed w-cell
   // stiff predictor: Newton corrections per spatial node with the full source
   // Jacobian solve and with the A = 0 shortcut, summed over nodes and steps
   unsigned long long pred_nfull, pred_nshort;
@@ -446,7 +459,6 @@ DEV void dt_finalize(StepState* st) {
   if (st->count <= 5) dt = dt * 0.2;
   if (st->t + dt > st->tf) dt = st->tf - st->t;
   st->dt = dt;
-  st->qhead = 0ull;
   st->hot_count = 0ull;
 }
 

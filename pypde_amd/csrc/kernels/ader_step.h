@@ -149,15 +149,21 @@ DEV void node_ctx(NodeCtx& c, int lane, NodeTab* nt) {
 // iterate then need not be staged in LDS every iteration.
 constexpr bool PRED_DQ = PDE_SECOND || PDE_USE_B;
 
-// derivative along d at this lane's node of buffer buf[slot][t][node][v]
-template <int d, int NTB>
-DEV void lds_deriv(const NodeCtx& c, const double (*buf)[NTB][ND][V], int t, double rdx, double* out) {
+// Row stride of the exchange buffers in doubles: odd, so that neighbouring
+// nodes' rows start in different banks (with V = 4 rows 32 bytes apart, two
+// thirds of the Picard predictor's cycles were bank conflicts: 512 x 512 at
+// order 4, 502 -> 332 us).
+constexpr int VL = V | 1;
+
+// derivative along d at this lane's node of buffer buf[t][slot][node][v]
+template <int d>
+DEV void lds_deriv(const NodeCtx& c, const double (*buf)[CPW][ND][VL], int t, double rdx, double* out) {
   constexpr int stride = ipow_c(N, D - 1 - d);
 #pragma unroll
   for (int v = 0; v < V; v++) {
-    double acc = c.der(d, 0) * buf[c.slot][t][c.base[d]][v];
+    double acc = c.der(d, 0) * buf[t][c.slot][c.base[d]][v];
 #pragma unroll
-    for (int j = 1; j < N; j++) acc = dfma(c.der(d, j), buf[c.slot][t][c.base[d] + j * stride][v], acc);
+    for (int j = 1; j < N; j++) acc = dfma(c.der(d, j), buf[t][c.slot][c.base[d] + j * stride][v], acc);
     out[v] = acc * rdx;
   }
 }
@@ -175,9 +181,17 @@ DEV void callS(double* out, const double* q) {
 // F, whose gradient traces need every time node's derivatives (NTF = N).
 constexpr int NTF = PDE_SECOND ? N : 1;
 struct PredLDS {
-  double q[CPW][N][ND][V];
+#if PDE_SECOND || PDE_USE_B
+  double q[N][CPW][ND][VL];
 #if PDE_USE_F
-  double f[D][CPW][NTF][ND][V];
+  double f[D][NTF][CPW][ND][VL];
+#endif
+#else
+  // without PRED_DQ q is staged only after the iterations, over f
+  union {
+    double q[N][CPW][ND][VL];
+    double f[D][NTF][CPW][ND][VL];
+  };
 #endif
 #if PDE_GUESS
   double red[64];  // per-lane residuals of the learned-guess check
@@ -209,7 +223,7 @@ DEV void grad_traces(const NodeCtx& c, PredLDS& sm, const Geom& g, long cell, bo
         double tmp[V];
         lds_deriv<d_>(c, sm.q, t, 1.0 / g.dX[d_], tmp);
 #pragma unroll
-        for (int v = 0; v < V; v++) sm.f[d_][c.slot][t][c.idx][v] = tmp[v];
+        for (int v = 0; v < V; v++) sm.f[d_][t][c.slot][c.idx][v] = tmp[v];
       }
     });
   }
@@ -228,10 +242,10 @@ DEV void grad_traces(const NodeCtx& c, PredLDS& sm, const Geom& g, long cell, bo
             for (int d_ = 0; d_ < D; d_++)
 #pragma unroll
               for (int v = 0; v < V; v++) {
-                double acc = (e ? T_END1[0] : T_END0[0]) * sm.f[d_][c.slot][t][c.idx][v];
+                double acc = (e ? T_END1[0] : T_END0[0]) * sm.f[d_][t][c.slot][c.idx][v];
 #pragma unroll
                 for (int m = 1; m < N; m++)
-                  acc = dfma(e ? T_END1[m] : T_END0[m], sm.f[d_][c.slot][t][c.idx + m * stride][v], acc);
+                  acc = dfma(e ? T_END1[m] : T_END0[m], sm.f[d_][t][c.slot][c.idx + m * stride][v], acc);
                 const int plane = ((((d * 2 + e) * N + t) * ND1 + j) * D + d_) * V + v;
                 trd[(long)plane * g.nwc + cell] = acc;
               }
@@ -267,7 +281,7 @@ DEV void node_rhs(const NodeCtx& c, PredLDS& sm, const double (&q)[N][V], const 
       double f[V];
       F(f, q[t], &dqs[t][0][0], d);
 #pragma unroll
-      for (int v = 0; v < V; v++) sm.f[d][c.slot][slot_t][c.idx][v] = f[v];
+      for (int v = 0; v < V; v++) sm.f[d][slot_t][c.slot][c.idx][v] = f[v];
     }
 #else
     (void)slot_t;
@@ -350,7 +364,7 @@ DEV void node_rhs_const(const NodeCtx& c, PredLDS& sm, const double (&q)[N][V], 
       double f[V];
       F(f, q[0], &dqs[0][0][0], d);
 #pragma unroll
-      for (int v = 0; v < V; v++) sm.f[d][c.slot][0][c.idx][v] = f[v];
+      for (int v = 0; v < V; v++) sm.f[d][0][c.slot][c.idx][v] = f[v];
     }
 #endif
   }
@@ -599,293 +613,17 @@ DEV bool newton_node(const NodeCtx& c, const double (&q)[N][V], double (&G)[N][V
 #endif
 
 #if PDE_V <= 8  // above, ader_wide_predictor.h
-// Persistent, work-queued: each wavefront claims cells from st->qhead (reset
-// by k_dt's last workgroup every step), iterates its CPW slots, and as soon as a slot's
-// cell has converged writes that cell's outputs and refills the slot with the
-// next unclaimed cell, so cells with many Newton iterations do not hold the
-// lanes of cells that need few.  Every cell's arithmetic is independent of
-// which slot or wavefront runs it.
-extern "C" __global__ void __launch_bounds__(64)
-k_predictor(const double* __restrict__ wh, const double* __restrict__ guess,
-            double* __restrict__ tr, double* __restrict__ vol, double* __restrict__ qh,
-            StepState* st, Geom g, double newton_tol, int newton_maxit,
-            double* __restrict__ trd) {
-  if (st->done) return;
-  __shared__ PredLDS sm;
-  const double dt = st->dt;
-  const int lane = threadIdx.x;
-  NodeCtx c;
-  node_ctx(c, lane, PRED_NODE_TAB(sm));
-  const bool lane_ok = c.slot < CPW;
-  const unsigned long long cellmask =
-      (ND == 64 ? ~0ull : ((1ull << ND) - 1ull)) << (lane_ok ? c.slot * ND : 0);
-#if PDE_STIFF
-  const int maxit = newton_maxit;
-#else
-  const int maxit = DG_IT;
-#endif
-  double w[V], q[N][V], rhs[N][V], dqs[N][D][V];
-  long cell = -1;
-  bool active = false;
-  int it = 0;
-  int learned = 0;
-  int fellback = 0;
-  double r0 = 0.0;
-  // per-lane statistics over the cells this lane's slot has run
-  unsigned long long s_iters = 0ull, s_cells = 0ull, s_cap = 0ull, s_fb = 0ull;
-  unsigned int s_max = 0u;
-  unsigned int n_full = 0u, n_short = 0u;  // node corrections of this lane
-
-  auto start_cell = [&](long cl) {
-    cell = cl;
-    active = cl >= 0;
-    it = 0;
-    fellback = 0;
-    r0 = 0.0;
-    learned = (PDE_GUESS && guess) ? 1 : 0;
-    if (active) {
-#pragma unroll
-      for (int v = 0; v < V; v++) w[v] = wh[(long)(c.idx * V + v) * g.nwc + cl];
-#pragma unroll
-      for (int t = 0; t < N; t++)
-#pragma unroll
-        for (int v = 0; v < V; v++)
-          q[t][v] = (PDE_GUESS && guess) ? guess[(long)((t * ND + c.idx) * V + v) * g.nwc + cl]
-                                         : w[v];
-    }
-  };
-  {
-    long long base = 0;
-    if (lane == 0) base = (long long)atomicAdd(&st->qhead, (unsigned long long)CPW);
-    base = __shfl(base, 0, 64);
-    long cl = (long)base + c.slot;
-    start_cell((lane_ok && cl < g.nwc) ? cl : -1);
-  }
-
-  while (__ballot(active) != 0ull) {
-    if (PRED_DQ && active) {
-#pragma unroll
-      for (int t = 0; t < N; t++)
-#pragma unroll
-        for (int v = 0; v < V; v++) sm.q[c.slot][t][c.idx][v] = q[t][v];
-    }
-    pred_sync();
-    node_rhs(c, sm, q, w, dt, g, active, rhs, dqs);
-    bool more = false;
-    bool skip = false;
-#if PDE_STIFF
-    // residual G = rhs - (DG_MAT (x) W) q   (dg.cpp:128-154)
-    double rmax = 0.0;
-    if (active) {
-#pragma unroll
-      for (int t = 0; t < N; t++)
-#pragma unroll
-        for (int v = 0; v < V; v++) {
-          double acc = (T_DGMAT[t][0] * c.WP()) * q[0][v];
-#pragma unroll
-          for (int s2 = 1; s2 < N; s2++) acc = dfma(T_DGMAT[t][s2] * c.WP(), q[s2][v], acc);
-          rhs[t][v] = rhs[t][v] - acc;
-          double a = dabs(rhs[t][v]);
-          rmax = (a > rmax || a != a) ? a : rmax;  // keeps a NaN
-        }
-    }
-#if PDE_GUESS
-    // while a cell is still on its learned guess, a residual that is not finite
-    // or larger than at the previous iterate sends it back to the plain guess
-    if (__ballot(active && learned) != 0ull) {
-      pred_sync();
-      sm.red[lane] = rmax;
-      pred_sync();
-      double cm = 0.0;
-#pragma unroll
-      for (int i = 0; i < ND; i++) {
-        double e = sm.red[(lane_ok ? c.slot : 0) * ND + i];
-        cm = (e > cm || e != e) ? e : cm;  // max that keeps a NaN
-      }
-      if (active && learned) {
-        if (!(cm <= (it > 0 ? r0 : 1.7976931348623157e308))) {
-#pragma unroll
-          for (int t = 0; t < N; t++)
-#pragma unroll
-            for (int v = 0; v < V; v++) q[t][v] = w[v];
-          fellback = 1;
-          learned = 0;
-          skip = true;
-        } else {
-          r0 = cm;
-        }
-      }
-    }
-#endif
-    if (active && !skip) {
-      if (newton_node(c, q, rhs, dt)) n_full++;
-      else n_short++;
-#pragma unroll
-      for (int t = 0; t < N; t++)
-#pragma unroll
-        for (int v = 0; v < V; v++) {
-          if (!(dabs(rhs[t][v]) <= newton_tol * (1.0 + dabs(q[t][v])))) more = true;
-          q[t][v] = q[t][v] + rhs[t][v];
-        }
-    }
-    if (skip) more = true;
-#else
-    (void)learned;
-    (void)r0;
-    (void)newton_tol;
-    if (active) {
-      // Picard: q1 = DG_MAT^-1 rhs / prod W  (dg.cpp:187-202)
-#pragma unroll
-      for (int t = 0; t < N; t++)
-#pragma unroll
-        for (int v = 0; v < V; v++) {
-          double acc = T_DGINV[t][0] * rhs[0][v];
-#pragma unroll
-          for (int s2 = 1; s2 < N; s2++) acc = dfma(T_DGINV[t][s2], rhs[s2][v], acc);
-          double q1 = acc * c.IWP();
-          if (dabs(q1 - q[t][v]) > DG_TOL * (1.0 + dabs(q[t][v]))) more = true;
-          q[t][v] = q1;
-        }
-    }
-#endif
-    const unsigned long long mb = __ballot(more);
-    bool fin = false;
-    if (active) {
-      it++;
-      if ((mb & cellmask) == 0ull || it >= maxit) {
-        active = false;
-        fin = true;
-      }
-    }
-    pred_sync();
-    if (__ballot(fin) == 0ull) continue;
-
-    // ---- finished slots: traces, volume term, optional full qh
-    if (fin) {
-#pragma unroll
-      for (int t = 0; t < N; t++)
-#pragma unroll
-        for (int v = 0; v < V; v++) sm.q[c.slot][t][c.idx][v] = q[t][v];
-    }
-    pred_sync();
-    if (fin) {
-      static_for<0, D>([&](auto dc) {
-        constexpr int d = decltype(dc)::value;
-        constexpr int stride = ipow_c(N, D - 1 - d);
-        if (c.kd[d] == 0) {
-          const int j = (c.idx / (stride * N)) * stride + c.idx % stride;
-#pragma unroll
-          for (int e = 0; e < 2; e++)
-#pragma unroll
-            for (int t = 0; t < N; t++)
-#pragma unroll
-              for (int v = 0; v < V; v++) {
-                double acc = (e ? T_END1[0] : T_END0[0]) * sm.q[c.slot][t][c.idx][v];
-#pragma unroll
-                for (int m = 1; m < N; m++)
-                  acc = dfma(e ? T_END1[m] : T_END0[m], sm.q[c.slot][t][c.idx + m * stride][v], acc);
-                const int plane = (((d * 2 + e) * N + t) * ND1 + j) * V + v;
-                tr[(long)plane * g.nwc + cell] = acc;
-              }
-        }
-      });
-      if (qh) {
-#pragma unroll
-        for (int t = 0; t < N; t++)
-#pragma unroll
-          for (int v = 0; v < V; v++) qh[(long)((t * ND + c.idx) * V + v) * g.nwc + cell] = q[t][v];
-      }
-    }
-#if PDE_SECOND
-    grad_traces(c, sm, g, cell, fin, trd);
-#endif
-#if PDE_USE_S || PDE_USE_B
-    // volume term (fv.cpp:33-85): per node sum over t, then over nodes in order
-    double part[V];
-    if (fin) {
-#pragma unroll
-      for (int t = 0; t < N; t++) {
-        double sv[V];
-        callS(sv, q[t]);
-#if PDE_USE_B
-        static_for<0, D>([&](auto dc) {
-          constexpr int d = decltype(dc)::value;
-          double dqd[V], b[V * V], bd[V];
-          lds_deriv<d>(c, sm.q, t, 1.0 / g.dX[d], dqd);
-          B(b, q[t], d);
-          b_times<PDE_B_QUIRK ? 2 : 0>(b, dqd, bd);
-#pragma unroll
-          for (int v = 0; v < V; v++) sv[v] = sv[v] - bd[v];
-        });
-#endif
-        double tmp = dt * T_W[t];
-#pragma unroll
-        for (int d = 0; d < D; d++) tmp = tmp * c.wk(d);
-#pragma unroll
-        for (int v = 0; v < V; v++) part[v] = (t == 0) ? tmp * sv[v] : dfma(tmp, sv[v], part[v]);
-      }
-    }
-    pred_sync();
-    if (fin) {
-#pragma unroll
-      for (int v = 0; v < V; v++) sm.q[c.slot][0][c.idx][v] = part[v];
-    }
-    pred_sync();
-    if (fin && c.idx == 0) {
-#pragma unroll
-      for (int v = 0; v < V; v++) {
-        double acc = sm.q[c.slot][0][0][v];
-#pragma unroll
-        for (int i = 1; i < ND; i++) acc = acc + sm.q[c.slot][0][i][v];
-        vol[(long)v * g.nwc + cell] = acc;
-      }
-    }
-    pred_sync();
-#endif
-    if (fin && c.idx == 0) {
-      s_iters += (unsigned long long)it;
-      s_cells += 1ull;
-      s_cap += (it >= maxit) ? 1ull : 0ull;
-      s_fb += (unsigned long long)fellback;
-      s_max = (unsigned int)it > s_max ? (unsigned int)it : s_max;
-    }
-    // ---- refill finished slots with the next unclaimed cells, in slot order
-    const unsigned long long lead = __ballot(fin && c.idx == 0);
-    long long base = 0;
-    if (lane == 0) base = (long long)atomicAdd(&st->qhead, (unsigned long long)__popcll(lead));
-    base = __shfl(base, 0, 64);
-    if (fin) {
-      const unsigned long long below = lead & ((1ull << (c.slot * ND)) - 1ull);
-      long cl = (long)base + __popcll(below);
-      start_cell(cl < g.nwc ? cl : -1);
-    }
-  }
-  // ---- statistics
-  s_iters = wave_sum_u64(s_iters);
-  s_cells = wave_sum_u64(s_cells);
-  s_cap = wave_sum_u64(s_cap);
-  s_fb = wave_sum_u64(s_fb);
-  s_max = wave_max_u32(s_max);
-  const unsigned long long w_full = wave_sum_u64(n_full), w_short = wave_sum_u64(n_short);
-  if (lane == 0 && s_cells) {
-    unsigned long long* ps = st->pstat[blockIdx.x & 63];
-    atomicAdd(&ps[0], s_iters);
-    atomicAdd(&ps[1], s_cells);
-    if (s_cap) atomicAdd(&ps[2], s_cap);
-    if (s_fb) atomicAdd(&ps[3], s_fb);
-    atomicMax(&ps[4], (unsigned long long)s_max);
-    if (w_full) atomicAdd(&ps[5], w_full);
-    if (w_short) atomicAdd(&ps[6], w_short);
-  }
-}
-
 // The space-time DG predictor over all reconstructed cells (dg.cpp:204-224):
 // initial guess (dg.cpp:12-20, 156-171), Picard (dg.cpp:187-202) or the
 // per-node stiff Newton in place of the reference's Newton-Krylov
 // (dg.cpp:173-185), then the face traces (evaluations.cpp:49-70,
 // fv.cpp:102-122) and the cell-volume term (fv.cpp:33-85) for the corrector.
-// Static schedule: one wavefront per group of CPW consecutive cells, which
-// stays until its slowest cell has converged.
+// One wavefront takes one group of CPW consecutive cells, until its slowest
+// cell has converged.  (A loop over groups with the next group's
+// reconstruction read ahead takes 150 registers instead of 102 at order 2 and
+// 322 instead of 212 at order 4.)  Statistics are counted with ballots, in
+// scalar registers: summing them across lanes at the end was a fifth of the
+// order-2 predictor's instructions.
 // MODE 0: every cell, by block.  MODE 1 (stiff, plain guess): the same cells,
 // but built without the full source-Jacobian solve: a cell where a node would
 // need it is dropped (no outputs, no statistics) and appended to hot[], so
@@ -905,6 +643,13 @@ DEV void predictor_static_body(PredLDS& sm, const double* __restrict__ wh,
   const int lane = threadIdx.x;
   NodeCtx c;
   node_ctx(c, lane, PRED_NODE_TAB(sm));
+  // this lane's planes of a cell: wh at (idx, v), traces at (time node, transverse node)
+  const double* const wh_lane = wh + (long)(c.idx * V) * g.nwc;
+  const int tt = c.idx / ND1, tj = c.idx % ND1;
+  // statistics of this wavefront's cells, the same in every lane
+  unsigned int s_iters = 0u, s_cells = 0u, s_cap = 0u, s_fb = 0u, s_max = 0u, s_full = 0u,
+               s_short = 0u;
+  auto count = [](bool x) { return (unsigned int)__popcll(__ballot(x)); };
   long cell;
   bool valid;
   if constexpr (MODE == 2) {
@@ -918,7 +663,7 @@ DEV void predictor_static_body(PredLDS& sm, const double* __restrict__ wh,
   double w[V], q[N][V], rhs[N][V], dqs[N][D][V];
   if (valid) {
 #pragma unroll
-    for (int v = 0; v < V; v++) w[v] = wh[(long)(c.idx * V + v) * g.nwc + cell];
+    for (int v = 0; v < V; v++) w[v] = wh_lane[(long)v * g.nwc + cell];
 #pragma unroll
     for (int t = 0; t < N; t++)
 #pragma unroll
@@ -937,7 +682,8 @@ DEV void predictor_static_body(PredLDS& sm, const double* __restrict__ wh,
   int learned = (PDE_GUESS && guess) ? 1 : 0;
   int fellback = 0;
   double r0 = 0.0;
-  unsigned int n_full = 0u, n_short = 0u;  // node corrections of this lane
+  unsigned int n_full = 0u, n_short = 0u;  // MODE 1: node corrections of this lane
+  unsigned int trips = 0u;                 // the slowest cell's iterations
   bool cell_hot = false;                   // MODE 1: the cell needs the full solve
   // One iteration for every cell still active; FIRST: the first iteration
   // from the plain guess, whose iterate is constant in time (the wave-uniform
@@ -950,7 +696,7 @@ DEV void predictor_static_body(PredLDS& sm, const double* __restrict__ wh,
 #pragma unroll
       for (int t = 0; t < N; t++)
 #pragma unroll
-        for (int v = 0; v < V; v++) sm.q[c.slot][t][c.idx][v] = q[t][v];
+        for (int v = 0; v < V; v++) sm.q[t][c.slot][c.idx][v] = q[t][v];
     }
     pred_sync();
     if constexpr (FIRST)
@@ -959,6 +705,8 @@ DEV void predictor_static_body(PredLDS& sm, const double* __restrict__ wh,
       node_rhs(c, sm, q, w, dt, g, active, rhs, dqs);
     bool more = false;
     bool skip = false;
+    trips++;
+    if constexpr (MODE != 1) s_iters += count(active && c.idx == 0);
 #if PDE_STIFF
     // residual G = rhs - (DG_MAT (x) W) q   (dg.cpp:128-154)
     double rmax = 0.0;
@@ -1003,13 +751,13 @@ DEV void predictor_static_body(PredLDS& sm, const double* __restrict__ wh,
       }
     }
 #endif
-    bool node_hot = false;
+    bool node_hot = false, node_full = false;
     if (active && !skip) {
-      if (newton_node<MODE != 1>(c, q, rhs, dt)) {
-        n_full++;
-        node_hot = MODE == 1;
-      } else {
-        n_short++;
+      node_full = newton_node<MODE != 1>(c, q, rhs, dt);
+      if constexpr (MODE == 1) {
+        node_hot = node_full;
+        n_full += node_full ? 1u : 0u;
+        n_short += node_full ? 0u : 1u;
       }
       if (!node_hot) {
 #pragma unroll
@@ -1020,6 +768,10 @@ DEV void predictor_static_body(PredLDS& sm, const double* __restrict__ wh,
             q[t][v] = q[t][v] + rhs[t][v];
           }
       }
+    }
+    if constexpr (MODE != 1) {
+      s_full += count(node_full);
+      s_short += count(active && !skip && !node_full);
     }
     if (skip) more = true;
     if constexpr (MODE == 1) {
@@ -1073,23 +825,27 @@ DEV void predictor_static_body(PredLDS& sm, const double* __restrict__ wh,
 #pragma unroll
     for (int t = 0; t < N; t++)
 #pragma unroll
-      for (int v = 0; v < V; v++) sm.q[c.slot][t][c.idx][v] = q[t][v];
+      for (int v = 0; v < V; v++) sm.q[t][c.slot][c.idx][v] = q[t][v];
   }
   pred_sync();
   if (done_here) {
     // traces with every lane busy: the N ND1 = ND lanes of a cell take one
-    // (time node t, transverse node j) each and write both ends e of every
+    // (time node tt, transverse node tj) each and write both ends e of every
     // direction d and variable v
-    const int t = c.idx / ND1, j = c.idx % ND1;
+    static_assert(TCW == CPW, "a trace block is a wavefront's cells");
+    double* const tr_lane =
+        tr + (MODE == 2 ? trace_at(g, tt * ND1 + tj, cell / CPW, (int)(cell % CPW))
+                        : trace_at(g, tt * ND1 + tj, (long)xcd_order(b.x, b.n), c.slot));
+    const long tr_plane = g.ntb * (V * TCW);
     static_for<0, D>([&](auto dc) {
       constexpr int d = decltype(dc)::value;
       constexpr int stride = ipow_c(N, D - 1 - d);
-      const int idx0 = (j / stride) * stride * N + j % stride;  // node with k_d = 0
+      const int idx0 = (tj / stride) * stride * N + tj % stride;  // node with k_d = 0
       double qm[N][V];
 #pragma unroll
       for (int m = 0; m < N; m++)
 #pragma unroll
-        for (int v = 0; v < V; v++) qm[m][v] = sm.q[c.slot][t][idx0 + m * stride][v];
+        for (int v = 0; v < V; v++) qm[m][v] = sm.q[tt][c.slot][idx0 + m * stride][v];
 #pragma unroll
       for (int e = 0; e < 2; e++)
 #pragma unroll
@@ -1097,8 +853,7 @@ DEV void predictor_static_body(PredLDS& sm, const double* __restrict__ wh,
           double acc = (e ? T_END1[0] : T_END0[0]) * qm[0][v];
 #pragma unroll
           for (int m = 1; m < N; m++) acc = dfma(e ? T_END1[m] : T_END0[m], qm[m][v], acc);
-          const int plane = (((d * 2 + e) * N + t) * ND1 + j) * V + v;
-          tr[(long)plane * g.nwc + cell] = acc;
+          tr_lane[(long)((d * 2 + e) * N * ND1) * tr_plane + v * TCW] = acc;
         }
     });
     if (qh) {
@@ -1140,7 +895,7 @@ DEV void predictor_static_body(PredLDS& sm, const double* __restrict__ wh,
   pred_sync();
   if (done_here) {
 #pragma unroll
-    for (int v = 0; v < V; v++) sm.q[c.slot][0][c.idx][v] = part[v];
+    for (int v = 0; v < V; v++) sm.q[0][c.slot][c.idx][v] = part[v];
   }
   pred_sync();
   // the cell's lane idx sums variable v = idx (+ ND, ...) over the nodes in order
@@ -1149,36 +904,36 @@ DEV void predictor_static_body(PredLDS& sm, const double* __restrict__ wh,
     for (int v0 = 0; v0 < V; v0 += ND) {
       const int v = v0 + c.idx;
       if (v < V) {
-        double acc = sm.q[c.slot][0][0][v];
+        double acc = sm.q[0][c.slot][0][v];
 #pragma unroll
-        for (int i = 1; i < ND; i++) acc = acc + sm.q[c.slot][0][i][v];
+        for (int i = 1; i < ND; i++) acc = acc + sm.q[0][c.slot][i][v];
         vol[(long)v * g.nwc + cell] = acc;
       }
     }
   }
 #endif
-  // ---- statistics (one contribution per cell)
-  unsigned long long mine = (done_here && c.idx == 0) ? (unsigned long long)it : 0ull;
-  unsigned long long cnt = (done_here && c.idx == 0) ? 1ull : 0ull;
-  unsigned long long cap = (done_here && c.idx == 0 && it >= maxit) ? 1ull : 0ull;
-  unsigned long long fb = (done_here && c.idx == 0) ? (unsigned long long)fellback : 0ull;
-  unsigned int mx = (done_here && c.idx == 0) ? (unsigned int)it : 0u;
-  if (!done_here) n_full = n_short = 0u;
-  mine = wave_sum_u64(mine);
-  cnt = wave_sum_u64(cnt);
-  cap = wave_sum_u64(cap);
-  fb = wave_sum_u64(fb);
-  mx = wave_max_u32(mx);
-  const unsigned long long w_full = wave_sum_u64(n_full), w_short = wave_sum_u64(n_short);
-  if (lane == 0) {
+  // ---- statistics
+  if constexpr (MODE == 1) {
+    if (!done_here) n_full = n_short = 0u;
+    s_iters += (unsigned int)wave_sum_u64(done_here && c.idx == 0 ? (unsigned long long)it : 0ull);
+    s_max = wave_max_u32(done_here && c.idx == 0 ? (unsigned int)it : 0u);
+    s_full += (unsigned int)wave_sum_u64(n_full);
+    s_short += (unsigned int)wave_sum_u64(n_short);
+  } else {
+    s_max = trips > s_max ? trips : s_max;
+  }
+  s_cells += count(done_here && c.idx == 0);
+  s_cap += count(done_here && c.idx == 0 && it >= maxit);
+  s_fb += count(done_here && c.idx == 0 && fellback);
+  if (lane == 0 && s_cells) {
     unsigned long long* ps = st->pstat[b.x & 63];
-    atomicAdd(&ps[0], mine);
-    atomicAdd(&ps[1], cnt);
-    if (cap) atomicAdd(&ps[2], cap);
-    if (fb) atomicAdd(&ps[3], fb);
-    atomicMax(&ps[4], (unsigned long long)mx);
-    if (w_full) atomicAdd(&ps[5], w_full);
-    if (w_short) atomicAdd(&ps[6], w_short);
+    atomicAdd(&ps[0], (unsigned long long)s_iters);
+    atomicAdd(&ps[1], (unsigned long long)s_cells);
+    if (s_cap) atomicAdd(&ps[2], (unsigned long long)s_cap);
+    if (s_fb) atomicAdd(&ps[3], (unsigned long long)s_fb);
+    atomicMax(&ps[4], (unsigned long long)s_max);
+    if (s_full) atomicAdd(&ps[5], (unsigned long long)s_full);
+    if (s_short) atomicAdd(&ps[6], (unsigned long long)s_short);
   }
 }
 
@@ -1224,18 +979,6 @@ k_predictor_hot(const double* __restrict__ wh, double* __restrict__ tr, double* 
                            nullptr, hw_blk(), hot);
 }
 #endif
-
-// The same with the register budget of two wavefronts per SIMD (spilling the
-// rest), for latency hiding where the single-wavefront kernel stalls.
-extern "C" __global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2, 2)))
-k_predictor_static2(const double* __restrict__ wh, const double* __restrict__ guess,
-                    double* __restrict__ tr, double* __restrict__ vol, double* __restrict__ qh,
-                    StepState* st, Geom g, double newton_tol, int newton_maxit,
-                   double* __restrict__ trd) {
-  __shared__ PredLDS sm;
-  predictor_static_body(sm, wh, guess, tr, vol, qh, st, g, newton_tol, newton_maxit, trd,
-                        hw_blk());
-}
 
 #endif  // PDE_V <= 8
 
@@ -1499,8 +1242,8 @@ DEV void flux_wide(const double* __restrict__ tr, double* __restrict__ ff, doubl
   long wl, wr;
   face_cells<d>(g, f, &wl, &wr);
   const int lane = threadIdx.x & 63, side = threadIdx.x >> 6;
-  const double* const trL = tr + (long)((((d * 2 + 1) * N + t) * ND1 + j) * V) * g.nwc + wl;
-  const double* const trR = tr + (long)((((d * 2 + 0) * N + t) * ND1 + j) * V) * g.nwc + wr;
+  const double* const trL = tr + trace_at(g, ((d * 2 + 1) * N + t) * ND1 + j, wl, 0);
+  const double* const trR = tr + trace_at(g, ((d * 2 + 0) * N + t) * ND1 + j, wr, 0);
   const long o = (long)((t * ND1 + j) * V) * nf + f;
   __shared__ WideMat wm[2];
 #if PDE_USE_F
@@ -1509,7 +1252,7 @@ DEV void flux_wide(const double* __restrict__ tr, double* __restrict__ ff, doubl
     double q[V], dq[D * V], f0[V];
     const double* const src = side ? trR : trL;
 #pragma unroll
-    for (int v = 0; v < V; v++) q[v] = src[(long)v * g.nwc];
+    for (int v = 0; v < V; v++) q[v] = src[v];
 #pragma unroll
     for (int i = 0; i < D * V; i++) dq[i] = 0.0;
     const double l = wide_max_abs_eigs(wm[side], q, dq, d, lane, f0);
@@ -1523,7 +1266,7 @@ DEV void flux_wide(const double* __restrict__ tr, double* __restrict__ ff, doubl
       const int v = threadIdx.x;
       const double s = dmax(lam[0], lam[1]);
       ff[o + (long)v * nf] =
-          s * (trL[(long)v * g.nwc] - trR[(long)v * g.nwc]) + (fs[0][v] + fs[1][v]);
+          s * (trL[v] - trR[v]) + (fs[0][v] + fs[1][v]);
     }
   }
 #endif
@@ -1536,8 +1279,8 @@ DEV void flux_wide(const double* __restrict__ tr, double* __restrict__ ff, doubl
     const int row = lane < V ? lane : 0;
 #pragma unroll
     for (int v = 0; v < V; v++) {
-      qL[v] = trL[(long)v * g.nwc];
-      Dq[v] = trR[(long)v * g.nwc] - qL[v];
+      qL[v] = trL[v];
+      Dq[v] = trR[v] - qL[v];
     }
 #pragma unroll
     for (int i = 0; i < N; i++) {
@@ -1608,9 +1351,12 @@ DEV void face_state(const double* __restrict__ tr, const double* __restrict__ tr
                     const FaceItem& it, int side, double* q, double* dq) {
   const long w = side ? it.wr : it.wl;
   const int e = side ? 0 : 1;
+  const int plane = ((d * 2 + e) * N + it.t) * ND1 + it.j;
+  // (block and place in it by a constant divisor, 32-bit where indices are)
+  const long block = g.idx32 ? (long)((unsigned)w / (unsigned)TCW) : w / TCW;
+  const double* const p = tr + trace_at(g, plane, block, (int)(w - block * TCW));
 #pragma unroll
-  for (int v = 0; v < V; v++)
-    q[v] = tr[(long)((((d * 2 + e) * N + it.t) * ND1 + it.j) * V + v) * g.nwc + w];
+  for (int v = 0; v < V; v++) q[v] = p[v * TCW];
 #pragma unroll
   for (int i = 0; i < D * V; i++) {
 #if PDE_SECOND
@@ -2475,14 +2221,6 @@ k_dt_b(const Member* ms, const BlkMap* map, int nm) {
 extern "C" __global__ void __launch_bounds__(64)
 k_predictor_static_b(const Member* ms, const BlkMap* map, int nm, double newton_tol,
                      int newton_maxit) {
-  __shared__ PredLDS sm;
-  PYPDE_BATCH_MEMBER
-  predictor_static_body(sm, M.wh, nullptr, M.tr, M.vol, nullptr, M.st, M.g, newton_tol,
-                        newton_maxit, M.trd, b);
-}
-extern "C" __global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2, 2)))
-k_predictor_static2_b(const Member* ms, const BlkMap* map, int nm, double newton_tol,
-                      int newton_maxit) {
   __shared__ PredLDS sm;
   PYPDE_BATCH_MEMBER
   predictor_static_body(sm, M.wh, nullptr, M.tr, M.vol, nullptr, M.st, M.g, newton_tol,

@@ -534,7 +534,7 @@ DEV void wide_predictor(WidePred& sm, const double* __restrict__ wh,
 #pragma unroll
         for (int m = 1; m < N; m++)
           acc = dfma(e ? T_END1[m] : T_END0[m], sm.q[t][idx0 + m * stride][v], acc);
-        tr[(long)((((d * 2 + e) * N + t) * ND1 + j) * V + v) * g.nwc + cell] = acc;
+        tr[trace_at(g, ((d * 2 + e) * N + t) * ND1 + j, cell, 0) + v] = acc;
       }
     }
   });

@@ -73,6 +73,7 @@ struct Geom {
   int ndt;
   unsigned fmul[2], fsh[2], rmul[2], rsh[2];
   int idx32;
+  long ntb;
 };
 
 // Multiplier and shift of the device's udiv for a divisor 1 <= d < 2^31:
@@ -92,7 +93,6 @@ struct StepState {
   unsigned int nan_flag, pad2;
   unsigned long long pred_iters, pred_cells, pred_capped, pred_fallbacks;
   unsigned int pred_maxit, pad3;
-  unsigned long long qhead;
   unsigned long long pred_nfull, pred_nshort;
   unsigned long long pred_iters32;
   unsigned long long hot_count;
@@ -307,19 +307,19 @@ int check_spec(const Spec& s, bool secondOrder, int FLUX) {
   return 0;
 }
 
-enum { K_WENO, K_DT, K_PRED, K_FLUX, K_UPDATE, K_A2S, K_S2A,
-       K_HARVEST, K_MLPGUESS, K_PRED_STATIC, K_PRED_STATIC2, K_EIG, K_P2R, K_PRED32,
+enum { K_WENO, K_DT, K_FLUX, K_UPDATE, K_A2S, K_S2A,
+       K_HARVEST, K_MLPGUESS, K_PRED_STATIC, K_EIG, K_P2R, K_PRED32,
        K_WENO_4x64, K_WENO_16x16, K_WENO_16x32, K_FLUX_64, K_FLUX_SPLIT,
        K_UPD1, K_UPD2, K_UPD4, K_UPD8, K_PRED_COLD, K_PRED_HOT, K_MLPPACK, K_PRED_COLD3,
        // batched ensemble kernels (modules built with PDE_BATCH only)
        K_B_WENO, K_B_WENO_4x64, K_B_WENO_16x16, K_B_WENO_16x32, K_B_DT, K_B_PRED_STATIC,
-       K_B_PRED_STATIC2, K_B_PRED_COLD, K_B_PRED_COLD3, K_B_PRED_HOT, K_B_FLUX, K_B_FLUX_64,
+       K_B_PRED_COLD, K_B_PRED_COLD3, K_B_PRED_HOT, K_B_FLUX, K_B_FLUX_64,
        K_B_FLUX_SPLIT, K_B_UPDATE, K_B_UPD1, K_B_UPD2,
        K_B_UPD4, K_B_UPD8, K_COUNT };
-const char* kernel_names[K_COUNT] = {"k_weno",   "k_dt",    "k_predictor",
+const char* kernel_names[K_COUNT] = {"k_weno",   "k_dt",
                                      "k_flux", "k_update",
                                      "k_aos_to_soa", "k_soa_to_aos", "k_harvest", "k_mlp_guess",
-                                     "k_predictor_static", "k_predictor_static2", "k_eig_batch",
+                                     "k_predictor_static", "k_eig_batch",
                                      "k_planes_to_rows", "k_predictor_f32",
                                      "k_weno_4x64", "k_weno_16x16", "k_weno_16x32",
                                      "k_flux_64", "k_flux_split",
@@ -327,7 +327,7 @@ const char* kernel_names[K_COUNT] = {"k_weno",   "k_dt",    "k_predictor",
                                      "k_predictor_cold", "k_predictor_hot", "k_mlp_pack",
                                      "k_predictor_cold3",
                                      "k_weno_b", "k_weno_4x64_b", "k_weno_16x16_b", "k_weno_16x32_b",
-                                     "k_dt_b", "k_predictor_static_b", "k_predictor_static2_b",
+                                     "k_dt_b", "k_predictor_static_b",
                                      "k_predictor_cold_b", "k_predictor_cold3_b", "k_predictor_hot_b",
                                      "k_flux_b", "k_flux_64_b", "k_flux_split_b",
                                      "k_update_b", "k_update_r1_b", "k_update_r2_b", "k_update_r4_b",
@@ -385,10 +385,6 @@ struct pypde_ctx {
   float* mlp_aux = nullptr;  // ... and its FP32 normalisation and bias vectors
   double* qh = nullptr;     // full predictor output (harvest)
   int n_cu = 0;             // compute units of the device
-  hipFunction_t pred_fn = nullptr;
-  long pred_blocks = 0;     // persistent predictor workgroups for pred_fn
-  bool pred_static = true;  // one wavefront per cell group instead of the work queue
-  bool pred_w2 = false;     // the two-wavefronts-per-SIMD register budget
   bool pred_fixed = false;  // schedule fixed by PYPDE_PRED_SCHEDULE (not tuned)
   bool pred_split = false;  // cold pass over every cell, hot pass over the cells it hands on
   bool pred_cold3 = false;  // ... with the cold pass built for three wavefronts per SIMD
@@ -492,8 +488,7 @@ int load_module(const Spec& spec, int device, hipModule_t* mod, hipFunction_t* f
     return fail(PYPDE_ERR_HIP, "hipModuleLoadData failed");
   for (int k = 0; k < K_COUNT; k++) {
     e.fn[k] = nullptr;
-    bool optional = ((k == K_FLUX_64 || k == K_FLUX_SPLIT || k == K_PRED ||
-                      k == K_PRED_STATIC2) && spec.V > WIDE_V) ||
+    bool optional = ((k == K_FLUX_64 || k == K_FLUX_SPLIT) && spec.V > WIDE_V) ||
                     k == K_MLPGUESS || k == K_MLPPACK || (k == K_PRED32 && !spec.mixed) ||
                     k == K_PRED_COLD || k == K_PRED_HOT || k == K_PRED_COLD3 || k >= K_B_WENO;
     if (hipModuleGetFunction(&e.fn[k], e.mod, kernel_names[k]) != hipSuccess) {
@@ -547,27 +542,6 @@ long flux_blocks(const Spec& s, int variant, const Geom& g) {
 bool stats_has_nodes(const pypde_stats* s) {
   return s->struct_size <= 0 ||
          (size_t)s->struct_size >= offsetof(pypde_stats, pred_iters_f32) + sizeof(long);
-}
-
-// Workgroups of the persistent predictor: as many as can be resident at once
-// (occupancy x compute units; PYPDE_PRED_BLOCKS overrides), never more than
-// there are groups of CPW cells.
-long predictor_blocks(pypde_ctx* c) {
-  if (c->pred_fn != c->fn[K_PRED]) {
-    c->pred_fn = c->fn[K_PRED];
-    int per_cu = 0;
-    if (hipModuleOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, c->pred_fn, 64, 0) != hipSuccess ||
-        per_cu < 1)
-      per_cu = 4;
-    if (c->n_cu < 1) c->n_cu = 256;
-    c->pred_blocks = (long)per_cu * c->n_cu;
-    if (const char* e = getenv("PYPDE_PRED_BLOCKS")) {
-      long v = atol(e);
-      if (v > 0) c->pred_blocks = v;
-    }
-  }
-  long groups = cdiv(c->g.nwc, c->CPW);
-  return c->pred_blocks < groups ? c->pred_blocks : groups;
 }
 
 // One timestep: boundaries + WENO, CFL reduction, predictor, face fluxes,
@@ -651,11 +625,8 @@ int enqueue_step(pypde_ctx* c, bool guess_now, std::vector<hipEvent_t>* evs) {
       const int kc = (c->pred_cold3 && c->fn[K_PRED_COLD3]) ? K_PRED_COLD3 : K_PRED_COLD;
       if ((rc = launch(c, kc, dim3(blocks), dim3(64), b))) return rc;
       if ((rc = launch(c, K_PRED_HOT, dim3(blocks), dim3(64), b))) return rc;
-    } else if (c->pred_static) {
-      if ((rc = launch(c, c->pred_w2 ? K_PRED_STATIC2 : K_PRED_STATIC,
-                       dim3((unsigned)cdiv(g.nwc, c->CPW)), dim3(64), a)))
-        return rc;
-    } else if ((rc = launch(c, K_PRED, dim3((unsigned)predictor_blocks(c)), dim3(64), a))) {
+    } else if ((rc = launch(c, K_PRED_STATIC,
+                            dim3((unsigned)cdiv(g.nwc, c->CPW)), dim3(64), a))) {
       return rc;
     }
   }
@@ -873,20 +844,12 @@ static pypde_ctx* create_ctx(const char* src, bool useF, bool useB, bool useS, c
   // DT_LANES in ader_kernels.h
   c->dt_lanes = V > WIDE_V ? 64 : secondOrder ? 2 * ndim : (ndim == 2 && V <= 5) ? 2 : 1;
   c->device = opts.device;
-  // Predictor schedule: the autotuner picks among the static one (one
-  // wavefront per group of CPW cells), the persistent work-queued kernel and
-  // the stiff cold/hot split; PYPDE_PRED_SCHEDULE fixes one instead.
-  c->pred_static = true;
+  // Predictor schedule: the autotuner weighs the stiff cold/hot split against
+  // one kernel; PYPDE_PRED_SCHEDULE ("split", or any other name for the one
+  // kernel) fixes it.  Above WIDE_V there is one predictor kernel.
   if (const char* e = getenv("PYPDE_PRED_SCHEDULE")) {
-    c->pred_static = strcmp(e, "queue") != 0;
-    c->pred_w2 = strcmp(e, "static2") == 0;
-    c->pred_split = strcmp(e, "split") == 0;
+    c->pred_split = strcmp(e, "split") == 0 && V <= WIDE_V;
     c->pred_fixed = true;
-  }
-  // above WIDE_V there is one predictor kernel
-  if (V > WIDE_V) {
-    c->pred_static = c->pred_fixed = true;
-    c->pred_w2 = c->pred_split = false;
   }
   Geom& g = c->g;
   memset(&g, 0, sizeof g);
@@ -908,6 +871,7 @@ static pypde_ctx* create_ctx(const char* src, bool useF, bool useB, bool useS, c
     for (int e = 0; e < ndim; e++) g.nf[d] *= (e == d) ? nX[e] + 1 : nX[e];
   }
   g.idx32 = g.nwc < (1L << 31);
+  g.ntb = cdiv(g.nwc, c->CPW);  // trace blocks hold CPW cells (TCW in ader_kernels.h)
   for (int d = 0; d < 2; d++) {
     long nf = d < ndim ? g.nf[d] : 1;
     udiv_magic(nf, &g.fmul[d], &g.fsh[d]);
@@ -940,7 +904,7 @@ static pypde_ctx* create_ctx(const char* src, bool useF, bool useB, bool useS, c
     return hipMalloc((void**)p, std::max<size_t>(n, 1) * sizeof(double)) == hipSuccess;
   };
   bool ok = alloc(&c->u, g.ncell * V) && alloc(&c->wh, g.nwc * c->ND * V) &&
-            alloc(&c->tr, g.nwc * NTR) && alloc(&c->tmp, g.ncell * V) &&
+            alloc(&c->tr, g.ntb * c->CPW * NTR) && alloc(&c->tmp, g.ncell * V) &&
             (!secondOrder || alloc(&c->trd, g.nwc * NTR * ndim)) &&
             ((!useS && !useB) || alloc(&c->vol, g.nwc * V));
   for (int d = 0; d < ndim && ok; d++) {
@@ -1030,7 +994,6 @@ void apply_tuning(pypde_ctx* c, const std::vector<int>& v) {
   c->tune.flux = (v[1] >= 0 && v[1] < flux_variants(c->V)) ? v[1] : 0;
   c->tune.update = (v[2] >= 0 && v[2] < N_UPD_V) ? v[2] : 0;
   if (!c->pred_fixed) {
-    c->pred_static = v[3] != 1;
     c->pred_split = (v[3] == 2 || v[3] == 3) && c->fn[K_PRED_COLD] != nullptr;
     c->pred_cold3 = v[3] == 3;
   }
@@ -1101,10 +1064,11 @@ int autotune(pypde_ctx* c) {
     return fail(PYPDE_ERR_HIP, "autotune: trial state upload failed");
   }
   double* keep_ret = c->ret;
-  const bool keep_static = c->pred_static, keep_split = c->pred_split, keep_c3 = c->pred_cold3;
+  const bool keep_split = c->pred_split, keep_c3 = c->pred_cold3;
   c->ret = nullptr;
   const int nw = c->D == 2 ? N_WENO_V : 1;
-  const int np = c->pred_fixed ? 1 : (c->fn[K_PRED_COLD] && c->hot ? N_PRED_V : 2);
+  // predictor trials: one kernel, the split, the split with the other cold pass
+  const int np = !c->pred_fixed && c->fn[K_PRED_COLD] && c->hot ? 3 : 1;
   const int nfl = flux_variants(c->V);
   const int ntrial = std::max(std::max(nw, nfl), std::max(N_UPD_V, np));
   const int reps = 2;
@@ -1116,9 +1080,8 @@ int autotune(pypde_ctx* c) {
     c->tune.flux = tk % nfl;
     c->tune.update = tk % N_UPD_V;
     if (!c->pred_fixed) {
-      c->pred_static = (tk % np) != 1;
-      c->pred_split = (tk % np) >= 2;
-      c->pred_cold3 = (tk % np) == 3;
+      c->pred_split = (tk % np) >= 1;
+      c->pred_cold3 = (tk % np) == 2;
     }
     rc = enqueue_step(c, false, &evs[k]);
     if (!rc && hipMemcpyAsync(c->u, c->tmp, ub, hipMemcpyDeviceToDevice, c->stream) != hipSuccess)
@@ -1156,7 +1119,6 @@ int autotune(pypde_ctx* c) {
     for (auto x : e) (void)hipEventDestroy(x);
   (void)hipFree(st_bak);
   c->ret = keep_ret;
-  c->pred_static = keep_static;
   c->pred_split = keep_split;
   c->pred_cold3 = keep_c3;
   if (rc) return rc;
@@ -1167,11 +1129,12 @@ int autotune(pypde_ctx* c) {
     return b;
   };
   std::vector<int> v = {best(tw, nw), best(tf, nfl), best(tu, N_UPD_V),
-                        c->pred_fixed ? (c->pred_static ? 0 : 1) : best(tp, np)};
+                        c->pred_fixed ? 0 : best(tp, np)};
+  if (v[3]) v[3]++;  // schedules 2 and 3 are the split's two builds
   apply_tuning(c, v);
   c->tune.source = 1;
   c->tune.ms[0] = tw[v[0]];
-  c->tune.ms[1] = tp[c->pred_fixed ? 0 : v[3]];
+  c->tune.ms[1] = tp[v[3] ? v[3] - 1 : 0];
   c->tune.ms[2] = tf[v[1]];
   c->tune.ms[3] = tu[v[2]];
   std::lock_guard<std::mutex> lk(g_mu);
@@ -1375,7 +1338,7 @@ struct EnsGroup {
   // launch variants: those the autotuner chose for the group's largest member
   // (the work queue replaced by the static schedule)
   int weno = 0, flux = 0, update = 0;
-  int pred = 0;  // 0 static, 1 static (two-wavefront budget), 2 split, 3 split (cold pass x3)
+  int pred = 0;  // 0 one kernel, 2 split, 3 split (cold pass x3)
 };
 
 struct pypde_ensemble {
@@ -1432,8 +1395,6 @@ static int batch_setup(pypde_ensemble* e, long cap) {
       gr.update = big->tune.update;
       if (big->pred_split && big->hot && big->fn[K_B_PRED_COLD] && big->fn[K_B_PRED_HOT])
         gr.pred = (big->pred_cold3 && big->fn[K_B_PRED_COLD3]) ? 3 : 2;
-      else if (big->pred_static && big->pred_w2)
-        gr.pred = 1;
       e->groups.push_back(gr);
       cells = 0;
     }
@@ -1540,7 +1501,7 @@ static int enqueue_group_step(pypde_ensemble* e, const EnsGroup& gr) {
   if (gr.pred >= 2) {
     if ((rc = go(gr.pred == 3 ? K_B_PRED_COLD3 : K_B_PRED_COLD, BS_PRED, 64, true))) return rc;
     if ((rc = go(K_B_PRED_HOT, BS_PRED, 64, true))) return rc;
-  } else if ((rc = go(gr.pred == 1 ? K_B_PRED_STATIC2 : K_B_PRED_STATIC, BS_PRED, 64, true))) {
+  } else if ((rc = go(K_B_PRED_STATIC, BS_PRED, 64, true))) {
     return rc;
   }
   if ((rc = go(B_FLUX_KID[gr.flux], BS_FLUX, flux_threads(c->spec, gr.flux), false))) return rc;
@@ -1858,7 +1819,7 @@ int pypde_get_tuning(pypde_ctx* c, int* choices, double* ms) {
     choices[0] = c->tune.weno;
     choices[1] = c->tune.flux;
     choices[2] = c->tune.update;
-    choices[3] = c->pred_split ? (c->pred_cold3 ? 3 : 2) : (c->pred_static ? 0 : 1);
+    choices[3] = c->pred_split ? (c->pred_cold3 ? 3 : 2) : 0;
     choices[4] = c->tune.source;
   }
   if (ms)
