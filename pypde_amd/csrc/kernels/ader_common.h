@@ -39,6 +39,47 @@ DEV double dfma(double a, double b, double c) { return __builtin_fma(a, b, c); }
 DEV double dabs(double a) { return __builtin_fabs(a); }
 DEV double dmax(double a, double b) { return __builtin_fmax(a, b); }
 DEV double dsqrt(double a) { return __builtin_sqrt(a); }
+// 1 / b and sqrt(a), correctly rounded as by the operators, for b and a well
+// inside the normal range (2^-1000 .. 2^1000), which the caller has checked:
+// Newton-Raphson and Goldschmidt steps on the hardware's estimate and a last
+// correction by the residual, exact in an fma (Markstein), without the
+// operand scaling and the special cases that make up half of the general
+// forms' instructions.  With the leaner root iteration below and matrices
+// kept in single registers (max_abs_eig's copy), a Rusanov face point of 2D
+// Euler went from 1692 to 1355 vector instructions and from 144 to 122
+// registers (2048 x 2048 at order 2: 1789 -> 1603 us; the 1024 x 256 channel
+// 306 -> 283), an Osher point from 238 to 160 registers (128 x 128: 131 -> 103).
+DEV double recip_mid(double b) {
+  double y = __builtin_amdgcn_rcp(b);
+  y = dfma(y, dfma(-b, y, 1.0), y);
+  y = dfma(y, dfma(-b, y, 1.0), y);
+  return dfma(dfma(-b, y, 1.0), y, y);
+}
+DEV double div_mid(double a, double b) {  // a / b, a and a / b as far inside the range
+  double y = __builtin_amdgcn_rcp(b);
+  y = dfma(y, dfma(-b, y, 1.0), y);
+  y = dfma(y, dfma(-b, y, 1.0), y);
+  const double q = a * y;
+  return dfma(dfma(-b, q, a), y, q);
+}
+DEV double sqrt_mid(double a) {
+  const double y = __builtin_amdgcn_rsq(a);
+  double g = a * y, h = 0.5 * y;
+  const double r = dfma(-h, g, 0.5);
+  g = dfma(g, r, g);
+  h = dfma(h, r, h);
+  g = dfma(dfma(-g, g, a), h, g);
+  return dfma(dfma(-g, g, a), h, g);
+}
+// this lane's bit of a wavefront mask (older compilers lack the builtin, which
+// uses the mask as it is)
+DEV bool lane_bit(unsigned long long mask) {
+#if __has_builtin(__builtin_amdgcn_inverse_ballot_w64)
+  return __builtin_amdgcn_inverse_ballot_w64(mask);
+#else
+  return ((mask >> __lane_id()) & 1ull) != 0;
+#endif
+}
 
 // node multi-index digit k_d of node idx (row-major, k_0 slowest)
 template <int d> DEV constexpr int kdig(int idx) { return (idx / ipow_c(N, D - 1 - d)) % N; }
@@ -140,23 +181,32 @@ DEV int ghost_src(int i, int type, int n, bool* flip) {
 // P x = mu e_1, P = I - beta v v^T, v = (v0, x[1..M-1]), beta = 2 / (v^T v).
 // A tail below 2^-900 in square norm counts as reduced (entries are <= 1).
 constexpr double HOUSE_TINY = 0x1p-900;
+// false (v and beta not set) when the column counts as reduced
 template <int M>
-DEV double house(const double* x, double* v) {
+DEV bool house(const double* x, double* v, double* beta) {
   double sigma = 0.0;
 #pragma unroll
   for (int i = 1; i < M; i++) sigma = dfma(x[i], x[i], sigma);
-  if (sigma <= HOUSE_TINY) {
-    v[0] = 1.0;
+  bool go = !(sigma <= HOUSE_TINY);
+  if (go) {
+    const double mu2 = dfma(x[0], x[0], sigma);
+    double v0;
+    if (mu2 <= 0x1p60) {
+      // sigma > 2^-900: the divisors lie in 2^-900 .. 2^62, sigma / (x0 + mu) above 2^-932
+      const double mu = sqrt_mid(mu2);
+      v0 = (x[0] <= 0.0) ? x[0] - mu : -div_mid(sigma, x[0] + mu);
+      *beta = 2.0 * recip_mid(dfma(v0, v0, sigma));
+    } else {  // infinities, NaN
+      const double mu = dsqrt(mu2);
+      v0 = (x[0] <= 0.0) ? x[0] - mu : -sigma / (x[0] + mu);
+      *beta = 2.0 / dfma(v0, v0, sigma);
+      go = *beta != 0.0;
+    }
+    v[0] = v0;
 #pragma unroll
-    for (int i = 1; i < M; i++) v[i] = 0.0;
-    return 0.0;
+    for (int i = 1; i < M; i++) v[i] = x[i];
   }
-  double mu = dsqrt(dfma(x[0], x[0], sigma));
-  double v0 = (x[0] <= 0.0) ? x[0] - mu : -sigma / (x[0] + mu);
-  v[0] = v0;
-#pragma unroll
-  for (int i = 1; i < M; i++) v[i] = x[i];
-  return 2.0 / dfma(v0, v0, sigma);
+  return go;
 }
 
 // The same reflector with one division: v^T v = 2 mu (mu - x0), so beta =
@@ -167,26 +217,35 @@ DEV double house(const double* x, double* v) {
 // a tail below 2^-500 in square norm counts as reduced, which keeps the
 // product above 2^-1000.
 constexpr double HOUSE1_TINY = 0x1p-500;
+// false (v, beta and mu not set) when the column counts as reduced
 template <int M>
-DEV double house1(const double* x, double* v, double* mu_out) {
+DEV bool house1(const double* x, double* v, double* beta, double* mu_out) {
   double sigma = 0.0;
 #pragma unroll
   for (int i = 1; i < M; i++) sigma = dfma(x[i], x[i], sigma);
-  if (sigma <= HOUSE1_TINY) {
-    v[0] = 1.0;
+  bool go = !(sigma <= HOUSE1_TINY);
+  if (go) {
+    const double mu2 = dfma(x[0], x[0], sigma);
+    const bool pos = x[0] > 0.0;
+    double mu, s, r;
+    if (mu2 <= 0x1p400) {
+      // sigma > 2^-500: the divisor lies in 2^-1000 .. 2^602, beta > 0
+      mu = sqrt_mid(mu2);
+      s = x[0] + mu;
+      r = recip_mid(pos ? (s * mu) * sigma : mu * (mu - x[0]));
+    } else {  // infinities, NaN
+      mu = dsqrt(mu2);
+      s = x[0] + mu;
+      r = 1.0 / (pos ? (s * mu) * sigma : mu * (mu - x[0]));
+      go = (pos ? s * (r * s) : r) != 0.0;
+    }
+    *mu_out = mu;
+    v[0] = pos ? -sigma * ((r * mu) * sigma) : x[0] - mu;
 #pragma unroll
-    for (int i = 1; i < M; i++) v[i] = 0.0;
-    return 0.0;
+    for (int i = 1; i < M; i++) v[i] = x[i];
+    *beta = pos ? s * (r * s) : r;
   }
-  const double mu = dsqrt(dfma(x[0], x[0], sigma));
-  *mu_out = mu;
-  const bool pos = x[0] > 0.0;
-  const double s = x[0] + mu;
-  const double r = 1.0 / (pos ? (s * mu) * sigma : mu * (mu - x[0]));
-  v[0] = pos ? -sigma * ((r * mu) * sigma) : x[0] - mu;
-#pragma unroll
-  for (int i = 1; i < M; i++) v[i] = x[i];
-  return pos ? s * (r * s) : r;
+  return go;
 }
 
 // H = P H on rows r0..r0+M-1 for the columns j with lo_c <= j <= hi_c.
@@ -273,81 +332,105 @@ DEV void hess_charpoly(const double* H, double* c) {
 // step lands near the roots at once, which is why the larger systems keep
 // Laguerre.  The Laguerre step n / (G +- sqrt((n-1)(n H - G^2))) is evaluated
 // multiplied through by p: n p / (p' +- sqrt((n-1)((n-1) p'^2 - n p p''))).
-// The K iterations are independent and advance in one loop; each
-// stops at its own convergence exactly as it would alone.  The fused Horner
-// recurrence for p, p' and p''/2 starts after its first two steps, which are
-// exact for the monic c (c[V] = 1, finite x).  Converged: |step| <= 4 eps
-// |x|, or |step| <= 1e-8 |x| with |step| |x| <= |previous step|^2
-// (superlinear convergence seen, so the remaining error is below
-// |step|^2.5).  ok[k] is false when root k does not converge in 40 steps;
-// dp[k] is p' where p was last evaluated (at the root, or one step of at most
-// 1e-8 |root| before it).
+// The fused Horner recurrence for p, p' and p''/2 starts after its first two
+// steps, which are exact for the monic c (c[V] = 1, finite x).  Converged:
+// |step| <= 4 eps |x|, or |step| <= 1e-8 |x| with |step| |x| <= |previous
+// step|^2 (superlinear convergence seen, so the remaining error is below
+// |step|^2.5), or an exact zero of p.  ok[k] is false when root k does not
+// converge in 40 steps; dp[k] is p' where p was last evaluated (at the root,
+// or one step of at most 1e-8 |root| before it).
+//
+// The K iterations are independent and advance in one loop (their latencies
+// overlap).  The loop is issue bound, so it carries no per-root state machine:
+// every lane keeps stepping until all of the wavefront's are done, and a
+// root's result is taken aside in the iteration that ends it.  One comparison
+// per step, |step| > max(1e-8 |x|, the smallest normal), rules all the ways to
+// end out (a zero of p steps by 0; a zero divisor steps to infinity or NaN,
+// which fails the comparison), so the full tests run only in the last one or
+// two steps: 28 instructions per root and step instead of 46.
 constexpr bool ROOT_HALLEY = V <= 5;
 template <int K>
 DEV void real_roots(const double (&c)[K][V + 1], const double (&x0)[K], double (&root)[K],
                     double (&dp)[K], bool (&ok)[K]) {
   double x[K], prev[K];
-  int state[K];  // 0 running, 1 converged, 2 failed
+  unsigned long long left[K], found[K];  // the wavefront's lanes still iterating, converged
 #pragma unroll
   for (int k = 0; k < K; k++) {
     x[k] = x0[k];
     prev[k] = 0.0;
-    state[k] = 0;
+    left[k] = __builtin_amdgcn_ballot_w64(true);
+    found[k] = 0;
     dp[k] = 0.0;
+    root[k] = 0.0;
   }
   for (int it = 0; it < 40; it++) {
-    bool any = false;
+    unsigned long long any = 0;
 #pragma unroll
-    for (int k = 0; k < K; k++) any = any || state[k] == 0;
-    if (!any) break;
+    for (int k = 0; k < K; k++) any |= left[k];
+    if (any == 0) break;
+    double b[K], d[K], den[K], xn[K], as[K];
+    unsigned long long near[K], stops = 0;
 #pragma unroll
     for (int k = 0; k < K; k++) {
       const double xk = x[k];
       const double b1 = xk + c[k][V - 1];
-      double f = 1.0, d = xk + b1, b = dfma(xk, b1, c[k][V - 2]);
+      double f = 1.0;
+      d[k] = xk + b1;
+      b[k] = dfma(xk, b1, c[k][V - 2]);
 #pragma unroll
       for (int j = V - 3; j >= 0; j--) {
-        f = dfma(xk, f, d);
-        d = dfma(xk, d, b);
-        b = dfma(xk, b, c[k][j]);
+        f = dfma(xk, f, d[k]);
+        d[k] = dfma(xk, d[k], b[k]);
+        b[k] = dfma(xk, b[k], c[k][j]);
       }
-      double num, den;
+      double num;
       if constexpr (ROOT_HALLEY) {
-        num = b * d;
-        den = dfma(d, d, -(b * f));
+        num = b[k] * d[k];
+        den[k] = dfma(d[k], d[k], -(b[k] * f));
       } else {
-        const double r =
-            (double)(V - 1) * ((double)(V - 1) * (d * d) - (double)(2 * V) * (f * b));
+        const double r = (double)(V - 1) *
+                         ((double)(V - 1) * (d[k] * d[k]) - (double)(2 * V) * (f * b[k]));
         const double sq = r > 0.0 ? dsqrt(r) : 0.0;
-        num = (double)V * b;
-        den = (d >= 0.0) ? d + sq : d - sq;
+        num = (double)V * b[k];
+        den[k] = (d[k] >= 0.0) ? d[k] + sq : d[k] - sq;
       }
-      const double step = num / den;
-      const double xn = xk - step;
-      const double as = dabs(step), ax = dabs(xn);
-      const bool conv = !(as > 4.0 * 2.220446049250313e-16 * ax) ||
-                        as <= 2.2250738585072014e-308 ||
-                        (as <= 1e-8 * ax && as * ax <= prev[k] * prev[k]);
-      // state update as selects (no branches): a running root records p'; an
-      // exact zero of p stops at xk, a zero denominator fails, otherwise the
-      // step is taken and convergence (finite root) or failure decided
-      const bool run = state[k] == 0;
-      const bool exact = b == 0.0;
-      const bool step_ok = run && !exact && (den != 0.0);
-      const int ns = exact ? 1 : !(den != 0.0) ? 2 : conv ? (ax <= 1e300 ? 1 : 2) : 0;
-      dp[k] = run ? d : dp[k];
-      x[k] = step_ok ? xn : xk;
-      prev[k] = step_ok ? as : prev[k];
-      state[k] = run ? ns : state[k];
+      const double step = num / den[k];
+      xn[k] = xk - step;
+      as[k] = dabs(step);
+      near[k] = left[k] & __builtin_amdgcn_ballot_w64(
+                              !(as[k] > dmax(1e-8 * dabs(xn[k]), 2.2250738585072014e-308)));
+      stops |= near[k];
+    }
+    if (stops != 0) {
+#pragma unroll
+      for (int k = 0; k < K; k++) {
+        const double ax = dabs(xn[k]);
+        const bool exact = b[k] == 0.0, fail = !(den[k] != 0.0);
+        const bool conv = !(as[k] > 4.0 * 2.220446049250313e-16 * ax) |
+                          (as[k] <= 2.2250738585072014e-308) |
+                          ((as[k] <= 1e-8 * ax) & (as[k] * ax <= prev[k] * prev[k]));
+        const unsigned long long end =
+            near[k] & (__builtin_amdgcn_ballot_w64(exact) | __builtin_amdgcn_ballot_w64(fail) |
+                       __builtin_amdgcn_ballot_w64(conv));
+        left[k] &= ~end;
+        // a zero divisor or an infinite root fails
+        found[k] |= end & (__builtin_amdgcn_ballot_w64(exact) |
+                           (__builtin_amdgcn_ballot_w64(ax <= 1e300) &
+                            ~__builtin_amdgcn_ballot_w64(fail)));
+        if (lane_bit(end)) {
+          root[k] = exact ? x[k] : xn[k];
+          dp[k] = d[k];
+        }
+      }
+    }
+#pragma unroll
+    for (int k = 0; k < K; k++) {
+      x[k] = xn[k];
+      prev[k] = as[k];
     }
   }
-  // a root converges where its iterate stops: at xk for an exact zero, at
-  // the last step's xn otherwise (a failed root is not used)
 #pragma unroll
-  for (int k = 0; k < K; k++) {
-    ok[k] = state[k] == 1;
-    root[k] = x[k];
-  }
+  for (int k = 0; k < K; k++) ok[k] = lane_bit(found[k]);
 }
 
 // Characteristic polynomial c of the scaled upper Hessenberg H and the
@@ -362,22 +445,28 @@ DEV void charpoly_setup(const double* H, double* c, double* xhi, double* xlo) {
   constexpr double inv_v = 1.0 / (double)V;
   const double mu = -(c[V - 1] * inv_v);
   const double s2 = dfma(-mu, mu, dfma(c[V - 1], c[V - 1], -2.0 * c[V - 2]) * inv_v);
-  if (s2 > 0.0 && s2 <= 1e300) {
+  double hi, lo;
+  if ((s2 > 0x1p-900) & (s2 <= 0x1p900)) {
+    const double w = 1.001 * sqrt_mid(s2 * (0.5 * (double)V));
+    hi = mu + w;
+    lo = mu - w;
+  } else if (s2 > 0.0 && s2 <= 1e300) {
     const double w = 1.001 * dsqrt(s2 * (0.5 * (double)V));
-    *xhi = mu + w;
-    *xlo = mu - w;
-    return;
-  }
-  double u = 0.0;
+    hi = mu + w;
+    lo = mu - w;
+  } else {
+    hi = 0.0;
 #pragma unroll
-  for (int i = 0; i < V; i++) {
-    double rs = 0.0;
+    for (int i = 0; i < V; i++) {
+      double rs = 0.0;
 #pragma unroll
-    for (int j = 0; j < V; j++) rs = rs + dabs(H[i * V + j]);
-    u = dmax(u, rs);
+      for (int j = 0; j < V; j++) rs = rs + dabs(H[i * V + j]);
+      hi = dmax(hi, rs);
+    }
+    lo = -hi;
   }
-  *xhi = u;
-  *xlo = -u;
+  *xhi = hi;
+  *xlo = lo;
 }
 
 // Given the largest and smallest real roots l1 > l2 of c, with p' = d1, d2
@@ -437,7 +526,8 @@ DEV bool charpoly_certify(const double* c, double l1, double l2, double d1, doub
       int e;
       (void)__builtin_frexp(t[k], &e);  // |t_k| = f 2^e, f in [0.5, 1)
       const int jj = m - k;
-      const int ce = e >= 0 ? (e + jj - 1) / jj : -((-e) / jj);
+      // ceil(e / jj), |e| < 1100
+      const int ce = (int)((unsigned)(e + 2048 * jj + jj - 1) / (unsigned)jj) - 2048;
       emax = ce > emax ? ce : emax;
     }
   }
@@ -448,18 +538,10 @@ DEV bool charpoly_certify(const double* c, double l1, double l2, double d1, doub
 }
 #endif
 
-// Scale A (destroyed) by the power of two 2^-e2 at or above its largest
-// |entry| above V = 5 or when that lies outside 2^+-64 (*scaled), and reduce
-// it to upper Hessenberg form in place.  False when A is zero, subnormal or
-// NaN; *early is then max |lambda|.
-DEV bool eig_prepare(double* H, int* e2out, bool* scaled, double* early) {
-  double scale = 0.0;
-#pragma unroll
-  for (int i = 0; i < V * V; i++) scale = dmax(scale, dabs(H[i]));
-  if (!(scale >= 2.2250738585072014e-308)) {
-    *early = (scale != scale) ? scale : 0.0;
-    return false;
-  }
+// Scale A (destroyed), its largest |entry| `scale` normal, by the power of two
+// 2^-e2 at or above `scale` above V = 5 or when that lies outside 2^+-64
+// (*scaled), and reduce it to upper Hessenberg form in place.
+DEV void eig_prepare(double* H, double scale, int* e2out, bool* scaled) {
   int e2;
   (void)__builtin_frexp(scale, &e2);  // scale = m 2^e2, m in [0.5, 1)
   *e2out = e2;
@@ -481,9 +563,8 @@ DEV bool eig_prepare(double* H, int* e2out, bool* scaled, double* early) {
     double x[m], vv[m];
 #pragma unroll
     for (int i = 0; i < m; i++) x[i] = H[(k + 1 + i) * V + k];
-    double mu = 0.0;
-    double beta = house1<m>(x, vv, &mu);
-    if (beta != 0.0) {
+    double mu, beta;
+    if (house1<m>(x, vv, &beta, &mu)) {
       // column k is x: P x = mu e_1, set rather than computed
       house_left<m, k + 1>(H, vv, beta, k + 1, V - 1);
       H[(k + 1) * V + k] = mu;
@@ -492,7 +573,6 @@ DEV bool eig_prepare(double* H, int* e2out, bool* scaled, double* early) {
       house_right<m, k + 1>(H, vv, beta, 0, V - 1);
     }
   });
-  return true;
 }
 
 // Francis double-shift QR on the scaled Hessenberg H (destroyed): max
@@ -597,8 +677,8 @@ DEV double eig_qr(double* H) {
               x[2] = H[(k + 2) * V + k - 1];
             }
           }
-          double beta = house<3>(x, v);
-          if (beta != 0.0) {
+          double beta;
+          if (house<3>(x, v, &beta)) {
             if constexpr (k >= 1) {
               if (k > lo) {
                 H[k * V + k - 1] = dsqrt(x[0] * x[0] + (x[1] * x[1] + x[2] * x[2]));
@@ -617,8 +697,8 @@ DEV double eig_qr(double* H) {
         if (hh == hi) {
           x[0] = H[(hh - 1) * V + hh - 2];
           x[1] = H[hh * V + hh - 2];
-          double beta = house<2>(x, v);
-          if (beta != 0.0) {
+          double beta;
+          if (house<2>(x, v, &beta)) {
             H[(hh - 1) * V + hh - 2] = dsqrt(x[0] * x[0] + x[1] * x[1]);
             H[hh * V + hh - 2] = 0.0;
             house_left<2, hh - 1>(H, v, beta, hh - 1, hh);
@@ -641,10 +721,14 @@ DEV double eig_qr(double* H) {
 // the remaining diagonal stands in for unresolved eigenvalues.  All array
 // indices are compile-time constants; run-time bounds only predicate.
 DEV double max_abs_eig(double* H) {
+  double scale = 0.0;
+#pragma unroll
+  for (int i = 0; i < V * V; i++) scale = dmax(scale, dabs(H[i]));
+  // zero or subnormal (0) or NaN
+  if (!(scale >= 2.2250738585072014e-308)) return (scale != scale) ? scale : 0.0;
   int e2 = 0;
   bool scaled = true;
-  double early;
-  if (!eig_prepare(H, &e2, &scaled, &early)) return early;
+  eig_prepare(H, scale, &e2, &scaled);
 #if PDE_V >= 3
   {
     double c[2][V + 1], x0[2], root[2], dp[2], r;
@@ -657,12 +741,13 @@ DEV double max_abs_eig(double* H) {
       return scaled ? __builtin_ldexp(r, e2) : r;
   }
 #endif
-  if (!scaled) {
-    const double pw = __builtin_ldexp(1.0, -e2);
+  // (a copy: with the QR steps on H itself the compiler keeps H as one long
+  // register tuple and copies all of it at every join above)
+  const double pw = scaled ? 1.0 : __builtin_ldexp(1.0, -e2);
+  double G[V * V];
 #pragma unroll
-    for (int i = 0; i < V * V; i++) H[i] = H[i] * pw;
-  }
-  return __builtin_ldexp(eig_qr(H), e2);
+  for (int i = 0; i < V * V; i++) G[i] = H[i] * pw;
+  return __builtin_ldexp(eig_qr(G), e2);
 }
 
 // ------------------------------------------------------ system functions
@@ -676,11 +761,11 @@ DEV void callF(double* out, const double* q, const double* dq, int d) {
 }
 
 // 1 / h_i for the forward-difference steps h_i = max(FD_EPS |q_i|, FD_EPS) =
-// 2^-26 m_i, m_i = max(|q_i|, 1) (exact: FD_EPS = 2^-26) with one division
+// 2^-26 m_i, m_i = max(|q_i|, 1) (exact: FD_EPS = 2^-26) with one reciprocal
 // for all of them: 1 / h_i = (2^26 / prod m) (prod_{j<i} m_j prod_{j>i} m_j).
 // When prod m passes 2^1000 each is divided on its own.
-DEV void fd_recips(const double* q, double* rh) {
-  double m[V], pre[V + 1], suf[V + 1];
+DEV void fd_recips(const double* q, double* m, double* rh) {
+  double pre[V + 1], suf[V + 1];
   pre[0] = 1.0;
 #pragma unroll
   for (int i = 0; i < V; i++) {
@@ -695,7 +780,7 @@ DEV void fd_recips(const double* q, double* rh) {
   suf[V] = 1.0;
 #pragma unroll
   for (int i = V - 1; i >= 0; i--) suf[i] = suf[i + 1] * m[i];
-  const double r = 0x1p26 / pre[V];
+  const double r = 0x1p26 * recip_mid(pre[V]);
 #pragma unroll
   for (int i = 0; i < V; i++) rh[i] = r * (pre[i] * suf[i + 1]);
 }
@@ -708,14 +793,13 @@ DEV void system_matrix(const double* q_in, const double* dq, int d, double* A, d
 #pragma unroll
   for (int i = 0; i < V; i++) q[i] = q_in[i];
 #if PDE_USE_F
-  double v1[V], v2[V], rh[V];
+  double v1[V], v2[V], m[V], rh[V];
   F(v1, q, dq, d);
-  fd_recips(q, rh);
+  fd_recips(q, m, rh);
 #pragma unroll
   for (int i = 0; i < V; i++) {
     double qi0 = q[i];
-    double h = dmax(FD_EPS * dabs(qi0), FD_EPS);
-    q[i] = qi0 + h;
+    q[i] = dfma(FD_EPS, m[i], qi0);  // q_i + h_i, h_i exact
     F(v2, q, dq, d);
     q[i] = qi0;
 #pragma unroll
@@ -812,8 +896,8 @@ DEV void real_schur(double* H, double* Z) {
     double x[m], vv[m];
 #pragma unroll
     for (int i = 0; i < m; i++) x[i] = H[(k + 1 + i) * V + k];
-    double beta = house<m>(x, vv);
-    if (beta != 0.0) {
+    double beta;
+    if (house<m>(x, vv, &beta)) {
       house_left<m, k + 1>(H, vv, beta, k, V - 1);
       house_right<m, k + 1>(H, vv, beta, 0, V - 1);
       house_right<m, k + 1>(Z, vv, beta, 0, V - 1);
@@ -946,8 +1030,8 @@ DEV void real_schur(double* H, double* Z) {
               x[2] = H[(k + 2) * V + k - 1];
             }
           }
-          double beta = house<3>(x, v);
-          if (beta != 0.0) {
+          double beta;
+          if (house<3>(x, v, &beta)) {
             if constexpr (k >= 1) {
               if (k > lo) {
                 H[k * V + k - 1] = dsqrt(x[0] * x[0] + (x[1] * x[1] + x[2] * x[2]));
@@ -967,8 +1051,8 @@ DEV void real_schur(double* H, double* Z) {
         if (hh == hi) {
           x[0] = H[(hh - 1) * V + hh - 2];
           x[1] = H[hh * V + hh - 2];
-          double beta = house<2>(x, v);
-          if (beta != 0.0) {
+          double beta;
+          if (house<2>(x, v, &beta)) {
             H[(hh - 1) * V + hh - 2] = dsqrt(x[0] * x[0] + x[1] * x[1]);
             H[hh * V + hh - 2] = 0.0;
             house_left<2, hh - 1>(H, v, beta, hh - 1, V - 1);

@@ -1476,9 +1476,9 @@ DEV void flux_point(const double* __restrict__ tr, double* __restrict__ ff,
 // chain 1 / FLUX_SPLIT as long and as many more wavefronts: what small grids
 // (few wavefronts, or a nearly empty last round of them) are bound by; the
 // same arithmetic on large ones, where the autotuner weighs it against one
-// thread per point.  Viscous flow on 64 x 64 cells: 20.8 us against 28.6 (both
-// directions); Osher on 128 x 128 155 against 131, Rusanov on 317 x 203 72
-// against 64: full rounds of wavefronts gain nothing from shorter ones.
+// thread per point.  Viscous flow on 64 x 64 cells: 18.5 us against 25.5 (both
+// directions); Osher on 128 x 128 103 against 110, Rusanov on 317 x 203 60.9
+// against 57.6: full rounds of wavefronts gain nothing from shorter ones.
 constexpr int FLUX_PARTS = PDE_FLUX == 0 ? 2 : PDE_FLUX == 1 ? 1 : N;  // first-order part
 constexpr int FLUX_SPLIT = FLUX_PARTS + (PDE_SECOND ? 2 : 0);
 struct FluxShared {
@@ -1590,8 +1590,8 @@ constexpr int FLUX_SPLIT = 1;
 // Every direction's faces in one launch: the workgroups of direction 0, then
 // those of direction 1 (flux_blocks on the host); one nearly empty last round
 // of wavefronts instead of one per direction (Osher on 128 x 128: 168 -> 131
-// us; the 1024 x 256 channel 334 -> 314; 2048 x 2048 at order 2 1845 -> 1789).  MODE 0: one thread per face
-// point, BS threads per workgroup; 1: split over FLUX_SPLIT wavefronts per 64
+// us; the 1024 x 256 channel 334 -> 314; 2048 x 2048 at order 2 1845 -> 1789).
+// MODE 0: one thread per face point, BS threads per workgroup; 1: split over FLUX_SPLIT wavefronts per 64
 // points.  Above V = 8 a workgroup takes one face point.
 template <int MODE, int BS>
 DEV void flux_all(const double* __restrict__ tr, const FaceOut& out, const Geom& g,

@@ -54,9 +54,8 @@ DEV void wide_hessenberg(WideMat& W, int lane) {
     for (int i = 0; i < m; i++) x[i] = W.H[k + 1 + i][k];
 #pragma unroll
     for (int i = 0; i < m; i++) h[i] = W.H[k + 1 + i][own];
-    double mu = 0.0;
-    const double beta = house1<m>(x, v, &mu);
-    if (beta != 0.0) {
+    double mu, beta;
+    if (house1<m>(x, v, &beta, &mu)) {
       auto reflect = [&]() {
         double s = v[0] * h[0];
 #pragma unroll
@@ -367,14 +366,13 @@ DEV double wide_max_abs_eig(WideMat& W, const double (&col)[V], int lane) {
 DEV void wide_system_column(WideMat& W, const double* q, const double* dq, int d, int lane,
                             double (&col)[V], double* f0) {
 #if PDE_USE_F
-  double v1[V], v2[V], rh[V], qq[V];
+  double v1[V], v2[V], m[V], rh[V], qq[V];
   F(v1, q, dq, d);
-  fd_recips(q, rh);
+  fd_recips(q, m, rh);
   double r1 = 0.0;
 #pragma unroll
   for (int i = 0; i < V; i++) {
-    const double h = dmax(FD_EPS * dabs(q[i]), FD_EPS);
-    qq[i] = i == lane ? q[i] + h : q[i];
+    qq[i] = i == lane ? dfma(FD_EPS, m[i], q[i]) : q[i];
     r1 = i == lane ? rh[i] : r1;
   }
   F(v2, qq, dq, d);
