@@ -73,7 +73,8 @@ struct StepState {
   // workgroup folds them into the totals above and clears them ([0]
   // iterations, [1] cells, [2] capped, [3] fallbacks, [4] max iterations, [5]
   // full and [6] shortcut node corrections, [7] FP32-phase iterations; [8]
-  // k_dt's partial maximum, folded by k_dt's last workgroup)
+  // k_dt's partial maximum, folded by k_dt's last workgroup; [9], [10] the
+  // tickets of k_dt's and the corrector's workgroups, last_workgroup)
   unsigned long long pstat[64][16];
 };
 
@@ -115,16 +116,33 @@ DEV double wave_max(double x) {
 // ticket, so the last ticket is drawn after every other workgroup's atomics
 // have completed.  No device-scope fence is used: on gfx950 every such fence
 // writes back or invalidates the XCD's L2, which costs more than a separate
-// one-workgroup launch.  n is the number of workgroups drawing from the
-// ticket; every thread of each of them must call it.
-DEV bool last_workgroup(unsigned int* ticket, unsigned int n) {
+// one-workgroup launch.  b.n is the number of workgroups drawing from the
+// ticket, numbered by b.x; every thread of each of them must call it.
+//
+// Atomics on one address complete one after the other, about 12 ns apart, which
+// bounds a launch of many short workgroups (k_dt on 2048 x 2048 cells, 32,800
+// workgroups: 388 us, 232 with two levels).  Above 128 workgroups each
+// therefore draws from one of 64 tickets, word `sub` of its pstat line, and
+// the last of each of the 64 from the common one; below, the second round
+// trip at the end would cost as much as it saves.
+DEV bool last_workgroup(StepState* st, unsigned int* ticket, int sub, const Blk& b) {
   __shared__ unsigned int is_last;
   __builtin_amdgcn_s_waitcnt(0);
   __syncthreads();
   if (threadIdx.x == 0) {
-    const unsigned int prev = atomicAdd(ticket, 1u);
-    is_last = (prev == n - 1) ? 1u : 0u;
-    if (is_last) atomicExch(ticket, 0u);
+    unsigned int n = b.n, last = 1u;
+    if (n > 128u) {
+      const unsigned int k = b.x & 63u, members = (n - k + 63u) >> 6;
+      unsigned long long* own = &st->pstat[k][sub];
+      last = atomicAdd(own, 1ull) == members - 1u ? 1u : 0u;
+      if (last) atomicExch(own, 0ull);
+      n = 64u;
+    }
+    if (last) {
+      last = atomicAdd(ticket, 1u) == n - 1u ? 1u : 0u;
+      if (last) atomicExch(ticket, 0u);
+    }
+    is_last = last;
   }
   __syncthreads();
   return is_last != 0u;
@@ -152,10 +170,15 @@ DEV unsigned int wave_max_u32(unsigned int x) {
 // 2D: one variable per workgroup (coordinate z), a TX x TY tile of output cells
 // per workgroup (256 threads); sweep 1 along axis 0 over the TX + 2N - 2 rows
 // and TY + 2N - 2 columns the tile needs, then sweep 2 along axis 1 for every
-// coefficient index k0.  The autotuner picks the tile per problem.
+// coefficient index k0.  The autotuner picks the tile per problem.  A thread
+// of sweep 2 forms all the nodes of its cell and variable, so it also has
+// their mean (k_dt's fma chain over the nodes): k_dt reads one value per
+// variable instead of N^2 (512 x 512 at order 4 34 -> 21 us, the 1024 x 256
+// channel at order 3 30 -> 24, for 0-1 us more here; at order 2 17 us less there
+// for 17 more here).
 template <int TX, int TY>
 DEV void weno_2d(const double* __restrict__ u, double* __restrict__ wh, const Geom& g, int ghost,
-                 int nin0, int nin1, long out_stride, const Blk& b) {
+                 int nin0, int nin1, long out_stride, double* __restrict__ wm, const Blk& b) {
   constexpr int H = 2 * N - 2;
   const int tid = threadIdx.x;
   constexpr int RX = TX + H, RY = TY + H, RYP = RY + 1;
@@ -193,22 +216,31 @@ DEV void weno_2d(const double* __restrict__ u, double* __restrict__ wh, const Ge
     }
   }
   __syncthreads();
-  for (int e = tid; e < N * TX * TY; e += 256) {
-    int c = e % TY, r = (e / TY) % TX, k0 = e / (TY * TX);
+  for (int e = tid; e < TX * TY; e += 256) {
+    int c = e % TY, r = e / TY;
     int i = i0 + r, j = j0 + c;
     if (i < no0 && j < no1) {
-      double out[N];
-      weno_line([&](int m) { return s1[k0][r][c + m]; }, out);
       long cell = (long)i * no1 + j;
+      double mean = 0.0;
+#pragma unroll(N <= 3 ? N : 1)
+      for (int k0 = 0; k0 < N; k0++) {
+        double out[N];
+        weno_line([&](int m) { return s1[k0][r][c + m]; }, out);
 #pragma unroll
-      for (int k1 = 0; k1 < N; k1++) wh[(long)((k0 * N + k1) * V + v) * out_stride + cell] = out[k1];
+        for (int k1 = 0; k1 < N; k1++) {
+          const int idx = k0 * N + k1;
+          wh[(long)(idx * V + v) * out_stride + cell] = out[k1];
+          mean = idx == 0 ? T_WP[0] * out[0] : dfma(T_WP[idx], out[k1], mean);
+        }
+      }
+      if (wm) wm[(long)v * out_stride + cell] = mean;
     }
   }
 }
 
 // 1D: 256 output cells per workgroup, all variables.
 DEV void weno_1d(const double* __restrict__ u, double* __restrict__ wh, const Geom& g, int ghost,
-                 int nin0, long out_stride, const Blk& b) {
+                 int nin0, long out_stride, double* __restrict__ wm, const Blk& b) {
   constexpr int H = 2 * N - 2;
   const int tid = threadIdx.x;
   constexpr int TX = 256;
@@ -237,8 +269,13 @@ DEV void weno_1d(const double* __restrict__ u, double* __restrict__ wh, const Ge
     if (i < no0) {
       double out[N];
       weno_line([&](int m) { return s0[v][r + m]; }, out);
+      double mean = 0.0;
 #pragma unroll
-      for (int k = 0; k < N; k++) wh[(long)(k * V + v) * out_stride + i] = out[k];
+      for (int k = 0; k < N; k++) {
+        wh[(long)(k * V + v) * out_stride + i] = out[k];
+        mean = k == 0 ? T_WP[0] * out[0] : dfma(T_WP[k], out[k], mean);
+      }
+      if (wm) wm[(long)v * out_stride + i] = mean;
     }
   }
 }
@@ -246,12 +283,12 @@ DEV void weno_1d(const double* __restrict__ u, double* __restrict__ wh, const Ge
 #define PYPDE_WENO_KERNEL(NAME, TX, TY)                                                        \
   extern "C" __global__ void __launch_bounds__(256)                                            \
   NAME(const double* __restrict__ u, double* __restrict__ wh, const StepState* __restrict__ st, \
-       Geom g, int ghost, int nin0, int nin1, long out_stride) {                               \
+       Geom g, int ghost, int nin0, int nin1, long out_stride, double* __restrict__ wm) {      \
     if (st && st->done) return;                                                                \
     if constexpr (D == 1)                                                                      \
-      weno_1d(u, wh, g, ghost, nin0, out_stride, hw_blk());                                    \
+      weno_1d(u, wh, g, ghost, nin0, out_stride, wm, hw_blk());                                \
     else                                                                                       \
-      weno_2d<TX, TY>(u, wh, g, ghost, nin0, nin1, out_stride, hw_blk());                      \
+      weno_2d<TX, TY>(u, wh, g, ghost, nin0, nin1, out_stride, wm, hw_blk());                  \
   }
 PYPDE_WENO_KERNEL(k_weno, 8, 32)
 PYPDE_WENO_KERNEL(k_weno_4x64, 4, 64)
@@ -291,20 +328,15 @@ constexpr int DT_LANES = V > 8 ? 64 : PDE_SECOND ? 2 * D : DT_PAIR ? 2 : 1;
 #if PDE_V > 8
 // One wavefront per w-cell: the cell's mean (lane v takes variable v), then
 // one eigenvalue problem per direction over the wavefront.
-DEV void dt_body(const double* __restrict__ wh, StepState* st, const Geom& g, const Blk& b) {
-  __shared__ WideMat wm[WIDE_WAVES];
+DEV void dt_body(const double* __restrict__ wh, const double* __restrict__ wm, StepState* st,
+                 const Geom& g, const Blk& b) {
+  __shared__ WideMat mats[WIDE_WAVES];
   const int lane = threadIdx.x & 63;
-  WideMat& W = wm[threadIdx.x >> 6];
+  WideMat& W = mats[threadIdx.x >> 6];
   const long c = (long)b.x * WIDE_WAVES + (threadIdx.x >> 6);
   double sum = 0.0;
   if (c < g.nwc) {
-    if (lane < V) {
-      double acc = T_WP[0] * wh[(long)lane * g.nwc + c];
-#pragma unroll
-      for (int idx = 1; idx < ND; idx++)
-        acc = dfma(T_WP[idx], wh[(long)(idx * V + lane) * g.nwc + c], acc);
-      W.P[0][lane] = acc;
-    }
+    if (lane < V) W.P[0][lane] = wm[(long)lane * g.nwc + c];
     wide_sync();
     double q[V], dq[D * V], f0[V];
 #pragma unroll
@@ -320,10 +352,11 @@ DEV void dt_body(const double* __restrict__ wh, StepState* st, const Geom& g, co
   }
   if (lane == 0 && sum > 0.0)
     atomicMax(&st->pstat[b.x & 63][8], (unsigned long long)__double_as_longlong(sum));
-  if (last_workgroup(&st->dt_ticket, b.n)) dt_finalize(st);
+  if (last_workgroup(st, &st->dt_ticket, 9, b)) dt_finalize(st);
 }
 #elif PDE_SECOND
-DEV void dt_body(const double* __restrict__ wh, StepState* st, const Geom& g, const Blk& b) {
+DEV void dt_body(const double* __restrict__ wh, const double* __restrict__ wm, StepState* st,
+                 const Geom& g, const Blk& b) {
   constexpr int CELLS = 256 / DT_LANES;  // a multiple of 64: `part` is the same in a wavefront
   __shared__ double lam[DT_LANES][CELLS];
   const int part = threadIdx.x / CELLS, k = threadIdx.x % CELLS;
@@ -336,12 +369,7 @@ DEV void dt_body(const double* __restrict__ wh, StepState* st, const Geom& g, co
       for (int v = 0; v < V; v++) w[idx][v] = wh[(long)(idx * V + v) * g.nwc + c];
     double q[V], dq[D * V];
 #pragma unroll
-    for (int v = 0; v < V; v++) {
-      double acc = T_WP[0] * w[0][v];
-#pragma unroll
-      for (int idx = 1; idx < ND; idx++) acc = dfma(T_WP[idx], w[idx][v], acc);
-      q[v] = acc;
-    }
+    for (int v = 0; v < V; v++) q[v] = wm[(long)v * g.nwc + c];
     static_for<0, D>([&](auto dc) {
       constexpr int d = decltype(dc)::value;
       double acc[V], tmp[V];
@@ -371,29 +399,20 @@ DEV void dt_body(const double* __restrict__ wh, StepState* st, const Geom& g, co
   const double m = wave_max(sum);
   if ((threadIdx.x & 63) == 0 && m > 0.0)
     atomicMax(&st->pstat[b.x & 63][8], (unsigned long long)__double_as_longlong(m));
-  if (last_workgroup(&st->dt_ticket, b.n)) dt_finalize(st);
+  if (last_workgroup(st, &st->dt_ticket, 9, b)) dt_finalize(st);
 }
 #else
-DEV void dt_body(const double* __restrict__ wh, StepState* st, const Geom& g, const Blk& b) {
+DEV void dt_body(const double* __restrict__ wh, const double* __restrict__ wm, StepState* st,
+                 const Geom& g, const Blk& b) {
   const long item = (long)b.x * 256 + threadIdx.x;
   const long c = DT_PAIR ? (item >> 1) : item;
   double sum = 0.0;
   if constexpr (DT_PAIR) {
     if (c < g.nwc) {
       const int dl = (int)(item & 1);
-      double w[ND][V];
-#pragma unroll
-      for (int idx = 0; idx < ND; idx++)
-#pragma unroll
-        for (int v = 0; v < V; v++) w[idx][v] = wh[(long)(idx * V + v) * g.nwc + c];
       double q[V], dq[D * V];
 #pragma unroll
-      for (int v = 0; v < V; v++) {
-        double acc = T_WP[0] * w[0][v];
-#pragma unroll
-        for (int idx = 1; idx < ND; idx++) acc = dfma(T_WP[idx], w[idx][v], acc);
-        q[v] = acc;
-      }
+      for (int v = 0; v < V; v++) q[v] = wm[(long)v * g.nwc + c];
       // a first-order F takes no gradient (the reference gives it none)
 #pragma unroll
       for (int i = 0; i < D * V; i++) dq[i] = 0.0;
@@ -404,19 +423,9 @@ DEV void dt_body(const double* __restrict__ wh, StepState* st, const Geom& g, co
       if (!(sum > 0.0)) sum = 0.0;
     }
   } else if (c < g.nwc) {
-    double w[ND][V];
-#pragma unroll
-    for (int idx = 0; idx < ND; idx++)
-#pragma unroll
-      for (int v = 0; v < V; v++) w[idx][v] = wh[(long)(idx * V + v) * g.nwc + c];
     double q[V], dq[D * V];
 #pragma unroll
-    for (int v = 0; v < V; v++) {
-      double acc = T_WP[0] * w[0][v];
-#pragma unroll
-      for (int idx = 1; idx < ND; idx++) acc = dfma(T_WP[idx], w[idx][v], acc);
-      q[v] = acc;
-    }
+    for (int v = 0; v < V; v++) q[v] = wm[(long)v * g.nwc + c];
     // a first-order F takes no gradient
 #pragma unroll
     for (int i = 0; i < D * V; i++) dq[i] = 0.0;
@@ -431,14 +440,14 @@ DEV void dt_body(const double* __restrict__ wh, StepState* st, const Geom& g, co
   if ((threadIdx.x & 63) == 0 && m > 0.0)
     atomicMax(&st->pstat[b.x & 63][8], (unsigned long long)__double_as_longlong(m));
   // the last workgroup to finish takes dt from the 64 slots
-  if (last_workgroup(&st->dt_ticket, b.n)) dt_finalize(st);
+  if (last_workgroup(st, &st->dt_ticket, 9, b)) dt_finalize(st);
 }
 #endif
 
 extern "C" __global__ void __launch_bounds__(256)
-k_dt(const double* __restrict__ wh, StepState* st, Geom g) {
+k_dt(const double* __restrict__ wh, const double* __restrict__ wm, StepState* st, Geom g) {
   if (st->done) return;
-  dt_body(wh, st, g, hw_blk());
+  dt_body(wh, wm, st, g, hw_blk());
 }
 
 // dt = CFL / MAX, x0.2 while count <= 5, clamped to tf - t (stepper.cpp:67-75),
@@ -473,14 +482,14 @@ k_eig_batch(const double* __restrict__ A, const double* __restrict__ x, double* 
 #if PDE_V > 8
   // a workgroup's 256 matrices, 64 in turn per wavefront (which is 0: Roe and
   // Osher stop at V = 8)
-  __shared__ WideMat wm[WIDE_WAVES];
+  __shared__ WideMat mats[WIDE_WAVES];
   const int lane = threadIdx.x & 63;
   const long i0 = (long)blockIdx.x * 256 + (threadIdx.x & ~63u);
   for (long k = i0; k < i0 + 64 && k < n; k++) {
     double col[V];
 #pragma unroll
     for (int r = 0; r < V; r++) col[r] = lane < V ? A[k * V * V + r * V + lane] : 0.0;
-    const double lam = wide_max_abs_eig(wm[threadIdx.x >> 6], col, lane);
+    const double lam = wide_max_abs_eig(mats[threadIdx.x >> 6], col, lane);
     if (lane == 0) out[k] = lam;
   }
   (void)x;

@@ -1741,7 +1741,7 @@ k_update(double* __restrict__ u, const double* __restrict__ vol, FaceBufs fbufs,
   if (st->done) return;
   const Blk b = hw_blk();
   update_cell(u, vol, fbufs, ret, st, g, b);
-  if (last_workgroup(&st->step_ticket, b.n)) advance_step(st, g.ndt);
+  if (last_workgroup(st, &st->step_ticket, 10, b)) advance_step(st, g.ndt);
 }
 
 // The corrector with one variable per thread and R consecutive x-rows per
@@ -1867,7 +1867,7 @@ DEV void update_rows(double* __restrict__ u, const double* __restrict__ vol, con
     if (st->done) return;                                                                      \
     const Blk b = hw_blk();                                                                    \
     update_rows<R_>(u, vol, fbufs, ret, st, g, b);                                             \
-    if (last_workgroup(&st->step_ticket, b.n)) advance_step(st, g.ndt);                        \
+    if (last_workgroup(st, &st->step_ticket, 10, b)) advance_step(st, g.ndt);                  \
   }
 PYPDE_UPDATE_ROWS(1)
 PYPDE_UPDATE_ROWS(2)
@@ -2201,9 +2201,9 @@ DEV int batch_member(const PDE_CONST_AS BlkMap* map, int nm, unsigned int blk) {
     PYPDE_BATCH_MEMBER                                                                         \
     if (M.st->done) return;                                                                    \
     if constexpr (D == 1)                                                                      \
-      weno_1d(M.u, M.wh, M.g, 1, 0, M.g.nwc, b);                                               \
+      weno_1d(M.u, M.wh, M.g, 1, 0, M.g.nwc, M.tr, b);                                         \
     else                                                                                       \
-      weno_2d<TX, TY>(M.u, M.wh, M.g, 1, 0, 0, M.g.nwc, b);                                    \
+      weno_2d<TX, TY>(M.u, M.wh, M.g, 1, 0, 0, M.g.nwc, M.tr, b);                              \
   }
 PYPDE_WENO_BATCH(k_weno_b, 8, 32)
 PYPDE_WENO_BATCH(k_weno_4x64_b, 4, 64)
@@ -2214,7 +2214,7 @@ extern "C" __global__ void __launch_bounds__(256)
 k_dt_b(const Member* ms, const BlkMap* map, int nm) {
   PYPDE_BATCH_MEMBER
   if (M.st->done) return;
-  dt_body(M.wh, M.st, M.g, b);
+  dt_body(M.wh, M.tr, M.st, M.g, b);
 }
 
 #if PDE_V <= 8
@@ -2275,7 +2275,7 @@ k_update_b(const Member* ms, const BlkMap* map, int nm) {
   if (M.st->done) return;
   const FaceBufs fbufs = {{M.ff[0], M.ff[1]}, {M.fb[0], M.fb[1]}};
   update_cell(M.u, M.vol, fbufs, nullptr, M.st, M.g, b);
-  if (last_workgroup(&M.st->step_ticket, b.n)) advance_step(M.st, M.g.ndt);
+  if (last_workgroup(M.st, &M.st->step_ticket, 10, b)) advance_step(M.st, M.g.ndt);
 }
 #define PYPDE_UPDATE_ROWS_BATCH(R_)                                                            \
   extern "C" __global__ void __launch_bounds__(256)                                           \
@@ -2284,7 +2284,7 @@ k_update_b(const Member* ms, const BlkMap* map, int nm) {
     if (M.st->done) return;                                                                    \
     const FaceBufs fbufs = {{M.ff[0], M.ff[1]}, {M.fb[0], M.fb[1]}};                           \
     update_rows<R_>(M.u, M.vol, fbufs, nullptr, M.st, M.g, b);                                 \
-    if (last_workgroup(&M.st->step_ticket, b.n)) advance_step(M.st, M.g.ndt);                  \
+    if (last_workgroup(M.st, &M.st->step_ticket, 10, b)) advance_step(M.st, M.g.ndt);          \
   }
 PYPDE_UPDATE_ROWS_BATCH(1)
 PYPDE_UPDATE_ROWS_BATCH(2)

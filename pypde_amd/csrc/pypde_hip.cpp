@@ -102,7 +102,8 @@ struct StepState {
   // workgroup folds them into the totals above and clears them ([0]
   // iterations, [1] cells, [2] capped, [3] fallbacks, [4] max iterations, [5]
   // full and [6] shortcut node corrections, [7] FP32-phase iterations; [8]
-  // k_dt's partial maximum, folded by k_dt's last workgroup)
+  // k_dt's partial maximum, folded by k_dt's last workgroup; [9], [10] the
+  // tickets of k_dt's and the corrector's workgroups)
   unsigned long long pstat[64][16];
 };
 
@@ -567,7 +568,10 @@ int enqueue_step(pypde_ctx* c, bool guess_now, std::vector<hipEvent_t>* evs) {
     const StepState* st = c->st;
     int ghost = 1, z = 0;
     long os = g.nwc;
-    std::vector<void*> a = {&uu, &w, &st, &g, &ghost, &z, &z, &os};
+    // the cells' means, which k_dt reads, lie in the trace buffer, unused until
+    // the predictor (and at least V doubles per w-cell)
+    double* wm = c->tr;
+    std::vector<void*> a = {&uu, &w, &st, &g, &ghost, &z, &z, &os, &wm};
     const int wv = c->D == 1 ? 0 : c->tune.weno;
     const int TX = WENO_TILE[wv][0], TY = WENO_TILE[wv][1];
     dim3 grid = c->D == 1 ? dim3((unsigned)cdiv(g.nw[0], 256))
@@ -578,8 +582,9 @@ int enqueue_step(pypde_ctx* c, bool guess_now, std::vector<hipEvent_t>* evs) {
   mark();
   {
     const double* w = c->wh;
+    const double* wm = c->tr;
     StepState* st = c->st;
-    std::vector<void*> a = {&w, &st, &g};
+    std::vector<void*> a = {&w, &wm, &st, &g};
     // its last workgroup also turns the wave-speed maximum into dt
     if ((rc = launch(c, K_DT, dim3((unsigned)cdiv(g.nwc * c->dt_lanes, 256)), dim3(256), a)))
       return rc;
@@ -2017,7 +2022,8 @@ int weno_solver(double* ret, double* u, int* nX, int ndim, int N, int V) {
   const StepState* st = nullptr;
   int ghost = 0, n0 = nX[0], n1 = ndim > 1 ? nX[1] : 1;
   {
-    void* a[] = {&dus, &dw, &st, &g, &ghost, &n0, &n1, &nout};
+    double* wm = nullptr;
+    void* a[] = {&dus, &dw, &st, &g, &ghost, &n0, &n1, &nout, &wm};
     unsigned gx = ndim == 1 ? (unsigned)cdiv(no[0], 256) : (unsigned)cdiv(no[1], 32);
     unsigned gy = ndim == 1 ? 1 : (unsigned)cdiv(no[0], 8);
     unsigned gz = ndim == 1 ? 1 : (unsigned)V;  // 2D: one variable per workgroup
@@ -2125,7 +2131,8 @@ int weno_solver_noalloc(pypde_ctx* c, double* ret, const double* u, const int* n
     memset(&g, 0, sizeof g);
     const StepState* st = nullptr;
     int ghost = 0, n0 = nX[0], n1 = ndim > 1 ? nX[1] : 1;
-    void* a[] = {&s_in, &s_out, &st, &g, &ghost, &n0, &n1, &nout};
+    double* wm = nullptr;
+    void* a[] = {&s_in, &s_out, &st, &g, &ghost, &n0, &n1, &nout, &wm};
     unsigned gx = ndim == 1 ? (unsigned)cdiv(no[0], 256) : (unsigned)cdiv(no[1], 32);
     unsigned gy = ndim == 1 ? 1 : (unsigned)cdiv(no[0], 8);
     unsigned gz = ndim == 1 ? 1 : (unsigned)V;
