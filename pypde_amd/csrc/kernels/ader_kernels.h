@@ -54,7 +54,8 @@ DEV unsigned udiv(unsigned n, unsigned m, unsigned sh) {
 struct StepState {
   double t, dt, tf, cfl;
   long long count, max_steps;
-  int push, done, nan_step, pad;
+  int push, done, nan_step;
+  int flip;  // 1D: the state lies in u2 (k_update_next)
   unsigned long long maxbits;   // unused (the wave-speed maximum lives in pstat[.][8])
   unsigned int nan_flag, pad2;
   unsigned long long pred_iters, pred_cells, pred_capped, pred_fallbacks;

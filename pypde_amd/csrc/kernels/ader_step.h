@@ -1874,6 +1874,114 @@ PYPDE_UPDATE_ROWS(2)
 PYPDE_UPDATE_ROWS(4)
 PYPDE_UPDATE_ROWS(8)
 
+#if PDE_D == 1 && PDE_V <= 8 && !PDE_SECOND
+// 1D: the corrector, the next step's reconstruction and its timestep in one
+// launch.  A 1D grid's kernels last about as long as a launch and one chain
+// of dependent loads take, so what counts is how many there are: on 200 cells
+// this one takes 10.4 us where the three took 5.8 + 4.2 + 5.4 and two more gaps
+// between launches.  A workgroup takes NEXT_W w-cells: it updates the cells their
+// stencils reach (2N - 2 more than it owns: the neighbours' are formed twice
+// instead of exchanged), reconstructs, and takes the wave speeds of its cells,
+// one lane each.  The state alternates between u and u2 (st->flip: which one
+// holds it), since neighbours read the old values; the run's last step writes
+// u in any case and reconstructs nothing.  Every value is formed by the
+// operations of update_cell, weno_1d and dt_body in their order.
+constexpr int NEXT_W = 64;
+extern "C" __global__ void __launch_bounds__(256)
+k_update_next(double* u, double* u2, const double* __restrict__ vol, FaceBufs fbufs,
+              double* __restrict__ ret, double* __restrict__ wh, StepState* st, Geom g) {
+  constexpr int RX = NEXT_W + 2 * N - 2;
+  __shared__ double s0[V][RX];
+  __shared__ double mean[V][NEXT_W];
+  if (st->done) return;
+  const Blk b = hw_blk();
+  const int tid = threadIdx.x, flip = st->flip, push = st->push;
+  const double dt = st->dt, tn = st->t + dt;
+  const bool last_step =
+      !(tn < st->tf) || (st->max_steps > 0 && st->count + 1 >= st->max_steps);
+  const bool snap = ret && push < g.ndt && tn >= (double)(push + 1) / (double)g.ndt * st->tf;
+  const double* const src = flip ? u2 : u;
+  double* const dst = last_step || flip ? u : u2;
+  const int i0 = (int)b.x * NEXT_W;
+  bool bad = false;
+  for (int e = tid; e < V * RX; e += 256) {
+    const int v = e / RX, r = e % RX, I = i0 + r;
+    const bool own = r >= N - 1 && r < N - 1 + NEXT_W && I >= N && I < N + g.nx[0];
+    if (I >= g.nb[0] || (last_step && !own)) continue;
+    bool f0 = false;
+    const int c = ghost_src(I, g.bc[0], g.nx[0], &f0);
+    double uc = src[(long)v * g.ncell + c];
+#if PDE_USE_S || PDE_USE_B
+    uc = uc + vol[(long)v * g.nwc + c + 1];
+#endif
+#if PDE_USE_F || PDE_USE_B
+#pragma unroll
+    for (int side = 0; side < 2; side++)
+#pragma unroll
+      for (int t = 0; t < N; t++) {
+        const double tmp = (dt * T_W[t]) / (2.0 * g.dX[0]);
+        const long o = (long)(t * V + v) * g.nf[0] + c + side;
+#if PDE_USE_F
+        const double f = fbufs.ff[0][o];
+#else
+        const double f = 0.0;
+#endif
+#if PDE_USE_B
+        const double bb = fbufs.fb[0][o];
+#else
+        const double bb = 0.0;
+#endif
+        uc = side == 0 ? uc - tmp * (bb - f) : uc - tmp * (bb + f);
+      }
+#endif
+    if (own) {
+      dst[(long)v * g.ncell + c] = uc;
+      if (uc != uc) bad = true;
+      if (snap) ret[((long)push * g.ncell + c) * V + v] = uc;
+    }
+    s0[v][r] = uc * (f0 ? g.refl[0][v] : 1.0);
+  }
+  if (bad) atomicOr(&st->nan_flag, 1u);
+  if (!last_step) {
+    __syncthreads();
+    for (int e = tid; e < V * NEXT_W; e += 256) {
+      const int v = e / NEXT_W, r = e % NEXT_W, i = i0 + r;
+      if (i >= g.nw[0]) continue;
+      double out[N], m = 0.0;
+      weno_line([&](int k) { return s0[v][r + k]; }, out);
+#pragma unroll
+      for (int k = 0; k < N; k++) {
+        wh[(long)(k * V + v) * g.nwc + i] = out[k];
+        m = k == 0 ? T_WP[0] * out[0] : dfma(T_WP[k], out[k], m);
+      }
+      mean[v][r] = m;
+    }
+    __syncthreads();
+    if (tid < NEXT_W) {
+      double sum = 0.0;
+      if (i0 + tid < g.nw[0]) {
+        double q[V], dq[V], f0[V];
+#pragma unroll
+        for (int v = 0; v < V; v++) {
+          q[v] = mean[v][tid];
+          dq[v] = 0.0;
+        }
+        sum = sum + max_abs_eigs(q, dq, 0, f0) / g.dX[0];
+        if (!(sum > 0.0)) sum = 0.0;
+      }
+      const double m = wave_max(sum);
+      if (tid == 0 && m > 0.0)
+        atomicMax(&st->pstat[b.x & 63][8], (unsigned long long)__double_as_longlong(m));
+    }
+  }
+  if (last_workgroup(st, &st->step_ticket, 10, b)) {
+    advance_step(st, g.ndt);
+    if (tid == 0) st->flip = dst == u ? 0 : 1;
+    if (!last_step) dt_finalize(st);
+  }
+}
+#endif
+
 // t += dt; count++; snapshot row; NaN and end-of-run checks (iterator.cpp:129-147).
 // Run by the first wavefront of the corrector's last workgroup, which also
 // folds the predictor's spread statistics into the totals (lane i takes slot

@@ -88,7 +88,8 @@ static void udiv_magic(long d, unsigned* mul, unsigned* sh) {
 struct StepState {
   double t, dt, tf, cfl;
   long long count, max_steps;
-  int push, done, nan_step, pad;
+  int push, done, nan_step;
+  int flip;  // 1D: the state lies in u2 (k_update_next)
   unsigned long long maxbits;
   unsigned int nan_flag, pad2;
   unsigned long long pred_iters, pred_cells, pred_capped, pred_fallbacks;
@@ -311,7 +312,7 @@ int check_spec(const Spec& s, bool secondOrder, int FLUX) {
 enum { K_WENO, K_DT, K_FLUX, K_UPDATE, K_A2S, K_S2A,
        K_HARVEST, K_MLPGUESS, K_PRED_STATIC, K_EIG, K_P2R, K_PRED32,
        K_WENO_4x64, K_WENO_16x16, K_WENO_16x32, K_FLUX_64, K_FLUX_SPLIT,
-       K_UPD1, K_UPD2, K_UPD4, K_UPD8, K_PRED_COLD, K_PRED_HOT, K_MLPPACK, K_PRED_COLD3,
+       K_UPD1, K_UPD2, K_UPD4, K_UPD8, K_PRED_COLD, K_PRED_HOT, K_MLPPACK, K_PRED_COLD3, K_NEXT,
        // batched ensemble kernels (modules built with PDE_BATCH only)
        K_B_WENO, K_B_WENO_4x64, K_B_WENO_16x16, K_B_WENO_16x32, K_B_DT, K_B_PRED_STATIC,
        K_B_PRED_COLD, K_B_PRED_COLD3, K_B_PRED_HOT, K_B_FLUX, K_B_FLUX_64,
@@ -326,7 +327,7 @@ const char* kernel_names[K_COUNT] = {"k_weno",   "k_dt",
                                      "k_flux_64", "k_flux_split",
                                      "k_update_r1", "k_update_r2", "k_update_r4", "k_update_r8",
                                      "k_predictor_cold", "k_predictor_hot", "k_mlp_pack",
-                                     "k_predictor_cold3",
+                                     "k_predictor_cold3", "k_update_next",
                                      "k_weno_b", "k_weno_4x64_b", "k_weno_16x16_b", "k_weno_16x32_b",
                                      "k_dt_b", "k_predictor_static_b",
                                      "k_predictor_cold_b", "k_predictor_cold3_b", "k_predictor_hot_b",
@@ -346,6 +347,13 @@ const int WENO_KID[N_WENO_V] = {K_WENO, K_WENO_4x64, K_WENO_16x16, K_WENO_16x32}
 const int FLUX_KID[N_FLUX_V] = {K_FLUX, K_FLUX_64, K_FLUX_SPLIT};
 const int UPD_KID[N_UPD_V] = {K_UPDATE, K_UPD1, K_UPD2, K_UPD4, K_UPD8};
 const int UPD_ROWS[N_UPD_V] = {0, 1, 2, 4, 8};
+constexpr int NEXT_W = 64;  // w-cells per workgroup of k_update_next (the kernels' NEXT_W)
+// Largest 1D grid, in w-cells, that steps with k_update_next.  It saves two
+// launches a step and forms a sixteenth of the cells twice, with one wavefront
+// in four at work on the wave speeds: 1D Euler at order 3, us a step with and
+// without: 2,000 cells 20.3 / 27.5, 8,192 21.8 / 29.1, 65,536 38.4 / 44.2, 131,072
+// 52.0 / 55.1, 262,144 76.8 / 77.4, 400,000 106.8 / 106.8, 1,000,000 243 / 217.
+constexpr long NEXT_MAX = 1l << 17;
 const int B_WENO_KID[N_WENO_V] = {K_B_WENO, K_B_WENO_4x64, K_B_WENO_16x16, K_B_WENO_16x32};
 const int B_FLUX_KID[N_FLUX_V] = {K_B_FLUX, K_B_FLUX_64, K_B_FLUX_SPLIT};
 const int B_UPD_KID[N_UPD_V] = {K_B_UPDATE, K_B_UPD1, K_B_UPD2, K_B_UPD4, K_B_UPD8};
@@ -491,7 +499,8 @@ int load_module(const Spec& spec, int device, hipModule_t* mod, hipFunction_t* f
     e.fn[k] = nullptr;
     bool optional = ((k == K_FLUX_64 || k == K_FLUX_SPLIT) && spec.V > WIDE_V) ||
                     k == K_MLPGUESS || k == K_MLPPACK || (k == K_PRED32 && !spec.mixed) ||
-                    k == K_PRED_COLD || k == K_PRED_HOT || k == K_PRED_COLD3 || k >= K_B_WENO;
+                    k == K_PRED_COLD || k == K_PRED_HOT || k == K_PRED_COLD3 || k == K_NEXT ||
+                    k >= K_B_WENO;
     if (hipModuleGetFunction(&e.fn[k], e.mod, kernel_names[k]) != hipSuccess) {
       e.fn[k] = nullptr;
       (void)hipGetLastError();
@@ -548,7 +557,10 @@ bool stats_has_nodes(const pypde_stats* s) {
 // One timestep: boundaries + WENO, CFL reduction, predictor, face fluxes,
 // corrector, bookkeeping (iterator.cpp:99-148).  Every kernel returns at once
 // when the device flag `done` is set, so whole chunks can be queued blind.
-int enqueue_step(pypde_ctx* c, bool guess_now, std::vector<hipEvent_t>* evs) {
+// next: the corrector's launch also makes the following step's reconstruction
+// and dt (1D, k_update_next); primed: the launch before this step did.
+int enqueue_step(pypde_ctx* c, bool guess_now, std::vector<hipEvent_t>* evs, bool next = false,
+                 bool primed = false) {
   Geom g = c->g;
   int rc;
   hipError_t mark_err = hipSuccess;  // first failure of a profiling event
@@ -562,7 +574,7 @@ int enqueue_step(pypde_ctx* c, bool guess_now, std::vector<hipEvent_t>* evs) {
     }
   };
   mark();
-  {
+  if (!primed) {
     const double* uu = c->u;
     double* w = c->wh;
     const StepState* st = c->st;
@@ -580,7 +592,7 @@ int enqueue_step(pypde_ctx* c, bool guess_now, std::vector<hipEvent_t>* evs) {
     if ((rc = launch(c, WENO_KID[wv], grid, dim3(256), a))) return rc;
   }
   mark();
-  {
+  if (!primed) {
     const double* w = c->wh;
     const double* wm = c->tr;
     StepState* st = c->st;
@@ -649,7 +661,14 @@ int enqueue_step(pypde_ctx* c, bool guess_now, std::vector<hipEvent_t>* evs) {
   }
   mark();
   mark();  // both directions run in the one launch: the second flux slot times nothing
-  {
+  if (next) {
+    double *uu = c->u, *u2 = c->tmp, *w = c->wh, *r = c->ret;
+    const double* v = c->vol;
+    FaceBufs fbufs = {{c->ff[0], c->ff[1]}, {c->fb[0], c->fb[1]}};
+    StepState* st = c->st;
+    std::vector<void*> a = {&uu, &u2, &v, &fbufs, &r, &w, &st, &g};
+    if ((rc = launch(c, K_NEXT, dim3((unsigned)cdiv(g.nwc, NEXT_W)), dim3(256), a))) return rc;
+  } else {
     double* uu = c->u;
     const double* v = c->vol;
     FaceBufs fbufs = {{c->ff[0], c->ff[1]}, {c->fb[0], c->fb[1]}};
@@ -1204,6 +1223,12 @@ static int run_loop(pypde_ctx* c, long max_steps, pypde_stats* stats, bool first
   std::vector<hipEvent_t> evs;
   hipGraphExec_t exec = nullptr;
   const bool graph = c->opts.use_graph && !c->opts.profile;
+  // 1D steps one after the other on the stream: the corrector's launch makes
+  // the next step's reconstruction and dt too (a harvested step keeps the
+  // reconstruction it started from)
+  const bool next =
+      c->fn[K_NEXT] && c->g.nwc <= NEXT_MAX && !graph && !c->opts.profile && !c->qh;
+  bool primed = false;
   int rc = 0;
   while (true) {
     // never queue past a step cap: the launch count equals the step count
@@ -1215,7 +1240,8 @@ static int run_loop(pypde_ctx* c, long max_steps, pypde_stats* stats, bool first
         if (hipGraphLaunch(exec, c->stream) != hipSuccess) rc = fail(PYPDE_ERR_HIP, "graph launch failed");
       } else {
         std::vector<hipEvent_t>* ep = c->opts.profile ? &evs : nullptr;
-        rc = enqueue_step(c, guess_now, ep);
+        rc = enqueue_step(c, guess_now, ep, next, primed);
+        primed = next;
       }
       guess_now = false;
     }
@@ -1232,6 +1258,15 @@ static int run_loop(pypde_ctx* c, long max_steps, pypde_stats* stats, bool first
     if (chunk < 64) chunk *= 2;
   }
   if (exec) (void)hipGraphExecDestroy(exec);
+  if (!rc && c->host_st.flip) {
+    // ended early (a NaN) with the state in the other buffer
+    c->host_st.flip = 0;
+    HIPCHK(hipMemcpyAsync(c->u, c->tmp, c->g.ncell * c->V * sizeof(double),
+                          hipMemcpyDeviceToDevice, c->stream));
+    HIPCHK(hipMemcpyAsync(&c->st->flip, &c->host_st.flip, sizeof(int), hipMemcpyHostToDevice,
+                          c->stream));
+    HIPCHK(hipStreamSynchronize(c->stream));
+  }
   if (rc) {
     for (auto e : evs) (void)hipEventDestroy(e);
     return rc;
