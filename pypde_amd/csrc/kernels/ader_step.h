@@ -1878,7 +1878,7 @@ PYPDE_UPDATE_ROWS(8)
 // 1D: the corrector, the next step's reconstruction and its timestep in one
 // launch.  A 1D grid's kernels last about as long as a launch and one chain
 // of dependent loads take, so what counts is how many there are: on 200 cells
-// this one takes 10.4 us where the three took 5.8 + 4.2 + 5.4 and two more gaps
+// this one takes 9.1 us where the three took 5.8 + 4.2 + 5.4 and two more gaps
 // between launches.  A workgroup takes NEXT_W w-cells: it updates the cells their
 // stencils reach (2N - 2 more than it owns: the neighbours' are formed twice
 // instead of exchanged), reconstructs, and takes the wave speeds of its cells,
@@ -1983,13 +1983,17 @@ k_update_next(double* u, double* u2, const double* __restrict__ vol, FaceBufs fb
 #endif
 
 // t += dt; count++; snapshot row; NaN and end-of-run checks (iterator.cpp:129-147).
-// Run by the first wavefront of the corrector's last workgroup, which also
-// folds the predictor's spread statistics into the totals (lane i takes slot
-// i, then sums and a max across the wavefront) and clears the slots.
+// Run by the corrector's last workgroup (256 threads): the first thread keeps
+// the clock while the second wavefront folds the predictor's spread statistics
+// into the totals (lane i takes slot i, then sums and a max across the
+// wavefront) and clears the slots -- 84 cross-lane moves that the clock, and in
+// 1D the next timestep behind it, would otherwise wait for (200 cells, with the
+// next timestep, 10.4 -> 9.1 us; 317 x 203 14.9 -> 13.4; viscous 64 x 64 7.9 -> 7.1).
 DEV void advance_step(StepState* st, int ndt) {
-  if (threadIdx.x >= 64) return;
-  {
-    unsigned long long* ps = st->pstat[threadIdx.x];
+  if (threadIdx.x >= 128) return;
+  if (threadIdx.x >= 64) {
+    const int slot = threadIdx.x - 64;
+    unsigned long long* ps = st->pstat[slot];
     unsigned long long a0 = wave_sum_u64(ps[0]), a1 = wave_sum_u64(ps[1]);
     unsigned long long a2 = wave_sum_u64(ps[2]), a3 = wave_sum_u64(ps[3]);
     unsigned long long a5 = wave_sum_u64(ps[5]), a6 = wave_sum_u64(ps[6]);
@@ -2002,7 +2006,7 @@ DEV void advance_step(StepState* st, int ndt) {
     }
 #pragma unroll
     for (int k = 0; k < 8; k++) ps[k] = 0ull;
-    if (threadIdx.x == 0) {
+    if (slot == 0) {
       st->pred_iters += a0;
       st->pred_cells += a1;
       st->pred_capped += a2;
