@@ -239,12 +239,16 @@ DEV void weno_2d(const double* __restrict__ u, double* __restrict__ wh, const Ge
   }
 }
 
-// 1D: 256 output cells per workgroup, all variables.
+// 1D: WENO1_W output cells per workgroup, all variables: 256, so that each
+// thread takes V values; above V = 8 16, about one value per thread, as a
+// grid of 200 cells and 17 variables was one workgroup's 17 turns otherwise
+// (13.0 -> 4.7 us).  At V = 3 tiles of 64 and 256 measure the same.
+constexpr int WENO1_W = V > 8 ? 16 : 256;
 DEV void weno_1d(const double* __restrict__ u, double* __restrict__ wh, const Geom& g, int ghost,
                  int nin0, long out_stride, double* __restrict__ wm, const Blk& b) {
   constexpr int H = 2 * N - 2;
   const int tid = threadIdx.x;
-  constexpr int TX = 256;
+  constexpr int TX = WENO1_W;
   constexpr int RX = TX + H;
   __shared__ double s0[V][RX];
   const int i0 = b.x * TX;

@@ -343,6 +343,8 @@ const char* kernel_names[K_COUNT] = {"k_weno",   "k_dt",
 // built for two or for three wavefronts per SIMD).
 constexpr int N_WENO_V = 4, N_FLUX_V = 3, N_UPD_V = 5, N_PRED_V = 4;
 const int WENO_TILE[N_WENO_V][2] = {{8, 32}, {4, 64}, {16, 16}, {16, 32}};
+// Cells per workgroup of the 1D reconstruction (the kernels' WENO1_W).
+constexpr int weno1_width(int v) { return v > 8 ? 16 : 256; }
 const int WENO_KID[N_WENO_V] = {K_WENO, K_WENO_4x64, K_WENO_16x16, K_WENO_16x32};
 const int FLUX_KID[N_FLUX_V] = {K_FLUX, K_FLUX_64, K_FLUX_SPLIT};
 const int UPD_KID[N_UPD_V] = {K_UPDATE, K_UPD1, K_UPD2, K_UPD4, K_UPD8};
@@ -586,7 +588,7 @@ int enqueue_step(pypde_ctx* c, bool guess_now, std::vector<hipEvent_t>* evs, boo
     std::vector<void*> a = {&uu, &w, &st, &g, &ghost, &z, &z, &os, &wm};
     const int wv = c->D == 1 ? 0 : c->tune.weno;
     const int TX = WENO_TILE[wv][0], TY = WENO_TILE[wv][1];
-    dim3 grid = c->D == 1 ? dim3((unsigned)cdiv(g.nw[0], 256))
+    dim3 grid = c->D == 1 ? dim3((unsigned)cdiv(g.nw[0], weno1_width(c->V)))
                           : dim3((unsigned)cdiv(g.nw[1], TY), (unsigned)cdiv(g.nw[0], TX),
                                  (unsigned)c->V);
     if ((rc = launch(c, WENO_KID[wv], grid, dim3(256), a))) return rc;
@@ -1456,7 +1458,7 @@ static int batch_setup(pypde_ensemble* e, long cap) {
         switch (s) {
           case BS_WENO:
             if (D == 1) {
-              gx = cdiv(g.nw[0], 256);
+              gx = cdiv(g.nw[0], weno1_width(V));
             } else {
               gx = cdiv(g.nw[1], WENO_TILE[gr.weno][1]);
               gy = cdiv(g.nw[0], WENO_TILE[gr.weno][0]);
@@ -2059,7 +2061,8 @@ int weno_solver(double* ret, double* u, int* nX, int ndim, int N, int V) {
   {
     double* wm = nullptr;
     void* a[] = {&dus, &dw, &st, &g, &ghost, &n0, &n1, &nout, &wm};
-    unsigned gx = ndim == 1 ? (unsigned)cdiv(no[0], 256) : (unsigned)cdiv(no[1], 32);
+    unsigned gx =
+        ndim == 1 ? (unsigned)cdiv(no[0], weno1_width(V)) : (unsigned)cdiv(no[1], 32);
     unsigned gy = ndim == 1 ? 1 : (unsigned)cdiv(no[0], 8);
     unsigned gz = ndim == 1 ? 1 : (unsigned)V;  // 2D: one variable per workgroup
     HIPCHK(hipModuleLaunchKernel(fn[K_WENO], gx, gy, gz, 256, 1, 1, 0, st0, a, nullptr));
@@ -2168,7 +2171,8 @@ int weno_solver_noalloc(pypde_ctx* c, double* ret, const double* u, const int* n
     int ghost = 0, n0 = nX[0], n1 = ndim > 1 ? nX[1] : 1;
     double* wm = nullptr;
     void* a[] = {&s_in, &s_out, &st, &g, &ghost, &n0, &n1, &nout, &wm};
-    unsigned gx = ndim == 1 ? (unsigned)cdiv(no[0], 256) : (unsigned)cdiv(no[1], 32);
+    unsigned gx =
+        ndim == 1 ? (unsigned)cdiv(no[0], weno1_width(V)) : (unsigned)cdiv(no[1], 32);
     unsigned gy = ndim == 1 ? 1 : (unsigned)cdiv(no[0], 8);
     unsigned gz = ndim == 1 ? 1 : (unsigned)V;
     if ((rc = go(K_WENO, gx, gy, gz, a))) return rc;
