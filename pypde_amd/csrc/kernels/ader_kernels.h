@@ -104,6 +104,15 @@ DEV unsigned int xcd_order(unsigned int i, unsigned int n) {
   return (k / XCD_RUN) * SPAN + x * XCD_RUN + k % XCD_RUN;
 }
 
+// Every kernel of a step returns at once when the run has ended.  The flag was
+// written by another kernel on another XCD, so reading it takes as long as
+// any load from memory; where a kernel's own first loads do not depend on
+// it, they are issued before the flag is tested (their addresses are valid
+// either way), and this keeps the compiler from sinking them below the test
+// (200 cells: predictor 7.3 -> 6.9 us, face flux 4.15 -> 3.9; viscous 64 x 64 0.3
+// less each).
+#define LOADS_FIRST() asm volatile("" ::: "memory")
+
 DEV double wave_max(double x) {
 #pragma unroll
   for (int o = 32; o >= 1; o >>= 1) x = dmax(x, __shfl_xor(x, o, 64));
@@ -319,15 +328,15 @@ DEV void cell_deriv(const double (&w)[ND][V], int idx, double rdx, double* out) 
 }
 
 // In 2D (V <= 5, no viscous term) two neighbouring lanes share a w-cell and
-// take one direction each: twice the wavefronts (a 1024 x 256 grid's 4140
-// fill 1.35 rounds of the 3072 slots at three per SIMD) with half the
-// eigenvalue work per lane.  Both lanes form the cell's (l_0 / dX_0) + (l_1 /
+// take one direction each: twice the wavefronts (a 1024 x 256 grid's 8,272 in
+// two rounds of the 4,096 slots at four per SIMD) with half the eigenvalue
+// work per lane.  Both lanes form the cell's (l_0 / dX_0) + (l_1 /
 // dX_1) from the pair's two terms.  The host launches DT_LANES * nwc threads.
 constexpr bool DT_PAIR = (D == 2) && (V <= 5) && !PDE_SECOND;
 // With a viscous F a w-cell has 2 D eigenvalue problems, each of which costs as
 // much as a whole first-order cell: a wavefront takes one of them for 64
 // cells and the sums go through LDS (64 x 64 cells, 69 wavefronts one after
-// the other's problems otherwise: 22 -> 10.7 us).
+// the other's problems otherwise: 22 -> 10.4 us).
 constexpr int DT_LANES = V > 8 ? 64 : PDE_SECOND ? 2 * D : DT_PAIR ? 2 : 1;
 
 #if PDE_V > 8
@@ -336,6 +345,7 @@ constexpr int DT_LANES = V > 8 ? 64 : PDE_SECOND ? 2 * D : DT_PAIR ? 2 : 1;
 DEV void dt_body(const double* __restrict__ wh, const double* __restrict__ wm, StepState* st,
                  const Geom& g, const Blk& b) {
   __shared__ WideMat mats[WIDE_WAVES];
+  if (st->done) return;
   const int lane = threadIdx.x & 63;
   WideMat& W = mats[threadIdx.x >> 6];
   const long c = (long)b.x * WIDE_WAVES + (threadIdx.x >> 6);
@@ -363,6 +373,7 @@ DEV void dt_body(const double* __restrict__ wh, const double* __restrict__ wm, S
 DEV void dt_body(const double* __restrict__ wh, const double* __restrict__ wm, StepState* st,
                  const Geom& g, const Blk& b) {
   constexpr int CELLS = 256 / DT_LANES;  // a multiple of 64: `part` is the same in a wavefront
+  if (st->done) return;
   __shared__ double lam[DT_LANES][CELLS];
   const int part = threadIdx.x / CELLS, k = threadIdx.x % CELLS;
   const long c = (long)b.x * CELLS + k;
@@ -411,34 +422,32 @@ DEV void dt_body(const double* __restrict__ wh, const double* __restrict__ wm, S
                  const Geom& g, const Blk& b) {
   const long item = (long)b.x * 256 + threadIdx.x;
   const long c = DT_PAIR ? (item >> 1) : item;
+  const int stop = st->done;
+  double q[V], dq[D * V];
+  if (c < g.nwc) {
+#pragma unroll
+    for (int v = 0; v < V; v++) q[v] = wm[(long)v * g.nwc + c];
+  }
+  LOADS_FIRST();
+  if (stop) return;
+  // a first-order F takes no gradient (the reference gives it none)
+#pragma unroll
+  for (int i = 0; i < D * V; i++) dq[i] = 0.0;
   double sum = 0.0;
-  if constexpr (DT_PAIR) {
-    if (c < g.nwc) {
+  if (c < g.nwc) {
+    if constexpr (DT_PAIR) {
       const int dl = (int)(item & 1);
-      double q[V], dq[D * V];
-#pragma unroll
-      for (int v = 0; v < V; v++) q[v] = wm[(long)v * g.nwc + c];
-      // a first-order F takes no gradient (the reference gives it none)
-#pragma unroll
-      for (int i = 0; i < D * V; i++) dq[i] = 0.0;
       double f0[V];
       const double part = max_abs_eigs(q, dq, dl, f0) / (dl ? g.dX[1] : g.dX[0]);
       const double other = __shfl_xor(part, 1, 64);
       sum = dl ? other + part : part + other;
-      if (!(sum > 0.0)) sum = 0.0;
+    } else {
+      static_for<0, D>([&](auto dc) {
+        constexpr int d = decltype(dc)::value;
+        double f0[V];
+        sum = sum + max_abs_eigs(q, dq, d, f0) / g.dX[d];
+      });
     }
-  } else if (c < g.nwc) {
-    double q[V], dq[D * V];
-#pragma unroll
-    for (int v = 0; v < V; v++) q[v] = wm[(long)v * g.nwc + c];
-    // a first-order F takes no gradient
-#pragma unroll
-    for (int i = 0; i < D * V; i++) dq[i] = 0.0;
-    static_for<0, D>([&](auto dc) {
-      constexpr int d = decltype(dc)::value;
-      double f0[V];
-      sum = sum + max_abs_eigs(q, dq, d, f0) / g.dX[d];
-    });
     if (!(sum > 0.0)) sum = 0.0;
   }
   double m = wave_max(sum);
@@ -451,7 +460,6 @@ DEV void dt_body(const double* __restrict__ wh, const double* __restrict__ wm, S
 
 extern "C" __global__ void __launch_bounds__(256)
 k_dt(const double* __restrict__ wh, const double* __restrict__ wm, StepState* st, Geom g) {
-  if (st->done) return;
   dt_body(wh, wm, st, g, hw_blk());
 }
 

@@ -637,8 +637,8 @@ DEV void predictor_static_body(PredLDS& sm, const double* __restrict__ wh,
                                const Geom& g, double newton_tol, int newton_maxit,
                                double* __restrict__ trd, const Blk& b,
                                unsigned int* __restrict__ hot = nullptr) {
-  if (st->done) return;
-  if (MODE == 2 && (unsigned long long)b.x * CPW >= st->hot_count) return;
+  const int stop = st->done;
+  if (MODE == 2 && (stop || (unsigned long long)b.x * CPW >= st->hot_count)) return;
   const double dt = st->dt;
   const int lane = threadIdx.x;
   NodeCtx c;
@@ -670,6 +670,8 @@ DEV void predictor_static_body(PredLDS& sm, const double* __restrict__ wh,
       for (int v = 0; v < V; v++)
         q[t][v] = (PDE_GUESS && guess) ? guess[(long)((t * ND + c.idx) * V + v) * g.nwc + cell] : w[v];
   }
+  LOADS_FIRST();
+  if (stop) return;
   const unsigned long long cellmask =
       (ND == 64 ? ~0ull : ((1ull << ND) - 1ull)) << (c.slot < CPW ? c.slot * ND : 0);
 #if PDE_STIFF
@@ -689,7 +691,8 @@ DEV void predictor_static_body(PredLDS& sm, const double* __restrict__ wh,
   // from the plain guess, whose iterate is constant in time (the wave-uniform
   // q = w), so the right-hand side needs F, S and the derivatives once.  It is
   // peeled off the loop so that the loop holds one right-hand side only
-  // (the stiff cold pass then needs 208 registers instead of 234).
+  // (the stiff cold pass, 157 registers for the reactive channel, needed 26
+  // more with both).
   auto iterate = [&](auto firstc) {
     constexpr bool FIRST = decltype(firstc)::value;
     if (PRED_DQ && active) {
@@ -1399,13 +1402,16 @@ DEV void face_b(const double* qL, const double* qR, double* __restrict__ fb, lon
 template <int d, int BS>
 DEV void flux_point(const double* __restrict__ tr, double* __restrict__ ff,
                     double* __restrict__ fb, const Geom& g, const double* __restrict__ trd,
-                    unsigned int blk) {
+                    const int* done, unsigned int blk) {
   FaceItem it;
+  const int stop = *done;
   if (!face_item<d>(g, blk, BS, threadIdx.x, &it)) return;
   const long nf = g.nf[d];
   double qL[V], qR[V], dqL[D * V], dqR[D * V];
   face_state<d>(tr, trd, g, it, 0, qL, dqL);
   face_state<d>(tr, trd, g, it, 1, qR, dqR);
+  LOADS_FIRST();
+  if (stop) return;
   const long o = (long)((it.t * ND1 + it.j) * V) * nf + it.f;
 #if PDE_USE_F
   {
@@ -1489,30 +1495,38 @@ struct FluxShared {
 template <int d>
 DEV void flux_split(FluxShared& sm, const double* __restrict__ tr, double* __restrict__ ff,
                     double* __restrict__ fb, const Geom& g, const double* __restrict__ trd,
-                    unsigned int blk) {
+                    const int* done, unsigned int blk) {
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   FaceItem it;
+  const int stop = *done;
   const bool ok = face_item<d>(g, blk, 64, lane, &it);
   const long nf = g.nf[d];
   double qL[V], qR[V], dqL[D * V], dqR[D * V], fl[V];
   if (ok) {
+    // this wavefront's side (Roe, Osher: both)
+    face_state<d>(tr, trd, g, it,
+                  PDE_FLUX != 0 && wave < FLUX_PARTS ? 0
+                  : wave >= FLUX_PARTS               ? wave - FLUX_PARTS
+                                                     : wave,
+                  qL, dqL);
+    if (PDE_FLUX != 0 && wave < FLUX_PARTS) face_state<d>(tr, trd, g, it, 1, qR, dqR);
+  }
+  LOADS_FIRST();
+  if (stop) return;
+  if (ok) {
 #if PDE_SECOND
     if (wave >= FLUX_PARTS) {
-      face_state<d>(tr, trd, g, it, wave - FLUX_PARTS, qL, dqL);
       sm.lam[wave][lane] = max_abs_eigs_second_order<d>(qL, dqL, g.dX[d]);
     } else
 #endif
     {
 #if PDE_FLUX == 0
-      face_state<d>(tr, trd, g, it, wave, qL, dqL);
       sm.lam[wave][lane] = max_abs_eigs(qL, dqL, d, fl);
       if (wave == 1) {
 #pragma unroll
         for (int v = 0; v < V; v++) sm.part[1][v][lane] = fl[v];
       }
 #else
-      face_state<d>(tr, trd, g, it, 0, qL, dqL);
-      face_state<d>(tr, trd, g, it, 1, qR, dqR);
       double Dq[V], q[V], A[V * V], ftmp[V], y[V], dqp[D * V];
 #if PDE_FLUX == 1
       double Mx[V * V];
@@ -1590,17 +1604,19 @@ constexpr int FLUX_SPLIT = 1;
 // Every direction's faces in one launch: the workgroups of direction 0, then
 // those of direction 1 (flux_blocks on the host); one nearly empty last round
 // of wavefronts instead of one per direction (Osher on 128 x 128: 168 -> 131
-// us; the 1024 x 256 channel 334 -> 314; 2048 x 2048 at order 2 1845 -> 1789).
-// MODE 0: one thread per face point, BS threads per workgroup; 1: split over FLUX_SPLIT wavefronts per 64
-// points.  Above V = 8 a workgroup takes one face point.
+// us; the 1024 x 256 channel 334 -> 314; 2048 x 2048 at order 2 1845 -> 1789;
+// since then 103, 280 and 1603 with the leaner wave speeds).  MODE 0: one thread
+// per face point, BS threads per workgroup; 1: split over FLUX_SPLIT wavefronts
+// per 64 points.  Above V = 8 a workgroup takes one face point.
 template <int MODE, int BS>
 DEV void flux_all(const double* __restrict__ tr, const FaceOut& out, const Geom& g,
-                  const double* __restrict__ trd, const Blk& b) {
+                  const double* __restrict__ trd, const int* done, const Blk& b) {
   constexpr int POINTS = V > 8 ? 1 : MODE ? 64 : BS;
   const unsigned int nb0 =
       D == 1 ? ~0u : (unsigned int)((g.nf[0] * (N * ND1) + POINTS - 1) / POINTS);
 #if PDE_V > 8
   (void)trd;
+  if (*done) return;
   if (b.x < nb0) flux_wide<0>(tr, out.ff[0], out.fb[0], g, b.x);
 #if PDE_D >= 2
   else flux_wide<1>(tr, out.ff[1], out.fb[1], g, b.x - nb0);
@@ -1609,16 +1625,16 @@ DEV void flux_all(const double* __restrict__ tr, const FaceOut& out, const Geom&
 #if PDE_USE_F
   if constexpr (MODE == 1) {
     __shared__ FluxShared sm;
-    if (b.x < nb0) flux_split<0>(sm, tr, out.ff[0], out.fb[0], g, trd, b.x);
+    if (b.x < nb0) flux_split<0>(sm, tr, out.ff[0], out.fb[0], g, trd, done, b.x);
 #if PDE_D >= 2
-    else flux_split<1>(sm, tr, out.ff[1], out.fb[1], g, trd, b.x - nb0);
+    else flux_split<1>(sm, tr, out.ff[1], out.fb[1], g, trd, done, b.x - nb0);
 #endif
     return;
   }
 #endif
-  if (b.x < nb0) flux_point<0, POINTS>(tr, out.ff[0], out.fb[0], g, trd, b.x);
+  if (b.x < nb0) flux_point<0, POINTS>(tr, out.ff[0], out.fb[0], g, trd, done, b.x);
 #if PDE_D >= 2
-  else flux_point<1, POINTS>(tr, out.ff[1], out.fb[1], g, trd, b.x - nb0);
+  else flux_point<1, POINTS>(tr, out.ff[1], out.fb[1], g, trd, done, b.x - nb0);
 #endif
 #endif
 }
@@ -1631,8 +1647,7 @@ DEV void flux_all(const double* __restrict__ tr, const FaceOut& out, const Geom&
   extern "C" __global__ void __launch_bounds__(BS)                                             \
   NAME(const double* __restrict__ tr, FaceOut out, const StepState* st, Geom g,                \
        const double* __restrict__ trd) {                                                       \
-    if (st->done) return;                                                                      \
-    flux_all<MODE, BS>(tr, out, g, trd, hw_blk());                                             \
+    flux_all<MODE, BS>(tr, out, g, trd, &st->done, hw_blk());                                  \
   }
 PYPDE_FLUX_KERNEL(k_flux, 0, 128)
 #if PDE_V <= 8
@@ -2325,7 +2340,6 @@ PYPDE_WENO_BATCH(k_weno_16x32_b, 16, 32)
 extern "C" __global__ void __launch_bounds__(256)
 k_dt_b(const Member* ms, const BlkMap* map, int nm) {
   PYPDE_BATCH_MEMBER
-  if (M.st->done) return;
   dt_body(M.wh, M.tr, M.st, M.g, b);
 }
 
@@ -2371,9 +2385,8 @@ k_predictor_hot_b(const Member* ms, const BlkMap* map, int nm, double newton_tol
   extern "C" __global__ void __launch_bounds__(BS)                                             \
   NAME(const Member* ms, const BlkMap* map, int nm) {                                          \
     PYPDE_BATCH_MEMBER                                                                         \
-    if (M.st->done) return;                                                                    \
     const FaceOut out = {{M.ff[0], M.ff[1]}, {M.fb[0], M.fb[1]}};                              \
-    flux_all<MODE, BS>(M.tr, out, M.g, M.trd, b);                                              \
+    flux_all<MODE, BS>(M.tr, out, M.g, M.trd, &M.st->done, b);                                 \
   }
 PYPDE_FLUX_BATCH(k_flux_b, 0, 128)
 #if PDE_V <= 8
