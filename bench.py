@@ -273,7 +273,7 @@ def window(st, w):
 
 PREDICTOR_KERNELS = {"split": ["k_predictor_cold", "k_predictor_hot"],
                      "split3": ["k_predictor_cold3", "k_predictor_hot"],
-                     "static": ["k_predictor_static"], "queue": ["k_predictor"]}
+                     "static": ["k_predictor_static"]}
 
 
 def predictor_roofline(st_k, win, K, guess=False):
@@ -311,7 +311,9 @@ def stencil_rooflines(st_k, K, N=ORDER, D=D, V=V, nx=NX, ny=NY):
     tun = st_k["tuning"]
     names = {"k_weno": "k_weno" + {"8x32": ""}.get(tun["weno_tile"], "_" + tun["weno_tile"]),
              "k_update": {"cell": "k_update"}.get(tun["update"],
-                                                 "k_update_r" + tun["update"][-1:])}
+                                                 "k_update_r" + tun["update"][-1:]),
+             "k_flux": {128: "k_flux"}.get(tun["flux_workgroup"],
+                                           "k_flux_%s" % tun["flux_workgroup"])}
     ncell, nwc = nx * ny, (nx + 2) * (ny + 2)
     ND = N ** D
     nf = [(nx + 1) * ny, nx * (ny + 1)]
@@ -322,7 +324,7 @@ def stencil_rooflines(st_k, K, N=ORDER, D=D, V=V, nx=NX, ny=NY):
     b_fv = 8 * (N ** (D + 1) * V * nwc + 2 * V * ncell)   # the FV stage's floor
     out = {}
     for name, b, t in (("k_weno", b_weno, ms["weno"]), ("k_update", b_update, ms["update"]),
-                       ("k_flux0+k_flux1", b_flux, ms["flux0"] + ms["flux1"]),
+                       ("k_flux", b_flux, ms["flux0"] + ms["flux1"]),
                        ("fv_stage", b_fv, ms["flux0"] + ms["flux1"] + ms["update"])):
         bw = b / (t * 1e-3) if t > 0 else 0.0
         kn = names.get(name, name)

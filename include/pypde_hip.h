@@ -175,9 +175,10 @@ int pypde_harvest_step(pypde_ctx *c, float *X, float *Y, long ldx, long col0, py
  * choices[5]: WENO tile (0 8x32, 1 4x64, 2 16x16, 3 16x32), flux workgroup (0
  * 128 and 1 64 threads of one face point each, 2 a point's eigenvalue problems
  * split over several wavefronts), corrector (0 one thread per cell, 1..4 one variable and
- * 1, 2, 4, 8 x-rows per thread), predictor (0 static, 1 work queue, 2 the
- * stiff predictor's cold/hot split, 3 the same with the cold pass built for
- * three wavefronts per SIMD), source (0 defaults, 1 measured, 2 tuning table,
+ * 1, 2, 4, 8 x-rows per thread; small 1D grids step with a corrector of their
+ * own, joined with the next reconstruction and dt), predictor (0 one kernel, 2
+ * the stiff predictor's cold/hot split, 3 the same with the cold pass built
+ * for three wavefronts per SIMD), source (0 defaults, 1 measured, 2 tuning table,
  * 3 PYPDE_TUNE_FORCE); ms[4]: the chosen WENO, predictor, flux (both
  * directions) and corrector trial times. */
 int pypde_get_tuning(pypde_ctx *c, int *choices, double *ms);

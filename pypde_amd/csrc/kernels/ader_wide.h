@@ -9,8 +9,8 @@
 // row j (right products), and scalars are formed by every lane alike.  What
 // bounds it is the latency of the dependent chains (Householder sums, Horner
 // steps, QR sweeps), hidden only by other wavefronts.  On the 17-variable
-// model, 200 cells, order 2: face flux 820 -> 58 us and timestep 445 -> 47 us
-// per launch (a matrix takes about 19,000 cycles to reduce, 5,300 for its
+// model, 200 cells, order 2, a launch: face flux 1340 -> 92 us and timestep 726 ->
+// 75 us (a matrix takes about 19,000 cycles to reduce, 5,300 for its
 // characteristic polynomial, 3,500 for the roots, 3,000 for the certificate
 // and, for the half of them that need it, 88,000 for QR).
 //

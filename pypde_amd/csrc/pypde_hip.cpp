@@ -338,9 +338,9 @@ const char* kernel_names[K_COUNT] = {"k_weno",   "k_dt",
 // Launch variants the autotuner chooses between (every variant of a kernel
 // computes identical results): WENO tiles, flux workgroup sizes, corrector
 // mappings (one thread per cell and all variables, or one variable and R
-// x-rows per thread), predictor schedules (static, work queue, and for the
-// stiff predictor with the plain guess the cold/hot split, its cold pass
-// built for two or for three wavefronts per SIMD).
+// x-rows per thread), predictor schedules (0 one kernel; for the stiff
+// predictor with the plain guess 2, 3 the cold/hot split, its cold pass built
+// for two or for three wavefronts per SIMD; 1 is not used).
 constexpr int N_WENO_V = 4, N_FLUX_V = 3, N_UPD_V = 5, N_PRED_V = 4;
 const int WENO_TILE[N_WENO_V][2] = {{8, 32}, {4, 64}, {16, 16}, {16, 32}};
 // Cells per workgroup of the 1D reconstruction (the kernels' WENO1_W).
@@ -1378,7 +1378,6 @@ struct EnsGroup {
   unsigned int blocks[BS_COUNT] = {};
   hipStream_t stream = nullptr;
   // launch variants: those the autotuner chose for the group's largest member
-  // (the work queue replaced by the static schedule)
   int weno = 0, flux = 0, update = 0;
   int pred = 0;  // 0 one kernel, 2 split, 3 split (cold pass x3)
 };
