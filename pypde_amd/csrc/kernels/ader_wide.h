@@ -9,8 +9,8 @@
 // row j (right products), and scalars are formed by every lane alike.  What
 // bounds it is the latency of the dependent chains (Householder sums, Horner
 // steps, QR sweeps), hidden only by other wavefronts.  On the 17-variable
-// model, 200 cells, order 2, a launch: face flux 1340 -> 92 us and timestep 726 ->
-// 75 us (a matrix takes about 19,000 cycles to reduce, 5,300 for its
+// model, 200 cells, order 2, a launch: face flux 1340 -> 88.5 us and timestep
+// 726 -> 72 us (a matrix takes about 19,000 cycles to reduce, 5,300 for its
 // characteristic polynomial, 3,500 for the roots, 3,000 for the certificate
 // and, for the half of them that need it, 88,000 for QR).
 //
@@ -148,9 +148,11 @@ DEV void wide_root_starts(const WideMat& W, const double (&c)[V + 1], int lane, 
   *xlo = -u;
 }
 
-// house<M> without branches: both forms of v0 are computed and one selected.
+// house<M>, every lane alike, with both forms of v0 computed and one selected.
 // *head receives sqrt(x0^2 + (x1^2 (+ x2^2))), the entry the reflector leaves,
-// whose square root overlaps the others'.
+// whose square root overlaps the others'.  Its chain of a square root and two
+// divisions is much of what a step of the QR waits for: without operand scaling
+// (sqrt_mid, in house's range) face flux 92 -> 88.5 us, timestep 75 -> 72 us.
 template <int M>
 DEV double wide_house(const double (&x)[3], double (&v)[3], double* head) {
   double sigma = x[1] * x[1];
@@ -159,13 +161,22 @@ DEV double wide_house(const double (&x)[3], double (&v)[3], double* head) {
     sigma = dfma(x[2], x[2], sigma);
     tail = tail + x[2] * x[2];
   }
-  const double mu = dsqrt(dfma(x[0], x[0], sigma));
-  *head = dsqrt(x[0] * x[0] + tail);
+  const double mu2 = dfma(x[0], x[0], sigma), h2 = x[0] * x[0] + tail;
+  v[1] = x[1];
+  v[2] = x[2];
+  if ((sigma > HOUSE_TINY) & (mu2 <= 0x1p60)) {
+    const double mu = sqrt_mid(mu2);
+    *head = sqrt_mid(h2);
+    const double low = x[0] - mu, high = -div_mid(sigma, x[0] + mu);
+    const double v0 = x[0] <= 0.0 ? low : high;
+    v[0] = v0;
+    return 2.0 * recip_mid(dfma(v0, v0, sigma));
+  }
+  const double mu = dsqrt(mu2);
+  *head = dsqrt(h2);
   const double low = x[0] - mu, high = -sigma / (x[0] + mu);
   const double v0 = x[0] <= 0.0 ? low : high;
   v[0] = v0;
-  v[1] = x[1];
-  v[2] = x[2];
   const double beta = 2.0 / dfma(v0, v0, sigma);
   return sigma <= HOUSE_TINY ? 0.0 : beta;
 }
