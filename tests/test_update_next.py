@@ -71,3 +71,27 @@ def test_largest_grid_of_the_joint_kernel_and_the_next(n):
         assert np.array_equal(sol.state(), want)
     finally:
         sol.close()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("name,order,stiff,bc", [("ncadvect", 3, False, 1), ("ncadvect", 2, True, 0),
+                                                 ("reactive2d", 3, True, 0), ("advect", 4, False, 1)])
+def test_source_and_nonconservative_terms(name, order, stiff, bc):
+    n, V = 100, systems.SYSTEMS[name]["V"]
+    if name == "reactive2d":
+        u0 = np.ascontiguousarray(systems.reactive_channel(n, 8, seed=5)[:, 3])
+        tf = 1e-2
+    else:
+        x = (np.arange(n) + 0.5) / n
+        u0 = np.stack([1.0 + 0.3 * np.sin(2 * np.pi * (x + 0.2 * v)) for v in range(V)], axis=1)
+        tf = 1.0
+    want, _, st, rc = cc.oracle_solve(name, u0, tf, [1.0], bc, order, stiff=stiff, max_steps=9)
+    assert rc == 0 and st.steps == 9 and np.isfinite(want).all()
+    sol = Solver(u0, [1.0], systems.source(name), order=order, stiff=stiff,
+                 boundaryTypes=["transitive", "periodic"][bc])
+    try:
+        got = sol.run(tf, max_steps=9)
+        assert got["steps"] == 9
+        assert np.array_equal(sol.state(), want)
+    finally:
+        sol.close()
