@@ -178,8 +178,13 @@ DEV void callS(double* out, const double* q) {
 }
 
 // F is staged in LDS one time node at a time (NTF = 1), except for a viscous
-// F, whose gradient traces need every time node's derivatives (NTF = N).
-constexpr int NTF = PDE_SECOND ? N : 1;
+// F, whose gradient traces need every time node's derivatives, and in the
+// stiff predictor with the plain guess (NTF = N): at two wavefronts per SIMD
+// nothing hides N exchanges one after the other, and all time nodes at once
+// overlap (reactive channel 436 -> 419 us, 219 -> 241 registers; the Picard
+// predictor's time does not change).  The split's cold pass, which is there
+// for its few registers (139, 233 with all at once), stages one at a time.
+constexpr int NTF = PDE_SECOND || (PDE_STIFF && !PDE_GUESS) ? N : 1;
 struct PredLDS {
 #if PDE_SECOND || PDE_USE_B
   double q[N][CPW][ND][VL];
@@ -262,6 +267,7 @@ DEV void grad_traces(const NodeCtx& c, PredLDS& sm, const Geom& g, long cell, bo
 // in dqs (zero when no term reads it).  With
 // NTF = 1, F of one time node at a time passes through LDS (two barriers per
 // time node); every (t, v) result is the same either way.
+template <int TF = NTF>
 DEV void node_rhs(const NodeCtx& c, PredLDS& sm, const double (&q)[N][V], const double* w,
                   double dt, const Geom& g, bool active, double (&rhs)[N][V],
                   double (&dqs)[N][D][V]) {
@@ -314,7 +320,7 @@ DEV void node_rhs(const NodeCtx& c, PredLDS& sm, const double (&q)[N][V], const 
       rhs[t][v] = rr * dt + c.c0(t) * w[v];
     }
   };
-  if constexpr (NTF == N) {
+  if constexpr (TF == N) {
     if (active) {
 #pragma unroll
       for (int t = 0; t < N; t++) eval_f(t, t);
@@ -705,7 +711,7 @@ DEV void predictor_static_body(PredLDS& sm, const double* __restrict__ wh,
     if constexpr (FIRST)
       node_rhs_const(c, sm, q, w, dt, g, active, rhs, dqs);
     else
-      node_rhs(c, sm, q, w, dt, g, active, rhs, dqs);
+      node_rhs<MODE == 1 && !PDE_SECOND ? 1 : NTF>(c, sm, q, w, dt, g, active, rhs, dqs);
     bool more = false;
     bool skip = false;
     trips++;

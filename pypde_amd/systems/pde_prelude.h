@@ -22,6 +22,17 @@
 #define PDE_LDEXP(x, k) __builtin_ldexp(x, k)
 #define PDE_FMA(a, b, c) __builtin_fma(a, b, c)
 #define PDE_FREXP(x, e) __builtin_frexp(x, e)
+/* p r + c with a constant c, which stays in scalar registers.  Left to itself
+ * the compiler keeps the coefficients of a polynomial in vector registers
+ * across the loops around it and, since the multiply-add it picks overwrites
+ * its addend, copies one before each step (reactive channel, predictor: 235 ->
+ * 219 registers and a twentieth fewer instructions per iteration). */
+__device__ static inline double pde_fma_const(double p, double r, double c) {
+  double out;
+  asm("v_fma_f64 %0, %1, %2, %3" : "=v"(out) : "v"(p), "v"(r), "s"(c));
+  return out;
+}
+#define PDE_FMA_C(p, r, c) pde_fma_const(p, r, c)
 #else
 #include <math.h>
 #define PDE_FN static inline
@@ -29,6 +40,7 @@
 #define PDE_LDEXP(x, k) ldexp(x, k)
 #define PDE_FMA(a, b, c) fma(a, b, c)
 #define PDE_FREXP(x, e) frexp(x, e)
+#define PDE_FMA_C(p, r, c) fma(p, r, c)
 #endif
 
 /* exp(x) by Cody-Waite argument reduction (x = k ln2 + r, |r| <= ln2/2, ln2 split
@@ -47,16 +59,16 @@ PDE_FN double pde_exp(double x) {
   r = PDE_FMA(-k, ln2_lo, r);
   /* 1/j! for j = 13 .. 1 */
   double p = 1.6059043836821613e-10;
-  p = PDE_FMA(p, r, 2.08767569878681e-09);
-  p = PDE_FMA(p, r, 2.505210838544172e-08);
-  p = PDE_FMA(p, r, 2.755731922398589e-07);
-  p = PDE_FMA(p, r, 2.7557319223985893e-06);
-  p = PDE_FMA(p, r, 2.48015873015873e-05);
-  p = PDE_FMA(p, r, 0.0001984126984126984);
-  p = PDE_FMA(p, r, 0.001388888888888889);
-  p = PDE_FMA(p, r, 0.008333333333333333);
-  p = PDE_FMA(p, r, 0.041666666666666664);
-  p = PDE_FMA(p, r, 0.16666666666666666);
+  p = PDE_FMA_C(p, r, 2.08767569878681e-09);
+  p = PDE_FMA_C(p, r, 2.505210838544172e-08);
+  p = PDE_FMA_C(p, r, 2.755731922398589e-07);
+  p = PDE_FMA_C(p, r, 2.7557319223985893e-06);
+  p = PDE_FMA_C(p, r, 2.48015873015873e-05);
+  p = PDE_FMA_C(p, r, 0.0001984126984126984);
+  p = PDE_FMA_C(p, r, 0.001388888888888889);
+  p = PDE_FMA_C(p, r, 0.008333333333333333);
+  p = PDE_FMA_C(p, r, 0.041666666666666664);
+  p = PDE_FMA_C(p, r, 0.16666666666666666);
   p = PDE_FMA(p, r, 0.5);
   p = PDE_FMA(p, r, 1.0);
   p = PDE_FMA(p, r, 1.0);
