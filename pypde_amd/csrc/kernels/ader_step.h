@@ -183,7 +183,7 @@ DEV void callS(double* out, const double* q) {
 // nothing hides N exchanges one after the other, and all time nodes at once
 // overlap (reactive channel 436 -> 419 us, 219 -> 241 registers; the Picard
 // predictor's time does not change).  The split's cold pass, which is there
-// for its few registers (139, 233 with all at once), stages one at a time.
+// for its few registers (141, 233 with all at once), stages one at a time.
 constexpr int NTF = PDE_SECOND || (PDE_STIFF && !PDE_GUESS) ? N : 1;
 struct PredLDS {
 #if PDE_SECOND || PDE_USE_B
@@ -697,7 +697,7 @@ DEV void predictor_static_body(PredLDS& sm, const double* __restrict__ wh,
   // from the plain guess, whose iterate is constant in time (the wave-uniform
   // q = w), so the right-hand side needs F, S and the derivatives once.  It is
   // peeled off the loop so that the loop holds one right-hand side only
-  // (the stiff cold pass, 157 registers for the reactive channel, needed 26
+  // (the stiff cold pass, 141 registers for the reactive channel, needed 26
   // more with both).
   auto iterate = [&](auto firstc) {
     constexpr bool FIRST = decltype(firstc)::value;
