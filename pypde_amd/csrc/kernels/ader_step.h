@@ -963,10 +963,11 @@ k_predictor_static(const double* __restrict__ wh, const double* __restrict__ gue
 extern "C" __global__ void __launch_bounds__(64)
 k_predictor_cold(const double* __restrict__ wh, double* __restrict__ tr, double* __restrict__ vol,
                  double* __restrict__ qh, StepState* st, Geom g, double newton_tol,
-                 int newton_maxit, unsigned int* __restrict__ hot) {
+                 int newton_maxit, unsigned int* __restrict__ hot,
+                 double* __restrict__ trd) {
   __shared__ PredLDS sm;
   predictor_static_body<1>(sm, wh, nullptr, tr, vol, qh, st, g, newton_tol, newton_maxit,
-                           nullptr, hw_blk(), hot);
+                           trd, hw_blk(), hot);
 }
 // The cold pass with the register budget of three wavefronts per SIMD (168
 // registers; whatever does not fit spills), for the autotuner to weigh
@@ -974,18 +975,20 @@ k_predictor_cold(const double* __restrict__ wh, double* __restrict__ tr, double*
 extern "C" __global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(3, 3)))
 k_predictor_cold3(const double* __restrict__ wh, double* __restrict__ tr, double* __restrict__ vol,
                   double* __restrict__ qh, StepState* st, Geom g, double newton_tol,
-                  int newton_maxit, unsigned int* __restrict__ hot) {
+                  int newton_maxit, unsigned int* __restrict__ hot,
+                  double* __restrict__ trd) {
   __shared__ PredLDS sm;
   predictor_static_body<1>(sm, wh, nullptr, tr, vol, qh, st, g, newton_tol, newton_maxit,
-                           nullptr, hw_blk(), hot);
+                           trd, hw_blk(), hot);
 }
 extern "C" __global__ void __launch_bounds__(64)
 k_predictor_hot(const double* __restrict__ wh, double* __restrict__ tr, double* __restrict__ vol,
                 double* __restrict__ qh, StepState* st, Geom g, double newton_tol,
-                int newton_maxit, unsigned int* __restrict__ hot) {
+                int newton_maxit, unsigned int* __restrict__ hot,
+                double* __restrict__ trd) {
   __shared__ PredLDS sm;
   predictor_static_body<2>(sm, wh, nullptr, tr, vol, qh, st, g, newton_tol, newton_maxit,
-                           nullptr, hw_blk(), hot);
+                           trd, hw_blk(), hot);
 }
 #endif
 
@@ -2365,7 +2368,7 @@ k_predictor_cold_b(const Member* ms, const BlkMap* map, int nm, double newton_to
   __shared__ PredLDS sm;
   PYPDE_BATCH_MEMBER
   predictor_static_body<1>(sm, M.wh, nullptr, M.tr, M.vol, nullptr, M.st, M.g, newton_tol,
-                           newton_maxit, nullptr, b, M.hot);
+                           newton_maxit, M.trd, b, M.hot);
 }
 extern "C" __global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(3, 3)))
 k_predictor_cold3_b(const Member* ms, const BlkMap* map, int nm, double newton_tol,
@@ -2373,7 +2376,7 @@ k_predictor_cold3_b(const Member* ms, const BlkMap* map, int nm, double newton_t
   __shared__ PredLDS sm;
   PYPDE_BATCH_MEMBER
   predictor_static_body<1>(sm, M.wh, nullptr, M.tr, M.vol, nullptr, M.st, M.g, newton_tol,
-                           newton_maxit, nullptr, b, M.hot);
+                           newton_maxit, M.trd, b, M.hot);
 }
 extern "C" __global__ void __launch_bounds__(64)
 k_predictor_hot_b(const Member* ms, const BlkMap* map, int nm, double newton_tol,
@@ -2381,7 +2384,7 @@ k_predictor_hot_b(const Member* ms, const BlkMap* map, int nm, double newton_tol
   __shared__ PredLDS sm;
   PYPDE_BATCH_MEMBER
   predictor_static_body<2>(sm, M.wh, nullptr, M.tr, M.vol, nullptr, M.st, M.g, newton_tol,
-                           newton_maxit, nullptr, b, M.hot);
+                           newton_maxit, M.trd, b, M.hot);
 }
 
 #endif

@@ -639,7 +639,7 @@ int enqueue_step(pypde_ctx* c, bool guess_now, std::vector<hipEvent_t>* evs, boo
     std::vector<void*> a = {&w, &gs, &t, &v, &qh, &st, &g, &tol, &maxit, &td};
     if (c->pred_split && c->fn[K_PRED_COLD] && c->fn[K_PRED_HOT] && !gs && c->hot) {
       unsigned int* hl = c->hot;
-      std::vector<void*> b = {&w, &t, &v, &qh, &st, &g, &tol, &maxit, &hl};
+      std::vector<void*> b = {&w, &t, &v, &qh, &st, &g, &tol, &maxit, &hl, &td};
       const unsigned blocks = (unsigned)cdiv(g.nwc, c->CPW);
       const int kc = (c->pred_cold3 && c->fn[K_PRED_COLD3]) ? K_PRED_COLD3 : K_PRED_COLD;
       if ((rc = launch(c, kc, dim3(blocks), dim3(64), b))) return rc;
