@@ -1,0 +1,26 @@
+// Extents of a launch of many workgroups.
+//
+// A launch is refused when gridDim.x * blockDim.x reaches 2^32 (the limit that
+// hip_runtime_api.h states).  With a workgroup of 128 threads per face point
+// a 17-variable grid of 2048 x 2048 cells at order 2 is past it, so workgroups
+// that do not fit in x continue in y; kernels number them x + y gridDim.x
+// (blk_x) and those past the last one, fewer than the grid has rows, find no work.
+#pragma once
+
+namespace pypde {
+
+constexpr unsigned long GRID_THREADS = (1ul << 32) - 1;
+
+struct Grid {
+  unsigned int x, y;
+};
+
+// The fewest rows of equal length that hold `blocks` workgroups of `threads`.
+inline Grid grid_of(unsigned long blocks, unsigned int threads,
+                    unsigned long limit = GRID_THREADS) {
+  const unsigned long fit = limit / threads > 0 ? limit / threads : 1;
+  const unsigned long rows = blocks > fit ? (blocks + fit - 1) / fit : 1;
+  return {(unsigned int)((blocks + rows - 1) / rows), (unsigned int)rows};
+}
+
+}  // namespace pypde

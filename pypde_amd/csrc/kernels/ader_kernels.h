@@ -88,6 +88,10 @@ struct Blk {
 DEV Blk hw_blk() {
   return {blockIdx.x, blockIdx.y, blockIdx.z, gridDim.x * gridDim.y * gridDim.z};
 }
+// Launches numbered in x alone: workgroups that do not fit in x continue in y
+// (grid_of in grid.h), and the last row may hold some past the last one.
+DEV unsigned int blk_x() { return blockIdx.y * gridDim.x + blockIdx.x; }
+DEV Blk lin_blk() { return {blk_x(), 0u, 0u, gridDim.x * gridDim.y}; }
 
 // Position of workgroup i of n in an order that gives each of the 8 XCDs
 // runs of XCD_RUN consecutive positions: workgroups are dispatched to the
@@ -300,7 +304,7 @@ DEV void weno_1d(const double* __restrict__ u, double* __restrict__ wh, const Ge
        Geom g, int ghost, int nin0, int nin1, long out_stride, double* __restrict__ wm) {      \
     if (st && st->done) return;                                                                \
     if constexpr (D == 1)                                                                      \
-      weno_1d(u, wh, g, ghost, nin0, out_stride, wm, hw_blk());                                \
+      weno_1d(u, wh, g, ghost, nin0, out_stride, wm, lin_blk());                               \
     else                                                                                       \
       weno_2d<TX, TY>(u, wh, g, ghost, nin0, nin1, out_stride, wm, hw_blk());                  \
   }
@@ -460,7 +464,7 @@ DEV void dt_body(const double* __restrict__ wh, const double* __restrict__ wm, S
 
 extern "C" __global__ void __launch_bounds__(256)
 k_dt(const double* __restrict__ wh, const double* __restrict__ wm, StepState* st, Geom g) {
-  dt_body(wh, wm, st, g, hw_blk());
+  dt_body(wh, wm, st, g, lin_blk());
 }
 
 // dt = CFL / MAX, x0.2 while count <= 5, clamped to tf - t (stepper.cpp:67-75),
@@ -497,7 +501,7 @@ k_eig_batch(const double* __restrict__ A, const double* __restrict__ x, double* 
   // Osher stop at V = 8)
   __shared__ WideMat mats[WIDE_WAVES];
   const int lane = threadIdx.x & 63;
-  const long i0 = (long)blockIdx.x * 256 + (threadIdx.x & ~63u);
+  const long i0 = (long)blk_x() * 256 + (threadIdx.x & ~63u);
   for (long k = i0; k < i0 + 64 && k < n; k++) {
     double col[V];
 #pragma unroll
@@ -508,7 +512,7 @@ k_eig_batch(const double* __restrict__ A, const double* __restrict__ x, double* 
   (void)x;
   (void)which;
 #else
-  const long i = (long)blockIdx.x * 256 + threadIdx.x;
+  const long i = (long)blk_x() * 256 + threadIdx.x;
   if (i >= n) return;
   double H[V * V];
 #pragma unroll

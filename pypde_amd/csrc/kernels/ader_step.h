@@ -953,7 +953,7 @@ k_predictor_static(const double* __restrict__ wh, const double* __restrict__ gue
                    double* __restrict__ trd) {
   __shared__ PredLDS sm;
   predictor_static_body(sm, wh, guess, tr, vol, qh, st, g, newton_tol, newton_maxit, trd,
-                        hw_blk());
+                        lin_blk());
 }
 
 #if PDE_STIFF && !PDE_GUESS
@@ -967,7 +967,7 @@ k_predictor_cold(const double* __restrict__ wh, double* __restrict__ tr, double*
                  double* __restrict__ trd) {
   __shared__ PredLDS sm;
   predictor_static_body<1>(sm, wh, nullptr, tr, vol, qh, st, g, newton_tol, newton_maxit,
-                           trd, hw_blk(), hot);
+                           trd, lin_blk(), hot);
 }
 // The cold pass with the register budget of three wavefronts per SIMD (168
 // registers; whatever does not fit spills), for the autotuner to weigh
@@ -979,7 +979,7 @@ k_predictor_cold3(const double* __restrict__ wh, double* __restrict__ tr, double
                   double* __restrict__ trd) {
   __shared__ PredLDS sm;
   predictor_static_body<1>(sm, wh, nullptr, tr, vol, qh, st, g, newton_tol, newton_maxit,
-                           trd, hw_blk(), hot);
+                           trd, lin_blk(), hot);
 }
 extern "C" __global__ void __launch_bounds__(64)
 k_predictor_hot(const double* __restrict__ wh, double* __restrict__ tr, double* __restrict__ vol,
@@ -988,7 +988,7 @@ k_predictor_hot(const double* __restrict__ wh, double* __restrict__ tr, double* 
                 double* __restrict__ trd) {
   __shared__ PredLDS sm;
   predictor_static_body<2>(sm, wh, nullptr, tr, vol, qh, st, g, newton_tol, newton_maxit,
-                           trd, hw_blk(), hot);
+                           trd, lin_blk(), hot);
 }
 #endif
 
@@ -1113,7 +1113,7 @@ k_predictor_f32(const double* __restrict__ wh, const double* __restrict__ gin,
   const int lane = threadIdx.x;
   NodeCtx c;
   node_ctx(c, lane, PRED_NODE_TAB(sm));
-  const long cell = (long)blockIdx.x * CPW + c.slot;
+  const long cell = (long)blk_x() * CPW + c.slot;
   const bool valid = (c.slot < CPW) && (cell < g.nwc);
   float rdx[D];
 #pragma unroll
@@ -1213,7 +1213,7 @@ k_predictor_f32(const double* __restrict__ wh, const double* __restrict__ gin,
   }
   unsigned long long mine = (valid && c.idx == 0) ? (unsigned long long)it : 0ull;
   mine = wave_sum_u64(mine);
-  if (lane == 0 && mine) atomicAdd(&st->pstat[blockIdx.x & 63][7], mine);
+  if (lane == 0 && mine) atomicAdd(&st->pstat[blk_x() & 63][7], mine);
 }
 #endif
 
@@ -1248,6 +1248,7 @@ DEV void flux_wide(const double* __restrict__ tr, double* __restrict__ ff, doubl
                    const Geom& g, long blk) {
   const long nf = g.nf[d];
   const long item = blk;
+  if (item >= nf * (N * ND1)) return;
   const long f = item % nf;
   const int j = (int)((item / nf) % ND1);
   const int t = (int)(item / (nf * ND1));
@@ -1656,7 +1657,7 @@ DEV void flux_all(const double* __restrict__ tr, const FaceOut& out, const Geom&
   extern "C" __global__ void __launch_bounds__(BS)                                             \
   NAME(const double* __restrict__ tr, FaceOut out, const StepState* st, Geom g,                \
        const double* __restrict__ trd) {                                                       \
-    flux_all<MODE, BS>(tr, out, g, trd, &st->done, hw_blk());                                  \
+    flux_all<MODE, BS>(tr, out, g, trd, &st->done, lin_blk());                                  \
   }
 PYPDE_FLUX_KERNEL(k_flux, 0, 128)
 #if PDE_V <= 8
@@ -1763,7 +1764,7 @@ extern "C" __global__ void __launch_bounds__(256)
 k_update(double* __restrict__ u, const double* __restrict__ vol, FaceBufs fbufs,
          double* __restrict__ ret, StepState* st, Geom g) {
   if (st->done) return;
-  const Blk b = hw_blk();
+  const Blk b = lin_blk();
   update_cell(u, vol, fbufs, ret, st, g, b);
   if (last_workgroup(st, &st->step_ticket, 10, b)) advance_step(st, g.ndt);
 }
@@ -1889,7 +1890,7 @@ DEV void update_rows(double* __restrict__ u, const double* __restrict__ vol, con
   k_update_r##R_(double* __restrict__ u, const double* __restrict__ vol, FaceBufs fbufs,      \
                  double* __restrict__ ret, StepState* st, Geom g) {                            \
     if (st->done) return;                                                                      \
-    const Blk b = hw_blk();                                                                    \
+    const Blk b = lin_blk();                                                                    \
     update_rows<R_>(u, vol, fbufs, ret, st, g, b);                                             \
     if (last_workgroup(st, &st->step_ticket, 10, b)) advance_step(st, g.ndt);                  \
   }
@@ -1918,7 +1919,7 @@ k_update_next(double* u, double* u2, const double* __restrict__ vol, FaceBufs fb
   __shared__ double s0[V][RX];
   __shared__ double mean[V][NEXT_W];
   if (st->done) return;
-  const Blk b = hw_blk();
+  const Blk b = lin_blk();
   const int tid = threadIdx.x, flip = st->flip, push = st->push;
   const double dt = st->dt, tn = st->t + dt;
   const bool last_step =
@@ -2057,14 +2058,14 @@ DEV void advance_step(StepState* st, int ndt) {
 
 // Interleaved [cell][v] <-> structure-of-arrays [v][cell].
 extern "C" __global__ void k_aos_to_soa(const double* __restrict__ a, double* __restrict__ s, long ncell) {
-  long i = (long)blockIdx.x * 256 + threadIdx.x;
+  long i = (long)blk_x() * 256 + threadIdx.x;
   if (i >= ncell * V) return;
   long c = i / V;
   int v = (int)(i % V);
   s[(long)v * ncell + c] = a[i];
 }
 extern "C" __global__ void k_soa_to_aos(const double* __restrict__ s, double* __restrict__ a, long ncell) {
-  long i = (long)blockIdx.x * 256 + threadIdx.x;
+  long i = (long)blk_x() * 256 + threadIdx.x;
   if (i >= ncell * V) return;
   long c = i / V;
   int v = (int)(i % V);
@@ -2079,7 +2080,7 @@ extern "C" __global__ void __launch_bounds__(256)
 k_planes_to_rows(const double* __restrict__ s, double* __restrict__ a, long ncell) {
   constexpr int P = ND * V, SLAB = P < 32 ? P : 32;
   __shared__ double t[SLAB][65];
-  const long c0 = (long)blockIdx.x * 64;
+  const long c0 = (long)blk_x() * 64;
   const int nc = ncell - c0 < 64 ? (int)(ncell - c0) : 64;
   for (int p0 = 0; p0 < P; p0 += SLAB) {
     const int np = P - p0 < SLAB ? P - p0 : SLAB;
@@ -2102,7 +2103,7 @@ constexpr int MLP_OUT = NT * V;
 extern "C" __global__ void __launch_bounds__(256)
 k_harvest(const double* __restrict__ wh, const double* __restrict__ qh, const StepState* st,
           float* __restrict__ X, float* __restrict__ Y, long ldx, long col0, long nwc) {
-  const long c = (long)blockIdx.x * 256 + threadIdx.x;
+  const long c = (long)blk_x() * 256 + threadIdx.x;
   if (c >= nwc) return;
   const double dt = st->dt;
   for (int k = 0; k < ND * V; k++) X[(long)k * ldx + col0 + c] = (float)wh[(long)k * nwc + c];
@@ -2172,7 +2173,7 @@ DEV const float* aux_src(const MLPW& m, int i, int* k) {
 
 extern "C" __global__ void __launch_bounds__(256)
 k_mlp_pack(MLPW m, bf16x4* __restrict__ pack, float* __restrict__ aux) {
-  const long i = (long)blockIdx.x * 256 + threadIdx.x;
+  const long i = (long)blk_x() * 256 + threadIdx.x;
   if (i < (long)NFRAG * 64) {
     const int lane = (int)(i % 64), f = (int)(i / 64);
     if (f < RB_HID * KB_IN)
@@ -2209,7 +2210,7 @@ k_mlp_guess(const double* __restrict__ wh, const StepState* st, const bf16x4* __
   const float* sa = aux;
   const double dt = st->dt;
   {
-    const long cb = (long)blockIdx.x * 4 + (threadIdx.x >> 6);
+    const long cb = (long)blk_x() * 4 + (threadIdx.x >> 6);
     const long cell = cb * 32 + (lane & 31);
     const bool ok = cell < nwc;
     bf16x4 xb[KB_IN];
@@ -2325,8 +2326,10 @@ DEV int batch_member(const PDE_CONST_AS BlkMap* map, int nm, unsigned int blk) {
 // member's own launch); declares M (the member) and b (the coordinates).
 #define PYPDE_BATCH_MEMBER                                                                     \
   const PDE_CONST_AS BlkMap* cmap = (const PDE_CONST_AS BlkMap*)map;                           \
-  const int m_ = batch_member(cmap, nm, blockIdx.x);                                           \
-  const unsigned int loc_ = blockIdx.x - cmap[m_].start;                                       \
+  const unsigned int blk_ = blk_x();                                                           \
+  if (blk_ >= cmap[nm].start) return;                                                          \
+  const int m_ = batch_member(cmap, nm, blk_);                                                 \
+  const unsigned int loc_ = blk_ - cmap[m_].start;                                             \
   const unsigned int gx_ = cmap[m_].gx, gy_ = cmap[m_].gy;                                     \
   const Blk b = {loc_ % gx_, (loc_ / gx_) % gy_, loc_ / (gx_ * gy_), gx_ * gy_ * cmap[m_].gz}; \
   const Member& M = *(const Member*)&((const PDE_CONST_AS Member*)ms)[m_];

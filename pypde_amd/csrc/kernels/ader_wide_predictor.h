@@ -393,6 +393,7 @@ DEV void wide_predictor(WidePred& sm, const double* __restrict__ wh,
   const double dt = st->dt;
   const int lane = threadIdx.x;
   const long cell = (long)xcd_order(blk.x, blk.n);
+  if (cell >= g.nwc) return;
 #pragma unroll 1
   for (int e = lane; e < ND * V; e += 64) {
     const int node = e / V, v = e % V;
@@ -591,7 +592,7 @@ k_predictor_static(const double* __restrict__ wh, const double* __restrict__ gue
                    double* __restrict__ trd) {
   __shared__ WidePred sm;
   (void)trd;
-  wide_predictor(sm, wh, guess, tr, vol, qh, st, g, newton_tol, newton_maxit, hw_blk());
+  wide_predictor(sm, wh, guess, tr, vol, qh, st, g, newton_tol, newton_maxit, lin_blk());
 }
 #if PDE_BATCH
 extern "C" __global__ void __launch_bounds__(64)

@@ -28,6 +28,7 @@
 #include <string>
 #include <vector>
 
+#include "grid.h"
 #include "tables.h"
 #include "transfer.h"
 
@@ -395,7 +396,7 @@ struct pypde_ctx {
   void* mlp_pack = nullptr;  // the attached model's BF16 weight fragments
   float* mlp_aux = nullptr;  // ... and its FP32 normalisation and bias vectors
   double* qh = nullptr;     // full predictor output (harvest)
-  int n_cu = 0;             // compute units of the device
+  unsigned long grid_threads = pypde::GRID_THREADS;  // threads of a launch's row of workgroups
   bool pred_fixed = false;  // schedule fixed by PYPDE_PRED_SCHEDULE (not tuned)
   bool pred_split = false;  // cold pass over every cell, hot pass over the cells it hands on
   bool pred_cold3 = false;  // ... with the cold pass built for three wavefronts per SIMD
@@ -528,6 +529,16 @@ int launch(pypde_ctx* c, int k, dim3 grid, dim3 block, std::vector<void*>& args)
   return 0;
 }
 
+// `blocks` workgroups of a kernel that numbers them along one axis (blk_x).
+dim3 lin_grid(long blocks, int threads, unsigned long limit = pypde::GRID_THREADS) {
+  const pypde::Grid g = pypde::grid_of((unsigned long)blocks, (unsigned)threads, limit);
+  return dim3(g.x, g.y);
+}
+
+int launch(pypde_ctx* c, int k, long blocks, int threads, std::vector<void*>& args) {
+  return launch(c, k, lin_grid(blocks, threads, c->grid_threads), dim3((unsigned)threads), args);
+}
+
 long cdiv(long a, long b) { return (a + b - 1) / b; }
 
 // Face-flux launches (FLUX_SPLIT and flux_all in ader_step.h): variants,
@@ -588,7 +599,7 @@ int enqueue_step(pypde_ctx* c, bool guess_now, std::vector<hipEvent_t>* evs, boo
     std::vector<void*> a = {&uu, &w, &st, &g, &ghost, &z, &z, &os, &wm};
     const int wv = c->D == 1 ? 0 : c->tune.weno;
     const int TX = WENO_TILE[wv][0], TY = WENO_TILE[wv][1];
-    dim3 grid = c->D == 1 ? dim3((unsigned)cdiv(g.nw[0], weno1_width(c->V)))
+    dim3 grid = c->D == 1 ? lin_grid(cdiv(g.nw[0], weno1_width(c->V)), 256, c->grid_threads)
                           : dim3((unsigned)cdiv(g.nw[1], TY), (unsigned)cdiv(g.nw[0], TX),
                                  (unsigned)c->V);
     if ((rc = launch(c, WENO_KID[wv], grid, dim3(256), a))) return rc;
@@ -600,7 +611,7 @@ int enqueue_step(pypde_ctx* c, bool guess_now, std::vector<hipEvent_t>* evs, boo
     StepState* st = c->st;
     std::vector<void*> a = {&w, &wm, &st, &g};
     // its last workgroup also turns the wave-speed maximum into dt
-    if ((rc = launch(c, K_DT, dim3((unsigned)cdiv(g.nwc * c->dt_lanes, 256)), dim3(256), a)))
+    if ((rc = launch(c, K_DT, cdiv(g.nwc * c->dt_lanes, 256), 256, a)))
       return rc;
   }
   mark();
@@ -613,7 +624,7 @@ int enqueue_step(pypde_ctx* c, bool guess_now, std::vector<hipEvent_t>* evs, boo
     long nwc = g.nwc;
     std::vector<void*> a = {&w, &st, &pk, &ax, &gb, &nwc};
     // four wavefronts of 32 cells per workgroup
-    if ((rc = launch(c, K_MLPGUESS, dim3((unsigned)cdiv(g.nwc, 128)), dim3(256), a))) return rc;
+    if ((rc = launch(c, K_MLPGUESS, cdiv(g.nwc, 128), 256, a))) return rc;
   }
   if (c->spec.mixed) {
     // FP32 phase: from the learned guess, a caller's guess or the plain one;
@@ -625,7 +636,7 @@ int enqueue_step(pypde_ctx* c, bool guess_now, std::vector<hipEvent_t>* evs, boo
     float tol32 = (float)c->opts.mixed_tol;
     int maxit32 = c->opts.mixed_maxit;
     std::vector<void*> a = {&w, &gin, &gout, &st, &g, &tol32, &maxit32};
-    if ((rc = launch(c, K_PRED32, dim3((unsigned)cdiv(g.nwc, 64 / c->ND)), dim3(64), a))) return rc;
+    if ((rc = launch(c, K_PRED32, cdiv(g.nwc, 64 / c->ND), 64, a))) return rc;
   }
   mark();
   {
@@ -640,12 +651,11 @@ int enqueue_step(pypde_ctx* c, bool guess_now, std::vector<hipEvent_t>* evs, boo
     if (c->pred_split && c->fn[K_PRED_COLD] && c->fn[K_PRED_HOT] && !gs && c->hot) {
       unsigned int* hl = c->hot;
       std::vector<void*> b = {&w, &t, &v, &qh, &st, &g, &tol, &maxit, &hl, &td};
-      const unsigned blocks = (unsigned)cdiv(g.nwc, c->CPW);
+      const long blocks = cdiv(g.nwc, c->CPW);
       const int kc = (c->pred_cold3 && c->fn[K_PRED_COLD3]) ? K_PRED_COLD3 : K_PRED_COLD;
-      if ((rc = launch(c, kc, dim3(blocks), dim3(64), b))) return rc;
-      if ((rc = launch(c, K_PRED_HOT, dim3(blocks), dim3(64), b))) return rc;
-    } else if ((rc = launch(c, K_PRED_STATIC,
-                            dim3((unsigned)cdiv(g.nwc, c->CPW)), dim3(64), a))) {
+      if ((rc = launch(c, kc, blocks, 64, b))) return rc;
+      if ((rc = launch(c, K_PRED_HOT, blocks, 64, b))) return rc;
+    } else if ((rc = launch(c, K_PRED_STATIC, cdiv(g.nwc, c->CPW), 64, a))) {
       return rc;
     }
   }
@@ -656,9 +666,8 @@ int enqueue_step(pypde_ctx* c, bool guess_now, std::vector<hipEvent_t>* evs, boo
     const StepState* st = c->st;
     const double* td = c->trd;
     std::vector<void*> a = {&t, &out, &st, &g, &td};
-    if ((rc = launch(c, FLUX_KID[c->tune.flux],
-                     dim3((unsigned)flux_blocks(c->spec, c->tune.flux, g)),
-                     dim3(flux_threads(c->spec, c->tune.flux)), a)))
+    if ((rc = launch(c, FLUX_KID[c->tune.flux], flux_blocks(c->spec, c->tune.flux, g),
+                     flux_threads(c->spec, c->tune.flux), a)))
       return rc;
   }
   mark();
@@ -669,7 +678,7 @@ int enqueue_step(pypde_ctx* c, bool guess_now, std::vector<hipEvent_t>* evs, boo
     FaceBufs fbufs = {{c->ff[0], c->ff[1]}, {c->fb[0], c->fb[1]}};
     StepState* st = c->st;
     std::vector<void*> a = {&uu, &u2, &v, &fbufs, &r, &w, &st, &g};
-    if ((rc = launch(c, K_NEXT, dim3((unsigned)cdiv(g.nwc, NEXT_W)), dim3(256), a))) return rc;
+    if ((rc = launch(c, K_NEXT, cdiv(g.nwc, NEXT_W), 256, a))) return rc;
   } else {
     double* uu = c->u;
     const double* v = c->vol;
@@ -679,7 +688,7 @@ int enqueue_step(pypde_ctx* c, bool guess_now, std::vector<hipEvent_t>* evs, boo
     std::vector<void*> a = {&uu, &v, &fbufs, &r, &st, &g};
     const int R = UPD_ROWS[c->tune.update];
     const long threads = R == 0 ? g.ncell : (long)c->V * cdiv(g.nx[0], R) * g.nx[1];
-    if ((rc = launch(c, UPD_KID[c->tune.update], dim3((unsigned)cdiv(threads, 256)), dim3(256), a)))
+    if ((rc = launch(c, UPD_KID[c->tune.update], cdiv(threads, 256), 256, a)))
       return rc;
   }
   mark();
@@ -908,6 +917,10 @@ static pypde_ctx* create_ctx(const char* src, bool useF, bool useB, bool useS, c
   // testing the path that grids of 2^31 flux items or w-cells take)
   if (const char* e = getenv("PYPDE_FLUX_IDX64"))
     if (e[0] == '1') g.idx32 = 0;
+  // PYPDE_GRID_THREADS=n: rows of at most n threads (for testing the numbering
+  // that launches of 2^32 threads and more take)
+  if (const char* e = getenv("PYPDE_GRID_THREADS"))
+    if (*e) c->grid_threads = strtoul(e, nullptr, 10);
   auto bail = [&](int code_) {
     rc = code_;
     pypde_destroy(c);
@@ -918,9 +931,6 @@ static pypde_ctx* create_ctx(const char* src, bool useF, bool useB, bool useS, c
     if (int r = compile_code(s, &code)) return bail(r);
     return bail(fail(PYPDE_ERR_HIP, "hipSetDevice(%d) failed: no usable GPU", c->device));
   }
-  if (hipDeviceGetAttribute(&c->n_cu, hipDeviceAttributeMultiprocessorCount, c->device) !=
-      hipSuccess)
-    c->n_cu = 0;
   if (int r = load_module(s, c->device, &c->mod, c->fn_plain, &c->code_key)) return bail(r);
   memcpy(c->fn, c->fn_plain, sizeof c->fn);
   if (pypde::take_stream(c->device, &c->stream) != hipSuccess)
@@ -973,7 +983,7 @@ int pypde_set_state(pypde_ctx* c, const double* u) {
   size_t n = c->g.ncell * c->V;
   HIPCHK(pypde::copy_to_device(c->tmp, u, n * sizeof(double), c->device, c->stream));
   std::vector<void*> a = {&c->tmp, &c->u, &c->g.ncell};
-  int rc = launch(c, K_A2S, dim3((unsigned)cdiv(n, 256)), dim3(256), a);
+  int rc = launch(c, K_A2S, cdiv((long)n, 256), 256, a);
   if (rc) return rc;
   HIPCHK(hipStreamSynchronize(c->stream));
   return 0;
@@ -983,7 +993,7 @@ int pypde_get_state(pypde_ctx* c, double* u) {
   HIPCHK(hipSetDevice(c->device));
   size_t n = c->g.ncell * c->V;
   std::vector<void*> a = {&c->u, &c->tmp, &c->g.ncell};
-  int rc = launch(c, K_S2A, dim3((unsigned)cdiv(n, 256)), dim3(256), a);
+  int rc = launch(c, K_S2A, cdiv((long)n, 256), 256, a);
   if (rc) return rc;
   HIPCHK(pypde::copy_to_host(u, c->tmp, n * sizeof(double), c->device, c->stream));
   return 0;
@@ -1334,7 +1344,7 @@ int pypde_run(pypde_ctx* c, double tf, long max_steps, int ndt, double* ret, pyp
   if (rows) {
     // final state into the last row (iterator.cpp:150)
     std::vector<void*> a = {&c->u, &c->tmp, &c->g.ncell};
-    int r2 = launch(c, K_S2A, dim3((unsigned)cdiv(row, 256)), dim3(256), a);
+    int r2 = launch(c, K_S2A, cdiv((long)row, 256), 256, a);
     if (r2) return r2;
     HIPCHK(hipMemcpyAsync(c->ret + (rows - 1) * row, c->tmp, row * sizeof(double),
                           hipMemcpyDeviceToDevice, c->stream));
@@ -1530,8 +1540,9 @@ static int enqueue_group_step(pypde_ensemble* e, const EnsGroup& gr) {
       a.push_back(&tol);
       a.push_back(&maxit);
     }
-    hipError_t err = hipModuleLaunchKernel(c->fn[kid], gr.blocks[stage], 1, 1, bs, 1, 1, 0,
-                                           gr.stream, a.data(), nullptr);
+    const dim3 grid = lin_grid(gr.blocks[stage], bs, c->grid_threads);
+    hipError_t err = hipModuleLaunchKernel(c->fn[kid], grid.x, grid.y, 1, bs, 1, 1, 0, gr.stream,
+                                           a.data(), nullptr);
     if (err != hipSuccess)
       return fail(PYPDE_ERR_HIP, "launch %s: %s", kernel_names[kid], hipGetErrorString(err));
     return 0;
@@ -1779,7 +1790,7 @@ int pypde_set_guess_model(pypde_ctx* c, const pypde_mlp* m) {
     void* pk = c->mlp_pack;
     float* ax = c->mlp_aux;
     std::vector<void*> a = {&mw, &pk, &ax};
-    int rc = launch(c, K_MLPPACK, dim3((unsigned)cdiv(std::max(nfrag * 64, naux), 256)), dim3(256), a);
+    int rc = launch(c, K_MLPPACK, cdiv(std::max(nfrag * 64, naux), 256), 256, a);
     if (rc) return rc;
     HIPCHK(hipStreamSynchronize(c->stream));
   }
@@ -1816,7 +1827,7 @@ int pypde_eig_batch(pypde_ctx* c, int which, const double* A, const double* x, l
   const double* a0 = dA;
   const double* x0 = dx;
   std::vector<void*> a = {&a0, &x0, &dout, &n, &which};
-  if ((rc = launch(c, K_EIG, dim3((unsigned)cdiv(n, 256)), dim3(256), a))) return done(rc);
+  if ((rc = launch(c, K_EIG, cdiv(n, 256), 256, a))) return done(rc);
   if (hipMemcpyAsync(out, dout, nout * sizeof(double), hipMemcpyDeviceToHost, c->stream) !=
           hipSuccess ||
       hipStreamSynchronize(c->stream) != hipSuccess)
@@ -1834,7 +1845,7 @@ int pypde_harvest_step(pypde_ctx* c, float* X, float* Y, long ldx, long col0, py
   const StepState* st = c->st;
   long nwc = c->g.nwc;
   std::vector<void*> a = {&w, &q, &st, &X, &Y, &ldx, &col0, &nwc};
-  rc = launch(c, K_HARVEST, dim3((unsigned)cdiv(nwc, 256)), dim3(256), a);
+  rc = launch(c, K_HARVEST, cdiv(nwc, 256), 256, a);
   if (rc) return rc;
   HIPCHK(hipStreamSynchronize(c->stream));
   (void)hipFree(c->qh);
@@ -2050,8 +2061,8 @@ int weno_solver(double* ret, double* u, int* nX, int ndim, int N, int V) {
   HIPCHK(pypde::copy_to_device(du, u, nin * V * sizeof(double), 0, st0));
   {
     void* a[] = {&du, &dus, &nin};
-    HIPCHK(hipModuleLaunchKernel(fn[K_A2S], (unsigned)cdiv(nin * V, 256), 1, 1, 256, 1, 1, 0, st0,
-                                 a, nullptr));
+    const dim3 gr = lin_grid(cdiv(nin * V, 256), 256);
+    HIPCHK(hipModuleLaunchKernel(fn[K_A2S], gr.x, gr.y, 1, 256, 1, 1, 0, st0, a, nullptr));
   }
   Geom g;
   memset(&g, 0, sizeof g);
@@ -2060,17 +2071,17 @@ int weno_solver(double* ret, double* u, int* nX, int ndim, int N, int V) {
   {
     double* wm = nullptr;
     void* a[] = {&dus, &dw, &st, &g, &ghost, &n0, &n1, &nout, &wm};
-    unsigned gx =
-        ndim == 1 ? (unsigned)cdiv(no[0], weno1_width(V)) : (unsigned)cdiv(no[1], 32);
-    unsigned gy = ndim == 1 ? 1 : (unsigned)cdiv(no[0], 8);
-    unsigned gz = ndim == 1 ? 1 : (unsigned)V;  // 2D: one variable per workgroup
-    HIPCHK(hipModuleLaunchKernel(fn[K_WENO], gx, gy, gz, 256, 1, 1, 0, st0, a, nullptr));
+    // 2D: one variable per workgroup
+    const dim3 gr = ndim == 1 ? lin_grid(cdiv(no[0], weno1_width(V)), 256)
+                              : dim3((unsigned)cdiv(no[1], 32), (unsigned)cdiv(no[0], 8),
+                                     (unsigned)V);
+    HIPCHK(hipModuleLaunchKernel(fn[K_WENO], gr.x, gr.y, gr.z, 256, 1, 1, 0, st0, a, nullptr));
   }
   // planes [node*V+v][cell] -> reference layout [cell][node][v]
   {
     void* a[] = {&dw, &du, &nout};
-    HIPCHK(hipModuleLaunchKernel(fn[K_P2R], (unsigned)cdiv(nout, P2R_CELLS), 1, 1, 256, 1, 1, 0,
-                                 st0, a, nullptr));
+    const dim3 gr = lin_grid(cdiv(nout, P2R_CELLS), 256);
+    HIPCHK(hipModuleLaunchKernel(fn[K_P2R], gr.x, gr.y, 1, 256, 1, 1, 0, st0, a, nullptr));
   }
   HIPCHK(pypde::copy_to_host(ret, du, nout * ND * V * sizeof(double), 0, st0));
   return 0;

@@ -1,0 +1,143 @@
+"""Launches whose workgroups continue in a second row of the grid, as they do
+from 2^32 threads on: the split into rows on the host, every kernel with rows
+of a few workgroups against one row, and a grid whose face flux is past the
+limit."""
+import os
+import subprocess
+
+import numpy as np
+import pytest
+
+from pypde_amd import systems
+from pypde_amd.solvers import Ensemble, Solver
+
+ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+
+
+def test_rows_hold_every_workgroup_below_the_limit(tmp_path):
+    main = tmp_path / "rows.cpp"
+    main.write_text('#include <cstdio>\n#include <cstdlib>\n#include "grid.h"\n'
+                    "int main(int n, char** a) {\n"
+                    "  for (int i = 1; i + 1 < n; i += 2) {\n"
+                    "    pypde::Grid g = pypde::grid_of(strtoul(a[i], 0, 10), atoi(a[i + 1]));\n"
+                    '    printf("%u %u\\n", g.x, g.y);\n  }\n}\n')
+    exe = str(tmp_path / "rows")
+    subprocess.run(["g++", "-std=c++17", "-I", os.path.join(ROOT, "pypde_amd", "csrc"), "-o", exe,
+                    str(main)], check=True)
+    # one workgroup, the largest single row, one more, and the 17-variable model's face points
+    # on 2048 x 2048 cells at order 2 and 4096 x 4096 at order 3
+    cases = [(1, 64), (2 ** 25 - 1, 128), (2 ** 25, 128), (2 ** 32 // 64 - 1, 64),
+             (2 * 2049 * 2048 * 4, 128), (2 * 4097 * 4096 * 9, 128), (3 * 10 ** 8, 1024)]
+    args = [str(x) for c in cases for x in c]
+    out = subprocess.run([exe] + args, check=True, capture_output=True, text=True).stdout.split("\n")
+    for (blocks, threads), line in zip(cases, out):
+        x, y = map(int, line.split())
+        assert x * threads < 2 ** 32 and blocks <= x * y < blocks + y
+        assert (y == 1) == (blocks * threads < 2 ** 32)
+
+
+def euler(nx, ny):
+    return np.ascontiguousarray(np.tile(systems.euler2d_modes(23, seed=3), (2, 2, 1))[:nx, :ny])
+
+
+def channel(nx, ny):
+    return systems.reactive_channel(nx, ny, seed=4)
+
+
+def gpr(*n):
+    u = np.zeros(n + (17,))
+    for i in np.ndindex(*n):
+        r = 1.0 if sum(i) < sum(n) / 2 else 0.5
+        u[i] = systems.gpr_state(r, r, (0.1 * r, 0.0, 0.02))
+    return u
+
+
+CASES = {
+    # the joint 1D kernel, and the separate ones
+    "tube": (lambda: systems.sod1d(1500), "euler1d", dict(order=3), "0,0,0,0"),
+    "tube_graph": (lambda: systems.sod1d(1500), "euler1d", dict(order=3, use_graph=True), "0,1,0,0"),
+    "euler_split": (lambda: euler(37, 41), "euler2d", dict(order=3), "1,2,1,0"),
+    "euler_rows": (lambda: euler(41, 37), "euler2d", dict(order=4), "2,0,3,0"),
+    "viscous": (lambda: euler(19, 21), "ns2d", dict(order=3, cfl=0.4), "0,2,2,0"),
+    "channel": (lambda: channel(48, 16), "reactive2d",
+                dict(order=3, stiff=True, reflect=systems.REACTIVE_REFLECT,
+                     boundaryTypes="reflective"), "0,1,1,2"),
+    "mixed": (lambda: euler(21, 34), "euler2d", dict(order=3, mixed=True), "0,0,0,0"),
+    "gpr1d": (lambda: gpr(70), "gpr", dict(order=2, stiff=True, cfl=0.5), "0,0,0,0"),
+    "gpr2d": (lambda: gpr(9, 11), "gpr", dict(order=2, stiff=True, cfl=0.5), "0,0,1,0"),
+}
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("name", list(CASES))
+def test_rows_give_the_same_bits(name, monkeypatch):
+    make, system, kw, tune = CASES[name]
+    u0 = make()
+    L = [n / 32 for n in u0.shape[:-1]]
+    monkeypatch.setenv("PYPDE_TUNE_FORCE", tune)
+    got = []
+    for row in ("", "768", "1280"):     # one row; 3 and 5 workgroups of 256 threads
+        monkeypatch.setenv("PYPDE_GRID_THREADS", row)
+        sol = Solver(u0, L, systems.source(system), **kw)
+        st = sol.run(1e300, max_steps=5)
+        got.append((sol.state(), st["pred_iters"], st["pred_cells"], st["pred_maxit"], st["t"]))
+        sol.close()
+    assert np.isfinite(got[0][0]).all()
+    for other in got[1:]:
+        assert np.array_equal(other[0], got[0][0]) and other[1:] == got[0][1:]
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("system,kw", [("euler2d", dict(order=3)),
+                                       ("gpr", dict(order=2, stiff=True, cfl=0.5))])
+def test_rows_of_batched_members(system, kw, monkeypatch):
+    if system == "euler2d":
+        grids = [euler(24, 31), euler(40, 12), euler(17, 19)]
+    else:
+        grids = [gpr(23), gpr(40), gpr(9)]
+    L = [[1.0] * (g.ndim - 1) for g in grids]
+    monkeypatch.setenv("PYPDE_TUNE_FORCE", "0,2,1,0")
+    got = []
+    for row in ("", "1280"):
+        monkeypatch.setenv("PYPDE_GRID_THREADS", row)
+        ens = Ensemble(grids, L, systems.source(system), **kw)
+        ens.run(1.0, max_steps=4)
+        got.append([ens.state(i) for i in range(len(grids))])
+        ens.close()
+    for a, b in zip(*got):
+        assert np.isfinite(a).all() and np.array_equal(a, b)
+
+
+NINE = """
+#define PDE_HAS_F 1
+PDE_FN void F(double *out, const double *Q, const double *dQ, int d) {
+  for (int i = 0; i < 9; i++) {
+    const double l = i > 0 ? Q[i - 1] : 0.0, r = i < 8 ? Q[i + 1] : 0.0;
+    out[i] = 0.5 * (l + r) * (1.0 + 0.1 * Q[0]);
+  }
+}
+"""
+
+
+@pytest.mark.gpu
+def test_face_points_past_the_limit_of_one_row(monkeypatch):
+    """2^25 cells of a nine-variable system: 2^25 + 1 face points of 128
+    threads.  The field repeats every 1024 cells, so each period equals a run
+    of one."""
+    monkeypatch.setenv("PYPDE_TUNE", "0")
+    period, n = 1024, 2 ** 25
+    x = (np.arange(period) + 0.5) / period
+    tile = np.stack([1.0 + 0.2 * np.sin(2 * np.pi * (x + 0.1 * v)) for v in range(9)], axis=1)
+    small = Solver(tile, [1.0], NINE, order=1, boundaryTypes="periodic", cfl=0.5)
+    small.run(1e300, max_steps=2)
+    want = small.state()
+    small.close()
+    print("one period done", flush=True)
+    u = np.tile(tile, (n // period, 1))
+    big = Solver(u, [float(n // period)], NINE, order=1, boundaryTypes="periodic", cfl=0.5)
+    assert big.run(1e300, max_steps=2)["steps"] == 2
+    print("2^25 cells done", flush=True)
+    u = big.state()
+    big.close()
+    assert np.isfinite(want).all() and not np.array_equal(want, tile)
+    assert np.array_equal(u.reshape(n // period, period, 9), np.broadcast_to(want, (n // period, period, 9)))
