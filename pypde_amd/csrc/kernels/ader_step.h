@@ -179,23 +179,36 @@ DEV void callS(double* out, const double* q) {
 
 // F is staged in LDS one time node at a time (NTF = 1), except for a viscous
 // F, whose gradient traces need every time node's derivatives, and in the
-// stiff predictor with the plain guess (NTF = N): at two wavefronts per SIMD
-// nothing hides N exchanges one after the other, and all time nodes at once
-// overlap (reactive channel 436 -> 419 us, 219 -> 241 registers; the Picard
-// predictor's time does not change).  The split's cold pass, which is there
-// for its few registers (141, 233 with all at once), stages one at a time.
-constexpr int NTF = PDE_SECOND || (PDE_STIFF && !PDE_GUESS) ? N : 1;
+// stiff predictor with the plain guess where a lane holds few values (NTF =
+// N): at two wavefronts per SIMD nothing hides N exchanges one after the
+// other, and all time nodes at once overlap (reactive channel 436 -> 419 us,
+// 219 -> 241 registers; the Picard predictor's time does not change).  In 2D
+// above N V = 16 the registers that takes cost a wavefront per SIMD or spill
+// (V = 5, order 4: 370 instead of 248; order 6: 253 spills instead of none),
+// us a step, 512 x 256 reactive channel, one at a time against all at once:
+// order 4 811 / 954, order 5 (256 x 128) 635 / 679, order 6 1473 / 1813; eight
+// coupled variables with B at order 4 1103 / 1274.  At N V <= 16 the two lie
+// within 3 % of each other, for the most part in favour of all at once.
+//
+// The split's cold pass, which is there for its few registers (139, 233 with
+// all at once) and its wavefronts, stages one at a time, in LDS of its own size
+// (channel: 8,136 bytes, 15,696 with all at once, which held 10 of the 12
+// wavefronts per compute unit that its registers admit).
+constexpr int NTF =
+    PDE_SECOND || (PDE_STIFF && !PDE_GUESS && (D == 1 || N * V <= 16)) ? N : 1;
+constexpr int NTF_COLD = PDE_SECOND ? N : 1;
+template <int TF>
 struct PredLDS {
 #if PDE_SECOND || PDE_USE_B
   double q[N][CPW][ND][VL];
 #if PDE_USE_F
-  double f[D][NTF][CPW][ND][VL];
+  double f[D][TF][CPW][ND][VL];
 #endif
 #else
   // without PRED_DQ q is staged only after the iterations, over f
   union {
     double q[N][CPW][ND][VL];
-    double f[D][NTF][CPW][ND][VL];
+    double f[D][TF][CPW][ND][VL];
   };
 #endif
 #if PDE_GUESS
@@ -218,7 +231,7 @@ struct PredLDS {
 // [d][side][t][transverse node][d_][v] of trd.  Call with every lane of the
 // wavefront (it synchronises); `on` marks lanes whose cell is done, and
 // sm.q must hold the converged q.
-DEV void grad_traces(const NodeCtx& c, PredLDS& sm, const Geom& g, long cell, bool on,
+DEV void grad_traces(const NodeCtx& c, PredLDS<N>& sm, const Geom& g, long cell, bool on,
                      double* __restrict__ trd) {
   if (on) {
     static_for<0, D>([&](auto dc_) {
@@ -267,8 +280,8 @@ DEV void grad_traces(const NodeCtx& c, PredLDS& sm, const Geom& g, long cell, bo
 // in dqs (zero when no term reads it).  With
 // NTF = 1, F of one time node at a time passes through LDS (two barriers per
 // time node); every (t, v) result is the same either way.
-template <int TF = NTF>
-DEV void node_rhs(const NodeCtx& c, PredLDS& sm, const double (&q)[N][V], const double* w,
+template <int TF>
+DEV void node_rhs(const NodeCtx& c, PredLDS<TF>& sm, const double (&q)[N][V], const double* w,
                   double dt, const Geom& g, bool active, double (&rhs)[N][V],
                   double (&dqs)[N][D][V]) {
   auto eval_f = [&](int t, int slot_t) {
@@ -351,7 +364,8 @@ DEV void node_rhs(const NodeCtx& c, PredLDS& sm, const double (&q)[N][V], const 
 // node: the first iteration from the plain guess).  F, B, S and the spatial
 // derivatives are then the same at every t, so they are evaluated once, at
 // t = 0, and reused; every value equals the one node_rhs computes.
-DEV void node_rhs_const(const NodeCtx& c, PredLDS& sm, const double (&q)[N][V], const double* w,
+template <int TF>
+DEV void node_rhs_const(const NodeCtx& c, PredLDS<TF>& sm, const double (&q)[N][V], const double* w,
                         double dt, const Geom& g, bool active, double (&rhs)[N][V],
                         double (&dqs)[N][D][V]) {
   if (active) {
@@ -637,7 +651,7 @@ DEV bool newton_node(const NodeCtx& c, const double (&q)[N][V], double (&G)[N][V
 // by MODE 1, with the full solve.  Every cell gets the same arithmetic as in
 // MODE 0.
 template <int MODE = 0>
-DEV void predictor_static_body(PredLDS& sm, const double* __restrict__ wh,
+DEV void predictor_static_body(PredLDS<MODE == 1 ? NTF_COLD : NTF>& sm, const double* __restrict__ wh,
                                const double* __restrict__ guess, double* __restrict__ tr,
                                double* __restrict__ vol, double* __restrict__ qh, StepState* st,
                                const Geom& g, double newton_tol, int newton_maxit,
@@ -711,7 +725,7 @@ DEV void predictor_static_body(PredLDS& sm, const double* __restrict__ wh,
     if constexpr (FIRST)
       node_rhs_const(c, sm, q, w, dt, g, active, rhs, dqs);
     else
-      node_rhs<MODE == 1 && !PDE_SECOND ? 1 : NTF>(c, sm, q, w, dt, g, active, rhs, dqs);
+      node_rhs(c, sm, q, w, dt, g, active, rhs, dqs);
     bool more = false;
     bool skip = false;
     trips++;
@@ -951,7 +965,7 @@ k_predictor_static(const double* __restrict__ wh, const double* __restrict__ gue
                    double* __restrict__ tr, double* __restrict__ vol, double* __restrict__ qh,
                    StepState* st, Geom g, double newton_tol, int newton_maxit,
                    double* __restrict__ trd) {
-  __shared__ PredLDS sm;
+  __shared__ PredLDS<NTF> sm;
   predictor_static_body(sm, wh, guess, tr, vol, qh, st, g, newton_tol, newton_maxit, trd,
                         lin_blk());
 }
@@ -965,7 +979,7 @@ k_predictor_cold(const double* __restrict__ wh, double* __restrict__ tr, double*
                  double* __restrict__ qh, StepState* st, Geom g, double newton_tol,
                  int newton_maxit, unsigned int* __restrict__ hot,
                  double* __restrict__ trd) {
-  __shared__ PredLDS sm;
+  __shared__ PredLDS<NTF_COLD> sm;
   predictor_static_body<1>(sm, wh, nullptr, tr, vol, qh, st, g, newton_tol, newton_maxit,
                            trd, lin_blk(), hot);
 }
@@ -977,7 +991,7 @@ k_predictor_cold3(const double* __restrict__ wh, double* __restrict__ tr, double
                   double* __restrict__ qh, StepState* st, Geom g, double newton_tol,
                   int newton_maxit, unsigned int* __restrict__ hot,
                   double* __restrict__ trd) {
-  __shared__ PredLDS sm;
+  __shared__ PredLDS<NTF_COLD> sm;
   predictor_static_body<1>(sm, wh, nullptr, tr, vol, qh, st, g, newton_tol, newton_maxit,
                            trd, lin_blk(), hot);
 }
@@ -986,7 +1000,7 @@ k_predictor_hot(const double* __restrict__ wh, double* __restrict__ tr, double* 
                 double* __restrict__ qh, StepState* st, Geom g, double newton_tol,
                 int newton_maxit, unsigned int* __restrict__ hot,
                 double* __restrict__ trd) {
-  __shared__ PredLDS sm;
+  __shared__ PredLDS<NTF> sm;
   predictor_static_body<2>(sm, wh, nullptr, tr, vol, qh, st, g, newton_tol, newton_maxit,
                            trd, lin_blk(), hot);
 }
@@ -2359,7 +2373,7 @@ k_dt_b(const Member* ms, const BlkMap* map, int nm) {
 extern "C" __global__ void __launch_bounds__(64)
 k_predictor_static_b(const Member* ms, const BlkMap* map, int nm, double newton_tol,
                      int newton_maxit) {
-  __shared__ PredLDS sm;
+  __shared__ PredLDS<NTF> sm;
   PYPDE_BATCH_MEMBER
   predictor_static_body(sm, M.wh, nullptr, M.tr, M.vol, nullptr, M.st, M.g, newton_tol,
                         newton_maxit, M.trd, b);
@@ -2368,7 +2382,7 @@ k_predictor_static_b(const Member* ms, const BlkMap* map, int nm, double newton_
 extern "C" __global__ void __launch_bounds__(64)
 k_predictor_cold_b(const Member* ms, const BlkMap* map, int nm, double newton_tol,
                    int newton_maxit) {
-  __shared__ PredLDS sm;
+  __shared__ PredLDS<NTF_COLD> sm;
   PYPDE_BATCH_MEMBER
   predictor_static_body<1>(sm, M.wh, nullptr, M.tr, M.vol, nullptr, M.st, M.g, newton_tol,
                            newton_maxit, M.trd, b, M.hot);
@@ -2376,7 +2390,7 @@ k_predictor_cold_b(const Member* ms, const BlkMap* map, int nm, double newton_to
 extern "C" __global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(3, 3)))
 k_predictor_cold3_b(const Member* ms, const BlkMap* map, int nm, double newton_tol,
                     int newton_maxit) {
-  __shared__ PredLDS sm;
+  __shared__ PredLDS<NTF_COLD> sm;
   PYPDE_BATCH_MEMBER
   predictor_static_body<1>(sm, M.wh, nullptr, M.tr, M.vol, nullptr, M.st, M.g, newton_tol,
                            newton_maxit, M.trd, b, M.hot);
@@ -2384,7 +2398,7 @@ k_predictor_cold3_b(const Member* ms, const BlkMap* map, int nm, double newton_t
 extern "C" __global__ void __launch_bounds__(64)
 k_predictor_hot_b(const Member* ms, const BlkMap* map, int nm, double newton_tol,
                   int newton_maxit) {
-  __shared__ PredLDS sm;
+  __shared__ PredLDS<NTF> sm;
   PYPDE_BATCH_MEMBER
   predictor_static_body<2>(sm, M.wh, nullptr, M.tr, M.vol, nullptr, M.st, M.g, newton_tol,
                            newton_maxit, M.trd, b, M.hot);
