@@ -960,7 +960,14 @@ DEV void predictor_static_body(PredLDS<MODE == 1 ? NTF_COLD : NTF>& sm, const do
   }
 }
 
+// The Picard kernel at order 5 with four variables needs 258 registers, two past
+// the budget of two wavefronts per SIMD; held to it, it spills two (512 x 512
+// Euler: 1041 -> 724 us).  Up to N V = 20 the budget binds nowhere else; beyond,
+// it costs spills by the dozen (25 at order 6, 46 for a viscous F at order 4)
+// and was the slower build wherever it was tried.
+constexpr int PRED_MIN_WAVES = !PDE_STIFF && !PRED_DQ && N * V <= 20 ? 2 : 1;
 extern "C" __global__ void __launch_bounds__(64)
+__attribute__((amdgpu_waves_per_eu(PRED_MIN_WAVES)))
 k_predictor_static(const double* __restrict__ wh, const double* __restrict__ guess,
                    double* __restrict__ tr, double* __restrict__ vol, double* __restrict__ qh,
                    StepState* st, Geom g, double newton_tol, int newton_maxit,
@@ -2371,6 +2378,7 @@ k_dt_b(const Member* ms, const BlkMap* map, int nm) {
 
 #if PDE_V <= 8
 extern "C" __global__ void __launch_bounds__(64)
+__attribute__((amdgpu_waves_per_eu(PRED_MIN_WAVES)))
 k_predictor_static_b(const Member* ms, const BlkMap* map, int nm, double newton_tol,
                      int newton_maxit) {
   __shared__ PredLDS<NTF> sm;

@@ -13,12 +13,12 @@ from pypde_amd import _capi, systems
 from pypde_amd.solvers import Solver
 
 
-def kernels(tmp_path, monkeypatch, system, N):
-    """{kernel: (registers, spilled, LDS bytes)} of the plain stiff 2D predictor."""
+def kernels(tmp_path, monkeypatch, system, N, stiff=True):
+    """{kernel: (registers, spilled, LDS bytes)} of the plain 2D predictor."""
     monkeypatch.setenv("PYPDE_HIP_CACHE", str(tmp_path))
     s = systems.SYSTEMS[system]
     _capi.compile_only(systems.source(system) + "/* footprint */", s["F"], s["B"], s["S"], 2, N,
-                       s["V"], stiff=True, use_M=s["M"])
+                       s["V"], stiff=stiff, use_M=s["M"])
     out = {}
     for f in tmp_path.glob("*.hsaco"):
         notes = subprocess.run(["/opt/rocm/llvm/bin/llvm-readelf", "--notes", str(f)], check=True,
@@ -42,6 +42,12 @@ def test_footprint_of_the_reactive_predictor(order, tmp_path, monkeypatch):
     assert regs <= 256 and spilled == 0 and lds * 8 <= 160 * 1024
     # twelve wavefronts of the cold pass per compute unit
     assert k["k_predictor_cold"][2] * 12 <= 160 * 1024
+
+
+@pytest.mark.parametrize("system,order", [("euler2d", 5), ("reactive2d", 4)])
+def test_footprint_of_the_picard_predictor(system, order, tmp_path, monkeypatch):
+    regs, spilled, _ = kernels(tmp_path, monkeypatch, system, order, False)["k_predictor_static"]
+    assert regs <= 256 and spilled <= 2   # two wavefronts per SIMD
 
 
 def start(system, ndim):
