@@ -1,10 +1,11 @@
 // Extents of a launch of many workgroups.
 //
-// A launch is refused when gridDim.x * blockDim.x reaches 2^32 (the limit that
-// hip_runtime_api.h states).  With a workgroup of 128 threads per face point
-// a 17-variable grid of 2048 x 2048 cells at order 2 is past it, so workgroups
-// that do not fit in x continue in y; kernels number them x + y gridDim.x
-// (blk_x) and those past the last one, fewer than the grid has rows, find no work.
+// gridDim.x * blockDim.x has to stay below 2^32 (hip_runtime_api.h).  A module
+// launch past it returns success all the same and leaves work out: with 2^25 + 1
+// face points of 128 threads, every cell of the grid came out wrong.  A
+// 17-variable grid of 2048 x 2048 cells at order 2 is past it too, so workgroups
+// that do not fit in x continue in y; kernels number them x + y gridDim.x (blk_x)
+// and those past the last one, fewer than the grid has rows, find no work.
 #pragma once
 
 namespace pypde {
