@@ -31,6 +31,7 @@
 #include "grid.h"
 #include "tables.h"
 #include "transfer.h"
+#include "tune.h"
 
 namespace {
 
@@ -1158,14 +1159,9 @@ int autotune(pypde_ctx* c) {
   c->pred_split = keep_split;
   c->pred_cold3 = keep_c3;
   if (rc) return rc;
-  auto best = [](const double* t, int n) {
-    int b = 0;
-    for (int i = 1; i < n; i++)
-      if (t[i] < t[b]) b = i;
-    return b;
-  };
-  std::vector<int> v = {best(tw, nw), best(tf, nfl), best(tu, N_UPD_V),
-                        c->pred_fixed ? 0 : best(tp, np)};
+  std::vector<int> v = {pypde::fastest(tw, nw), pypde::fastest(tf, nfl),
+                        pypde::fastest(tu, N_UPD_V),
+                        c->pred_fixed ? 0 : pypde::predictor_schedule(tp, np)};
   if (v[3]) v[3]++;  // schedules 2 and 3 are the split's two builds
   apply_tuning(c, v);
   c->tune.source = 1;
