@@ -398,6 +398,7 @@ struct pypde_ctx {
   float* mlp_aux = nullptr;  // ... and its FP32 normalisation and bias vectors
   double* qh = nullptr;     // full predictor output (harvest)
   unsigned long grid_threads = pypde::GRID_THREADS;  // threads of a launch's row of workgroups
+  bool alternating = false;  // 1D steps under way: the state may lie in tmp (settle)
   bool pred_fixed = false;  // schedule fixed by PYPDE_PRED_SCHEDULE (not tuned)
   bool pred_split = false;  // cold pass over every cell, hot pass over the cells it hands on
   bool pred_cold3 = false;  // ... with the cold pass built for three wavefronts per SIMD
@@ -979,8 +980,29 @@ pypde_ctx* pypde_create(const char* src, bool useF, bool useB, bool useS, int* n
                     secondOrder, opts_in, rc_out, false);
 }
 
+// Brings the state of 1D steps, which alternates between u and tmp, back to u.
+// Without effect where the last run already did; after one that failed in
+// between, every entry that reads or replaces the state calls it first.
+static int settle(pypde_ctx* c) {
+  if (!c->alternating) return 0;
+  int flip = 0;
+  HIPCHK(hipMemcpyAsync(&flip, &c->st->flip, sizeof flip, hipMemcpyDeviceToHost, c->stream));
+  HIPCHK(hipStreamSynchronize(c->stream));
+  if (flip) {
+    flip = 0;
+    HIPCHK(hipMemcpyAsync(c->u, c->tmp, c->g.ncell * c->V * sizeof(double),
+                          hipMemcpyDeviceToDevice, c->stream));
+    HIPCHK(hipMemcpyAsync(&c->st->flip, &flip, sizeof flip, hipMemcpyHostToDevice, c->stream));
+    HIPCHK(hipStreamSynchronize(c->stream));
+  }
+  c->host_st.flip = 0;
+  c->alternating = false;
+  return 0;
+}
+
 int pypde_set_state(pypde_ctx* c, const double* u) {
   HIPCHK(hipSetDevice(c->device));
+  if (int r = settle(c)) return r;
   size_t n = c->g.ncell * c->V;
   HIPCHK(pypde::copy_to_device(c->tmp, u, n * sizeof(double), c->device, c->stream));
   std::vector<void*> a = {&c->tmp, &c->u, &c->g.ncell};
@@ -992,6 +1014,7 @@ int pypde_set_state(pypde_ctx* c, const double* u) {
 
 int pypde_get_state(pypde_ctx* c, double* u) {
   HIPCHK(hipSetDevice(c->device));
+  if (int r = settle(c)) return r;
   size_t n = c->g.ncell * c->V;
   std::vector<void*> a = {&c->u, &c->tmp, &c->g.ncell};
   int rc = launch(c, K_S2A, cdiv((long)n, 256), 256, a);
@@ -1236,6 +1259,7 @@ static int run_loop(pypde_ctx* c, long max_steps, pypde_stats* stats, bool first
   // reconstruction it started from)
   const bool next =
       c->fn[K_NEXT] && c->g.nwc <= NEXT_MAX && !graph && !c->opts.profile && !c->qh;
+  c->alternating = next;
   bool primed = false;
   int rc = 0;
   while (true) {
@@ -1256,8 +1280,12 @@ static int run_loop(pypde_ctx* c, long max_steps, pypde_stats* stats, bool first
     if (rc) break;
     const long long count_before = c->host_st.count;
     // (the spread statistics are zero between steps and stay on the device)
-    HIPCHK(pypde::copy_to_host(&c->host_st, c->st, offsetof(StepState, pstat), c->device,
-                               c->stream));
+    const hipError_t e = pypde::copy_to_host(&c->host_st, c->st, offsetof(StepState, pstat),
+                                             c->device, c->stream);
+    if (e != hipSuccess) {
+      rc = fail(PYPDE_ERR_HIP, "step state readback: %s", hipGetErrorString(e));
+      break;
+    }
     if (c->host_st.done) break;
     if (c->host_st.count == count_before) {
       rc = fail(PYPDE_ERR_HIP, "no progress in %d steps", n);
@@ -1266,15 +1294,9 @@ static int run_loop(pypde_ctx* c, long max_steps, pypde_stats* stats, bool first
     if (chunk < 64) chunk *= 2;
   }
   if (exec) (void)hipGraphExecDestroy(exec);
-  if (!rc && c->host_st.flip) {
-    // ended early (a NaN) with the state in the other buffer
-    c->host_st.flip = 0;
-    HIPCHK(hipMemcpyAsync(c->u, c->tmp, c->g.ncell * c->V * sizeof(double),
-                          hipMemcpyDeviceToDevice, c->stream));
-    HIPCHK(hipMemcpyAsync(&c->st->flip, &c->host_st.flip, sizeof(int), hipMemcpyHostToDevice,
-                          c->stream));
-    HIPCHK(hipStreamSynchronize(c->stream));
-  }
+  // a run ends in u, but for a NaN or an error
+  if (!rc && !c->host_st.flip) c->alternating = false;
+  if (int r = settle(c)) rc = rc ? rc : r;
   if (rc) {
     for (auto e : evs) (void)hipEventDestroy(e);
     return rc;
@@ -1312,6 +1334,7 @@ static int run_loop(pypde_ctx* c, long max_steps, pypde_stats* stats, bool first
 
 int pypde_run(pypde_ctx* c, double tf, long max_steps, int ndt, double* ret, pypde_stats* stats) {
   HIPCHK(hipSetDevice(c->device));
+  if (int r = settle(c)) return r;
   if (ndt < 0) return fail(PYPDE_ERR_ARG, "ndt < 0");
   size_t rows = (size_t)ndt;
   size_t row = c->g.ncell * c->V;
@@ -1353,6 +1376,7 @@ int pypde_run(pypde_ctx* c, double tf, long max_steps, int ndt, double* ret, pyp
 
 int pypde_step(pypde_ctx* c, long steps, double tf, pypde_stats* stats) {
   HIPCHK(hipSetDevice(c->device));
+  if (int r = settle(c)) return r;
   HIPCHK(hipMemcpyAsync(&c->host_st, c->st, sizeof(StepState), hipMemcpyDeviceToHost, c->stream));
   HIPCHK(hipStreamSynchronize(c->stream));
   StepState s = c->host_st;
