@@ -92,6 +92,7 @@ hipError_t slice_up(Lane* l, char* dev, const char* host, size_t n, hipStream_t 
       const hipError_t w = hipEventSynchronize(l->ev[k]);
       if (e == hipSuccess) e = w;
     }
+  if (e != hipSuccess) (void)hipStreamSynchronize(s);  // nothing may still read the lane
   return e;
 }
 
