@@ -149,26 +149,38 @@ hipError_t staged(size_t n, int device, Slice slice) {
   return hipSuccess;
 }
 
+// Pinned, managed and device memory, which the runtime copies by itself without
+// staging (and the host may not be able to read).
+bool known_to_runtime(const void* p) {
+  hipPointerAttribute_t a;
+  if (hipPointerGetAttributes(&a, p) == hipSuccess) return a.type != hipMemoryTypeUnregistered;
+  (void)hipGetLastError();
+  return false;
+}
+
+hipError_t direct(void* dst, const void* src, size_t n, hipMemcpyKind kind, hipStream_t s) {
+  const hipError_t e = hipMemcpyAsync(dst, src, n, kind, s);
+  return e == hipSuccess ? hipStreamSynchronize(s) : e;
+}
+
 }  // namespace
 
 hipError_t copy_to_device(void* dev, const void* host, size_t n, int device, hipStream_t s) {
   if (!n) return hipSuccess;
-  hipError_t e = staged(n, device, [&](Lane* l, size_t a, size_t len) {
+  if (known_to_runtime(host)) return direct(dev, host, n, hipMemcpyDefault, s);
+  const hipError_t e = staged(n, device, [&](Lane* l, size_t a, size_t len) {
     return slice_up(l, (char*)dev + a, (const char*)host + a, len, s);
   });
-  if (e != hipErrorOutOfMemory) return e;
-  e = hipMemcpyAsync(dev, host, n, hipMemcpyHostToDevice, s);
-  return e == hipSuccess ? hipStreamSynchronize(s) : e;
+  return e == hipErrorOutOfMemory ? direct(dev, host, n, hipMemcpyHostToDevice, s) : e;
 }
 
 hipError_t copy_to_host(void* host, const void* dev, size_t n, int device, hipStream_t s) {
   if (!n) return hipSuccess;
-  hipError_t e = staged(n, device, [&](Lane* l, size_t a, size_t len) {
+  if (known_to_runtime(host)) return direct(host, dev, n, hipMemcpyDefault, s);
+  const hipError_t e = staged(n, device, [&](Lane* l, size_t a, size_t len) {
     return slice_down(l, (char*)host + a, (const char*)dev + a, len, s);
   });
-  if (e != hipErrorOutOfMemory) return e;
-  e = hipMemcpyAsync(host, dev, n, hipMemcpyDeviceToHost, s);
-  return e == hipSuccess ? hipStreamSynchronize(s) : e;
+  return e == hipErrorOutOfMemory ? direct(host, dev, n, hipMemcpyDeviceToHost, s) : e;
 }
 
 hipError_t take_stream(int device, hipStream_t* s) {

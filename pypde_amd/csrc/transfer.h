@@ -7,7 +7,8 @@
 
 namespace pypde {
 
-// Both return when `host` may be read or reused and the copy has completed;
+// Both return when `host` may be read or reused and the copy has completed.  It
+// may also be pinned, managed or device memory, which is copied without staging;
 // work queued on `stream` before the call is complete too.
 hipError_t copy_to_device(void* dev, const void* host, size_t n, int device, hipStream_t stream);
 hipError_t copy_to_host(void* host, const void* dev, size_t n, int device, hipStream_t stream);

@@ -22,7 +22,7 @@ inline std::deque<Copy> pending;      // one queue for every stream
 inline size_t done = 0;               // copies carried out
 inline std::map<hipEvent_t, size_t> marks;
 inline int records_left = -1;         // hipEventRecord calls until one fails; -1: none does
-inline int host_allocations = 0, live_buffers = 0, host_copies = 0;
+inline int host_allocations = 0, live_buffers = 0;
 inline std::map<const void*, hipMemoryType> known;  // registered with the runtime
 
 inline void run(size_t upto) {
@@ -31,11 +31,6 @@ inline void run(size_t upto) {
     pending.pop_front();
     done++;
   }
-}
-inline bool reads(const void* p, size_t n) {  // a queued copy from [p, p + n)
-  for (auto& c : pending)
-    if ((const char*)c.src >= (const char*)p && (const char*)c.src < (const char*)p + n) return true;
-  return false;
 }
 
 }  // namespace fake

@@ -50,3 +50,23 @@ def test_no_copy_is_in_flight_after_a_failed_event(tmp_path):
     CHECK(fake::pending.empty());
   }
 """)
+
+
+def test_memory_of_the_runtime_is_left_to_it(tmp_path):
+    """Pinned, managed and device memory go to the runtime in one copy; the
+    host touches none of it and allocates no buffer."""
+    run(tmp_path, """
+  const size_t n = (size_t(2) << 20) + 8;
+  std::vector<char> a(n, 7), dev(n), b(n);
+  for (hipMemoryType t : {hipMemoryTypeHost, hipMemoryTypeDevice, hipMemoryTypeManaged}) {
+    std::fill(dev.begin(), dev.end(), 0);
+    std::fill(b.begin(), b.end(), 0);
+    fake::known[a.data()] = t;
+    fake::known[b.data()] = t;
+    const size_t before = fake::done;
+    CHECK(pypde::copy_to_device(dev.data(), a.data(), n, 0, nullptr) == hipSuccess);
+    CHECK(pypde::copy_to_host(b.data(), dev.data(), n, 0, nullptr) == hipSuccess);
+    CHECK(fake::host_allocations == 0 && fake::done == before + 2);
+    CHECK(b == a && fake::pending.empty());
+  }
+""")
