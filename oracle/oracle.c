@@ -1575,7 +1575,8 @@ static void lu_solve_neg(int V, double *P, int n, double h[MAXN][MAXV]) {
     }
     for (int i = V - 1; i >= 0; i--) {
       double acc = b[i];
-      for (int j = i + 1; j < V; j++) acc = fma(-P[i * V + j], b[j], acc);
+      /* b[j] holds x_j = -y_j already */
+      for (int j = i + 1; j < V; j++) acc = fma(P[i * V + j], b[j], acc);
       b[i] = -(acc * rd[i]);
     }
   }

@@ -621,10 +621,10 @@ DEV bool newton_node(const NodeCtx& c, const double (&q)[N][V], double (&G)[N][V
       b[i] = acc;
     }
 #pragma unroll
-    for (int i = V - 1; i >= 0; i--) {
+    for (int i = V - 1; i >= 0; i--) {  // b[j] holds x_j = -y_j already
       double acc = b[i];
 #pragma unroll
-      for (int j = i + 1; j < V; j++) acc = dfma(-P[i * V + j], b[j], acc);
+      for (int j = i + 1; j < V; j++) acc = dfma(P[i * V + j], b[j], acc);
       b[i] = -(acc * rd[i]);
     }
   }

@@ -366,10 +366,10 @@ DEV bool wide_newton(WideGroup& G, const double (&qn)[N], const double (&gt)[N],
   if (l >= V && l < V + N) {
     double x[V];
 #pragma unroll
-    for (int i = V - 1; i >= 0; i--) {
+    for (int i = V - 1; i >= 0; i--) {  // x[j] is -y_j already
       double acc = P[i];
 #pragma unroll
-      for (int j = i + 1; j < V; j++) acc = dfma(-G.A[i][j], x[j], acc);
+      for (int j = i + 1; j < V; j++) acc = dfma(G.A[i][j], x[j], acc);
       x[i] = -(acc * G.row[i]);
     }
 #pragma unroll
