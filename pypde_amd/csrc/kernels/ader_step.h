@@ -2094,11 +2094,12 @@ extern "C" __global__ void k_soa_to_aos(const double* __restrict__ s, double* __
 }
 
 // Reconstruction planes [node * V + v][cell] -> the reference's weno_solver
-// layout [cell][node][v] (api.cpp:32-48): 64 cells per workgroup, through LDS
+// layout [cell][node][v] (api.cpp:32-48), ncell cells of planes `stride` cells
+// long: 64 cells per workgroup, through LDS
 // in slabs of 32 planes, so that reads run along cells and writes along the
 // row.
 extern "C" __global__ void __launch_bounds__(256)
-k_planes_to_rows(const double* __restrict__ s, double* __restrict__ a, long ncell) {
+k_planes_to_rows(const double* __restrict__ s, double* __restrict__ a, long ncell, long stride) {
   constexpr int P = ND * V, SLAB = P < 32 ? P : 32;
   __shared__ double t[SLAB][65];
   const long c0 = (long)blk_x() * 64;
@@ -2106,7 +2107,7 @@ k_planes_to_rows(const double* __restrict__ s, double* __restrict__ a, long ncel
   for (int p0 = 0; p0 < P; p0 += SLAB) {
     const int np = P - p0 < SLAB ? P - p0 : SLAB;
     for (int e = threadIdx.x; e < np * 64; e += 256)
-      if (e % 64 < nc) t[e / 64][e % 64] = s[(long)(p0 + e / 64) * ncell + c0 + e % 64];
+      if (e % 64 < nc) t[e / 64][e % 64] = s[(long)(p0 + e / 64) * stride + c0 + e % 64];
     __syncthreads();
     for (int e = threadIdx.x; e < nc * np; e += 256)
       a[(c0 + e / np) * P + p0 + e % np] = t[e % np][e / np];

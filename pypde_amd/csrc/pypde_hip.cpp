@@ -39,6 +39,7 @@ namespace {
 
 constexpr int MAXV = 17;
 constexpr int P2R_CELLS = 64;  // cells per workgroup of k_planes_to_rows
+constexpr long ROWS_DOUBLES = 1l << 25;  // rows of weno_solver's result formed at once (256 MB)
 constexpr int WIDE_V = 8;  // above this V the kernels of ader_wide.h and ader_wide_predictor.h
 thread_local std::string g_err;
 
@@ -2073,9 +2074,13 @@ int weno_solver(double* ret, double* u, int* nX, int ndim, int N, int V) {
   hipStream_t st0 = rel.stream;
   int ND = 1;
   for (int d = 0; d < ndim; d++) ND *= N;
-  // du holds the input, then the rows of the result
+  // du holds the input, then rows of the result: all of them, or as many as
+  // ROWS_DOUBLES and the input's size allow, so that a result may fill the GPU
+  const long row = (long)ND * V;
+  long span = std::max(std::max(nin * V, ROWS_DOUBLES) / row / P2R_CELLS, 1l) * P2R_CELLS;
+  span = std::min(span, nout);
   double *&du = rel.du, *&dus = rel.dus, *&dw = rel.dw;
-  HIPCHK(hipMalloc((void**)&du, std::max(nin, nout * ND) * V * sizeof(double)));
+  HIPCHK(hipMalloc((void**)&du, std::max(nin * V, span * row) * sizeof(double)));
   HIPCHK(hipMalloc((void**)&dus, nin * V * sizeof(double)));
   HIPCHK(hipMalloc((void**)&dw, nout * ND * V * sizeof(double)));
   HIPCHK(pypde::copy_to_device(du, u, nin * V * sizeof(double), 0, st0));
@@ -2098,12 +2103,14 @@ int weno_solver(double* ret, double* u, int* nX, int ndim, int N, int V) {
     HIPCHK(hipModuleLaunchKernel(fn[K_WENO], gr.x, gr.y, gr.z, 256, 1, 1, 0, st0, a, nullptr));
   }
   // planes [node*V+v][cell] -> reference layout [cell][node][v]
-  {
-    void* a[] = {&dw, &du, &nout};
-    const dim3 gr = lin_grid(cdiv(nout, P2R_CELLS), 256);
+  for (long c0 = 0; c0 < nout; c0 += span) {
+    long n = std::min(span, nout - c0);
+    const double* planes = dw + c0;
+    void* a[] = {&planes, &du, &n, &nout};
+    const dim3 gr = lin_grid(cdiv(n, P2R_CELLS), 256);
     HIPCHK(hipModuleLaunchKernel(fn[K_P2R], gr.x, gr.y, 1, 256, 1, 1, 0, st0, a, nullptr));
+    HIPCHK(pypde::copy_to_host(ret + c0 * row, du, n * row * sizeof(double), 0, st0));
   }
-  HIPCHK(pypde::copy_to_host(ret, du, nout * ND * V * sizeof(double), 0, st0));
   return 0;
 }
 
@@ -2208,7 +2215,7 @@ int weno_solver_noalloc(pypde_ctx* c, double* ret, const double* u, const int* n
     if ((rc = go(K_WENO, gx, gy, gz, a))) return rc;
   }
   {
-    void* a[] = {&s_out, &ret, &nout};
+    void* a[] = {&s_out, &ret, &nout, &nout};
     if ((rc = go(K_P2R, (unsigned)cdiv(nout, P2R_CELLS), 1, 1, a))) return rc;
   }
   if (!stream) HIPCHK(hipStreamSynchronize(s));
