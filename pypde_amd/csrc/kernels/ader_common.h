@@ -192,7 +192,7 @@ DEV bool house(const double* x, double* v, double* beta) {
     const double mu2 = dfma(x[0], x[0], sigma);
     double v0;
     if (mu2 <= 0x1p60) {
-      // sigma > 2^-900: the divisors lie in 2^-900 .. 2^62, sigma / (x0 + mu) above 2^-932
+      // sigma > 2^-900: the divisors lie in 2^-900 .. 2^63, sigma / (x0 + mu) above 2^-932
       const double mu = sqrt_mid(mu2);
       v0 = (x[0] <= 0.0) ? x[0] - mu : -div_mid(sigma, x[0] + mu);
       *beta = 2.0 * recip_mid(dfma(v0, v0, sigma));
@@ -229,7 +229,8 @@ DEV bool house1(const double* x, double* v, double* beta, double* mu_out) {
     const bool pos = x[0] > 0.0;
     double mu, s, r;
     if (mu2 <= 0x1p400) {
-      // sigma > 2^-500: the divisor lies in 2^-1000 .. 2^602, beta > 0
+      // sigma > 2^-500 and sigma <= mu^2, s <= 2 mu: the divisor lies in 2^-1000 ..
+      // 2^801, beta > 0
       mu = sqrt_mid(mu2);
       s = x[0] + mu;
       r = recip_mid(pos ? (s * mu) * sigma : mu * (mu - x[0]));
