@@ -149,9 +149,21 @@ def make_options(newton_tol=1e-12, newton_maxit=100, max_steps=0, reflect=None, 
 
 
 def compile_only(src, useF, useB, useS, ndim, N, V, stiff=False, use_M=False, b_quirk=0, flux=0,
-                 second=False, mixed=False, ensemble=False):
+                 second=False, mixed=False, ensemble=False, large=False):
     """Compile (or fetch from the code-object cache) without a GPU; ensemble =
-    True gives the code object of ensemble members (with the batched kernels)."""
+    True gives the code object of ensemble members (with the batched kernels),
+    large = True the one that large grids take above eight variables."""
+    if large and V > 8:
+        before = os.environ.get("PYPDE_WIDE")
+        os.environ["PYPDE_WIDE"] = "0"
+        try:
+            return compile_only(src, useF, useB, useS, ndim, N, V, stiff, use_M, b_quirk, flux,
+                                second, mixed, ensemble)
+        finally:
+            if before is None:
+                del os.environ["PYPDE_WIDE"]
+            else:
+                os.environ["PYPDE_WIDE"] = before
     o = make_options(use_M=use_M, b_quirk=b_quirk, mixed=mixed)
     fn = lib().pypde_hip_compile_ensemble if ensemble else lib().pypde_hip_compile
     rc = fn(src.encode(), useF, useB, useS, ndim, N, V, stiff, int(flux), bool(second), C.byref(o))

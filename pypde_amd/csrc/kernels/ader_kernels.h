@@ -39,7 +39,7 @@ struct Geom {
 // complete), and what a face point reads of a block, its V variables, lies in
 // the same lines (2048 x 2048 at order 2, predictor 848 -> 729 us: it writes
 // 2.1 GB of traces, which is what bounds it).
-constexpr int TCW = V > 8 ? 1 : 64 / ND;
+constexpr int TCW = PDE_WIDE_PRED ? 1 : 64 / ND;
 DEV long trace_at(const Geom& g, int plane, long block, int slot) {
   return ((long)plane * g.ntb + block) * (V * TCW) + slot;  // + v * TCW
 }
@@ -341,9 +341,9 @@ constexpr bool DT_PAIR = (D == 2) && (V <= 5) && !PDE_SECOND;
 // much as a whole first-order cell: a wavefront takes one of them for 64
 // cells and the sums go through LDS (64 x 64 cells, 69 wavefronts one after
 // the other's problems otherwise: 22 -> 10.4 us).
-constexpr int DT_LANES = V > 8 ? 64 : PDE_SECOND ? 2 * D : DT_PAIR ? 2 : 1;
+constexpr int DT_LANES = PDE_WIDE_EIG ? 64 : PDE_SECOND ? 2 * D : DT_PAIR ? 2 : 1;
 
-#if PDE_V > 8
+#if PDE_WIDE_EIG
 // One wavefront per w-cell: the cell's mean (lane v takes variable v), then
 // one eigenvalue problem per direction over the wavefront.
 DEV void dt_body(const double* __restrict__ wh, const double* __restrict__ wm, StepState* st,
@@ -496,7 +496,7 @@ DEV void dt_finalize(StepState* st) {
 extern "C" __global__ void __launch_bounds__(256)
 k_eig_batch(const double* __restrict__ A, const double* __restrict__ x, double* __restrict__ out,
             long n, int which) {
-#if PDE_V > 8
+#if PDE_WIDE_EIG
   // a workgroup's 256 matrices, 64 in turn per wavefront (which is 0: Roe and
   // Osher stop at V = 8)
   __shared__ WideMat mats[WIDE_WAVES];

@@ -632,7 +632,7 @@ DEV bool newton_node(const NodeCtx& c, const double (&q)[N][V], double (&G)[N][V
 }
 #endif
 
-#if PDE_V <= 8  // above, ader_wide_predictor.h
+#if !PDE_WIDE_PRED  // else ader_wide_predictor.h
 // The space-time DG predictor over all reconstructed cells (dg.cpp:204-224):
 // initial guess (dg.cpp:12-20, 156-171), Picard (dg.cpp:187-202) or the
 // per-node stiff Newton in place of the reference's Newton-Krylov
@@ -1013,7 +1013,7 @@ k_predictor_hot(const double* __restrict__ wh, double* __restrict__ tr, double* 
 }
 #endif
 
-#endif  // PDE_V <= 8
+#endif  // !PDE_WIDE_PRED
 
 #if PDE_MIXED
 // ---------------------------------------------- mixed precision: FP32 phase
@@ -1261,8 +1261,8 @@ DEV void face_cells(const Geom& g, long f, long* wl, long* wr) {
   }
 }
 
-#if PDE_V > 8
-// Above V = 8 (Rusanov, first-order F): one face point per workgroup of two
+#if PDE_WIDE_EIG
+// Above V = 8 on small grids (Rusanov, first-order F): one face point per workgroup of two
 // wavefronts, one for each side's wave speed and F.
 template <int d>
 DEV void flux_wide(const double* __restrict__ tr, double* __restrict__ ff, double* __restrict__ fb,
@@ -1336,7 +1336,7 @@ DEV void flux_wide(const double* __restrict__ tr, double* __restrict__ ff, doubl
   }
 #endif
 }
-#else  // PDE_V <= 8
+#else  // !PDE_WIDE_EIG
 // Face f, time node t and transverse node j of flux item `item` of direction
 // d, and its two w-cells; false past the last item.
 struct FaceItem {
@@ -1630,7 +1630,7 @@ DEV void flux_split(FluxShared& sm, const double* __restrict__ tr, double* __res
 #else
 constexpr int FLUX_SPLIT = 1;
 #endif
-#endif  // PDE_V <= 8
+#endif  // !PDE_WIDE_EIG
 
 // Every direction's faces in one launch: the workgroups of direction 0, then
 // those of direction 1 (flux_blocks on the host); one nearly empty last round
@@ -1642,10 +1642,10 @@ constexpr int FLUX_SPLIT = 1;
 template <int MODE, int BS>
 DEV void flux_all(const double* __restrict__ tr, const FaceOut& out, const Geom& g,
                   const double* __restrict__ trd, const int* done, const Blk& b) {
-  constexpr int POINTS = V > 8 ? 1 : MODE ? 64 : BS;
+  constexpr int POINTS = PDE_WIDE_EIG ? 1 : MODE ? 64 : BS;
   const unsigned int nb0 =
       D == 1 ? ~0u : (unsigned int)((g.nf[0] * (N * ND1) + POINTS - 1) / POINTS);
-#if PDE_V > 8
+#if PDE_WIDE_EIG
   (void)trd;
   if (*done) return;
   if (b.x < nb0) flux_wide<0>(tr, out.ff[0], out.fb[0], g, b.x);
@@ -1670,7 +1670,8 @@ DEV void flux_all(const double* __restrict__ tr, const FaceOut& out, const Geom&
 #endif
 }
 
-// k_flux: 128 threads (one face point each; above V = 8 one point together),
+// k_flux: 128 threads, one face point each; above V = 8 one point together, or on
+// large grids 64 threads, one point each.
 // k_flux_64: 64 threads, k_flux_split: FLUX_SPLIT wavefronts per 64 points.
 // The autotuner picks one per problem; every face point's arithmetic is the
 // same.
@@ -1680,7 +1681,8 @@ DEV void flux_all(const double* __restrict__ tr, const FaceOut& out, const Geom&
        const double* __restrict__ trd) {                                                       \
     flux_all<MODE, BS>(tr, out, g, trd, &st->done, lin_blk());                                  \
   }
-PYPDE_FLUX_KERNEL(k_flux, 0, 128)
+constexpr int FLUX_BS = V > 8 && !PDE_WIDE_EIG ? 64 : 128;
+PYPDE_FLUX_KERNEL(k_flux, 0, FLUX_BS)
 #if PDE_V <= 8
 PYPDE_FLUX_KERNEL(k_flux_64, 0, 64)
 PYPDE_FLUX_KERNEL(k_flux_split, 1, 64 * FLUX_SPLIT)
@@ -2377,7 +2379,7 @@ k_dt_b(const Member* ms, const BlkMap* map, int nm) {
   dt_body(M.wh, M.tr, M.st, M.g, b);
 }
 
-#if PDE_V <= 8
+#if !PDE_WIDE_PRED
 extern "C" __global__ void __launch_bounds__(64)
 __attribute__((amdgpu_waves_per_eu(PRED_MIN_WAVES)))
 k_predictor_static_b(const Member* ms, const BlkMap* map, int nm, double newton_tol,
@@ -2414,7 +2416,7 @@ k_predictor_hot_b(const Member* ms, const BlkMap* map, int nm, double newton_tol
 }
 
 #endif
-#endif  // PDE_V <= 8
+#endif  // !PDE_WIDE_PRED
 
 #define PYPDE_FLUX_BATCH(NAME, MODE, BS)                                                       \
   extern "C" __global__ void __launch_bounds__(BS)                                             \
@@ -2423,7 +2425,7 @@ k_predictor_hot_b(const Member* ms, const BlkMap* map, int nm, double newton_tol
     const FaceOut out = {{M.ff[0], M.ff[1]}, {M.fb[0], M.fb[1]}};                              \
     flux_all<MODE, BS>(M.tr, out, M.g, M.trd, &M.st->done, b);                                 \
   }
-PYPDE_FLUX_BATCH(k_flux_b, 0, 128)
+PYPDE_FLUX_BATCH(k_flux_b, 0, FLUX_BS)
 #if PDE_V <= 8
 PYPDE_FLUX_BATCH(k_flux_64_b, 0, 64)
 PYPDE_FLUX_BATCH(k_flux_split_b, 1, 64 * FLUX_SPLIT)

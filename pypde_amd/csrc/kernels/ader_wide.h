@@ -1,10 +1,12 @@
-// Wave speeds of systems with more than eight variables, one wavefront per
-// matrix.  Compiled by hipRTC after ader_common.h, for PDE_V > 8 only.
+// Wave speeds of systems with more than eight variables on small grids, one
+// wavefront per matrix.  Compiled by hipRTC after ader_common.h where
+// PDE_WIDE_EIG (or, for the helpers, PDE_WIDE_PRED) is 1.
 //
-// One lane per matrix (as for V <= 8) does not fit here: a 17 x 17 matrix and
-// its reduction need some 600 registers, so they lived in scratch (4-8 KB per
-// lane), and a 200-cell line has only 402 face points, seven wavefronts on
-// the whole GPU, each a serial chain of spilled accesses.  Here the matrix
+// One lane per matrix, which larger grids take (wide_matrices in tune.h gives the
+// line), leaves a small grid waiting: a 17 x 17 matrix and its reduction need
+// some 600 registers, so they live in scratch (4-8 KB per lane), and a 200-cell
+// line has only 402 face points, seven wavefronts on the whole GPU, each a serial
+// chain of spilled accesses.  Here the matrix
 // lies in LDS, lane j works on column j (left products, Jacobian columns) or
 // row j (right products), and scalars are formed by every lane alike.  What
 // bounds it is the latency of the dependent chains (Householder sums, Horner

@@ -1,7 +1,8 @@
 // Space-time predictor of systems with more than eight variables, one
-// wavefront per cell.  Compiled by hipRTC after ader_step.h, for PDE_V > 8 only.
+// wavefront per cell.  Compiled by hipRTC after ader_step.h where PDE_WIDE_PRED
+// is 1: on small grids, and for stiff systems of 14 variables and more on all.
 //
-// With one lane per spatial node (V <= 8) the 17-variable stiff Newton step
+// With one lane per spatial node the 17-variable stiff Newton step
 // holds three 17 x 17 matrices per lane, 10,000 spilled registers, and 202
 // cells of two nodes fill seven wavefronts.  Here a cell's iterate lies in
 // LDS: F and S run with one lane per space-time node, everything elementwise

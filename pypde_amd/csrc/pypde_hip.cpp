@@ -40,7 +40,7 @@ namespace {
 constexpr int MAXV = 17;
 constexpr int P2R_CELLS = 64;  // cells per workgroup of k_planes_to_rows
 constexpr long ROWS_DOUBLES = 1l << 25;  // rows of weno_solver's result formed at once (256 MB)
-constexpr int WIDE_V = 8;  // above this V the kernels of ader_wide.h and ader_wide_predictor.h
+constexpr int WIDE_V = 8;  // above this V a wavefront may share a matrix or a cell (Spec::wide)
 thread_local std::string g_err;
 
 int fail(int code, const char* fmt, ...) {
@@ -161,6 +161,14 @@ struct Spec {
   bool second = false;  // F depends on the gradient (viscous, secondOrder)
   bool mixed = false;   // FP32 predictor phase before the FP64 one
   bool batch = false;   // also the batched ensemble kernels (one launch per stage)
+  // V > WIDE_V: one wavefront per matrix (ader_wide.h) instead of one lane, for
+  // grids of few matrices (wide_matrices in tune.h)
+  bool wide = false;
+  // ... and per cell in the predictor (ader_wide_predictor.h), on large grids too
+  // for a stiff one whose three V x V matrices a lane cannot hold: 200,000 cells, 1D
+  // order 2, wavefront against lane, in ms: V = 9 1.22 / 0.18, 12 1.86 / 1.22, 14
+  // 2.34 / 2.52, 17 3.56 / 9.23
+  bool wide_pred() const { return wide || (V >= 14 && stiff); }
 };
 
 std::string full_source(const Spec& s, const pypde::Tables& T) {
@@ -174,6 +182,8 @@ std::string full_source(const Spec& s, const pypde::Tables& T) {
   o << "#define PDE_GUESS " << (int)s.guess << "\n#define PDE_FLUX " << s.flux << "\n";
   o << "#define PDE_SECOND " << (int)s.second << "\n#define PDE_MIXED " << (int)s.mixed << "\n";
   o << "#define PDE_BATCH " << (int)s.batch << "\n";
+  o << "#define PDE_WIDE_EIG " << (int)s.wide << "\n#define PDE_WIDE_PRED " << (int)s.wide_pred()
+    << "\n";
   o << "constexpr int ipow_c(int b, int e) { return e <= 0 ? 1 : b * ipow_c(b, e - 1); }\n";
   o << pypde::tables_source(T, s.D);
   o << PRELUDE_SRC << "\n";
@@ -182,9 +192,9 @@ std::string full_source(const Spec& s, const pypde::Tables& T) {
   if (s.mixed)  // the same physics once more, in FP32, for the mixed predictor's first phase
     o << REAL32_SRC << "\nnamespace f32 {\n#define double R\n#line 1 \"system (FP32)\"\n" << s.src
       << "\n#undef double\n}  // namespace f32\n";
-  if (s.V > WIDE_V) o << WIDE_SRC << "\n";
+  if (s.wide_pred()) o << WIDE_SRC << "\n";
   o << KERNELS_SRC << "\n" << STEP_SRC << "\n";
-  if (s.V > WIDE_V) o << WIDE_PRED_SRC << "\n";
+  if (s.wide_pred()) o << WIDE_PRED_SRC << "\n";
   return o.str();
 }
 
@@ -461,7 +471,8 @@ void release_module(int device, hipModule_t mod) {
 std::string spec_id(const Spec& s) {
   std::ostringstream o;
   o << s.D << ' ' << s.N << ' ' << s.V << ' ' << s.useF << s.useB << s.useS << s.useM << s.stiff
-    << s.guess << s.second << s.mixed << s.batch << ' ' << s.b_quirk << ' ' << s.flux << '\n'
+    << s.guess << s.second << s.mixed << s.batch << s.wide << ' ' << s.b_quirk << ' ' << s.flux
+    << '\n'
     << s.src;
   return o.str();
 }
@@ -544,17 +555,18 @@ int launch(pypde_ctx* c, int k, long blocks, int threads, std::vector<void*>& ar
 
 long cdiv(long a, long b) { return (a + b - 1) / b; }
 
-// Face-flux launches (FLUX_SPLIT and flux_all in ader_step.h): variants,
+// Face-flux launches (FLUX_SPLIT, FLUX_BS and flux_all in ader_step.h): variants,
 // threads per workgroup, and workgroups over every direction's faces.
 int flux_variants(int V) { return V > WIDE_V ? 1 : N_FLUX_V; }
 int flux_threads(const Spec& s, int variant) {
-  if (s.V > WIDE_V || variant == 0) return 128;
+  if (s.V > WIDE_V) return s.wide ? 128 : 64;
+  if (variant == 0) return 128;
   if (variant == 1) return 64;
   const int parts = !s.useF ? 1 : s.flux == 0 ? 2 : s.flux == 1 ? 1 : s.N;
   return 64 * (parts + (s.useF && s.second ? 2 : 0));
 }
 long flux_blocks(const Spec& s, int variant, const Geom& g) {
-  const long points = s.V > WIDE_V ? 1 : variant == 0 ? 128 : 64;
+  const long points = s.wide ? 1 : s.V <= WIDE_V && variant == 0 ? 128 : 64;
   long blocks = 0;
   for (int d = 0; d < s.D; d++) {
     const long items = g.nf[d] * s.N * (s.D == 2 ? s.N : 1);
@@ -704,6 +716,28 @@ int enqueue_step(pypde_ctx* c, bool guess_now, std::vector<hipEvent_t>* evs, boo
   return 0;
 }
 
+// Whether systems of V variables run one wavefront per matrix where a face-flux
+// launch takes `matrices` of them.  PYPDE_WIDE=0 or 1 says so for any grid.
+bool wide_form(int V, double matrices) {
+  if (V <= WIDE_V) return false;
+  if (const char* e = getenv("PYPDE_WIDE"))
+    if (*e) return *e != '0';
+  return matrices <= (double)pypde::wide_matrices(V);
+}
+
+// Matrices of a grid's face-flux launch: two per face point.
+double flux_matrices(const int* nX, int ndim, int N) {
+  double points = 0.0, nodes = N;
+  for (int d = 0; d < ndim; d++) {
+    double faces = nX[d] + 1.0;
+    for (int e = 0; e < ndim; e++)
+      if (e != d) faces *= nX[e];
+    points += faces;
+    if (d > 0) nodes *= N;
+  }
+  return 2.0 * points * nodes;
+}
+
 int make_spec(Spec* s, const char* src, bool useF, bool useB, bool useS, int ndim, int N, int V,
               bool STIFF, const pypde_options* o) {
   s->src = src ? src : "";
@@ -771,6 +805,7 @@ int pypde_hip_compile(const char* src, bool useF, bool useB, bool useS, int ndim
   s.mixed = opts && (size_t)opts->struct_size >= offsetof(pypde_options, mixed_maxit) + sizeof(int) &&
             opts->mixed;
   s.guess = s.mixed;
+  s.wide = wide_form(V, 0.0);
   int rc = check_spec(s, secondOrder, FLUX);
   if (rc) return rc;
   std::vector<char> code;
@@ -791,6 +826,7 @@ int pypde_hip_compile_ensemble(const char* src, bool useF, bool useB, bool useS,
   s.flux = FLUX;
   s.second = secondOrder;
   s.batch = true;
+  s.wide = wide_form(V, 0.0);
   int rc = check_spec(s, secondOrder, FLUX);
   if (rc) return rc;
   std::vector<char> code;
@@ -822,7 +858,8 @@ void pypde_destroy(pypde_ctx* c) {
 static pypde_ctx* create_ctx(const char* src, bool useF, bool useB, bool useS, const int* nX,
                              int ndim, const double* dX, double CFL, const int* boundaryTypes,
                              bool STIFF, int FLUX, int N, int V, bool secondOrder,
-                             const pypde_options* opts_in, int* rc_out, bool batch) {
+                             const pypde_options* opts_in, int* rc_out, bool batch,
+                             double matrices = -1.0) {
   int dummy;
   int& rc = rc_out ? *rc_out : dummy;
   pypde_options opts;
@@ -869,6 +906,7 @@ static pypde_ctx* create_ctx(const char* src, bool useF, bool useB, bool useS, c
       return nullptr;
     }
   }
+  s.wide = wide_form(V, matrices >= 0.0 ? matrices : flux_matrices(nX, ndim, N));
   pypde_ctx* c = new pypde_ctx();
   c->spec = s;
   c->opts = opts;
@@ -878,15 +916,15 @@ static pypde_ctx* create_ctx(const char* src, bool useF, bool useB, bool useS, c
   c->ND = 1;
   for (int d = 0; d < ndim; d++) c->ND *= N;
   c->NT = c->ND * N;
-  c->CPW = V > WIDE_V ? 1 : 64 / c->ND;
+  c->CPW = s.wide_pred() ? 1 : 64 / c->ND;
   // DT_LANES in ader_kernels.h
-  c->dt_lanes = V > WIDE_V ? 64 : secondOrder ? 2 * ndim : (ndim == 2 && V <= 5) ? 2 : 1;
+  c->dt_lanes = s.wide ? 64 : secondOrder ? 2 * ndim : (ndim == 2 && V <= 5) ? 2 : 1;
   c->device = opts.device;
   // Predictor schedule: the autotuner weighs the stiff cold/hot split against
   // one kernel; PYPDE_PRED_SCHEDULE ("split", or any other name for the one
-  // kernel) fixes it.  Above WIDE_V there is one predictor kernel.
+  // kernel) fixes it.  One wavefront per cell leaves one predictor kernel.
   if (const char* e = getenv("PYPDE_PRED_SCHEDULE")) {
-    c->pred_split = strcmp(e, "split") == 0 && V <= WIDE_V;
+    c->pred_split = strcmp(e, "split") == 0 && !s.wide_pred();
     c->pred_fixed = true;
   }
   Geom& g = c->g;
@@ -1640,13 +1678,16 @@ pypde_ensemble* pypde_ensemble_create(int n, const char* src, bool useF, bool us
     rc = fail(PYPDE_ERR_ARG, "ensemble: per-member guesses are not supported");
     return nullptr;
   }
+  // all members run the same kernels, side by side: their matrices count together
+  double matrices = 0.0;
+  for (int i = 0; i < n; i++) matrices += flux_matrices(nX + i * ndim, ndim, N);
   auto* e = new pypde_ensemble();
   for (int i = 0; i < n; i++) {
     int nx[2] = {nX[i * ndim], ndim > 1 ? nX[i * ndim + 1] : 1};
     double dx[2] = {dX[i * ndim], ndim > 1 ? dX[i * ndim + 1] : 1.0};
     int bc[2] = {boundaryTypes[0], ndim > 1 ? boundaryTypes[1] : 0};
     pypde_ctx* c = create_ctx(src, useF, useB, useS, nx, ndim, dx, CFL, bc, STIFF, FLUX, N, V,
-                              secondOrder, opts, &rc, true);
+                              secondOrder, opts, &rc, true, matrices);
     if (!c) {
       pypde_ensemble_destroy(e);
       return nullptr;
@@ -2039,6 +2080,7 @@ int pypde_mlp_adam(float* w, const float* g, float* m, float* v, long n, float l
 int weno_solver(double* ret, double* u, int* nX, int ndim, int N, int V) {
   Spec s;
   make_spec(&s, "", false, false, false, ndim, N, V, false, nullptr);
+  s.wide = V > WIDE_V;  // (only the reconstruction runs: the form that compiles faster)
   int rc = check_spec(s, false, 0);
   if (rc) return rc;
   long nin = 1, nout = 1;

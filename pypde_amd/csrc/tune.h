@@ -21,4 +21,21 @@ inline int predictor_schedule(const double* ms, int n) {
   return b > 0 && ms[b] < 0.95 * ms[0] ? b : 0;
 }
 
+// The most V x V matrices (V > 8) in a face-flux launch, two per face point, up to
+// which one wavefront per matrix is the faster form; above, one lane per matrix.
+// A wavefront hides the latency of a lane's chain but works for one matrix, 20
+// ns each at V = 9 and 77 at 17; lanes take as long for one wavefront's 64 matrices
+// as for a GPU full of them.  Measured, 1D order 2, us of wavefront / lane:
+//   V = 9   8,000 matrices  221 / 230      80,000   1659 / 232      800,000  16070 / 982
+//   V = 10  8,000           261 / 232      80,000   1930 / 244
+//   V = 12  8,000           376 / 531      80,000   3094 / 545      800,000  30184 / 2653
+//   V = 14  8,000           446 / 1200     80,000   3746 / 1339     800,000  36301 / 8299
+//   V = 17  8,000           754 / 2681     80,000   6322 / 3762     800,000  61787 / 23939
+//   V = 17 (GPR)            80,000  1938-2847 / 1893-2944           400,000  9166-13870 / 5254-10952
+// At 17 variables a lane's matrix lies in scratch and the lane form takes minutes to
+// compile, so the line stays where the GPR model has it.
+inline long wide_matrices(int V) {
+  return V <= 11 ? 9000 : V <= 13 ? 14000 : V <= 15 ? 27000 : 90000;
+}
+
 }  // namespace pypde

@@ -85,6 +85,10 @@ def standard_configs(full=False):
         s = SYSTEMS["gpr"]
         out.append(dict(src=source("gpr"), useF=True, useB=True, useS=True, ndim=ndim, N=N, V=17,
                         stiff=stiff, use_M=False, flux=0, b_quirk=quirk, ensemble=ens))
+    # ... and the kernels that its large grids take (over a minute to compile)
+    if full:
+        out.append(dict(src=source("gpr"), useF=True, useB=True, useS=True, ndim=1, N=2, V=17,
+                        stiff=False, use_M=False, flux=0, b_quirk=1, large=True))
     return out
 
 
