@@ -2,10 +2,11 @@
 //
 // gridDim.x * blockDim.x has to stay below 2^32 (hip_runtime_api.h).  A module
 // launch past it returns success all the same and leaves work out: with 2^25 + 1
-// face points of 128 threads, every cell of the grid came out wrong.  A
-// 17-variable grid of 2048 x 2048 cells at order 2 is past it too, so workgroups
-// that do not fit in x continue in y; kernels number them x + y gridDim.x (blk_x)
-// and those past the last one, fewer than the grid has rows, find no work.
+// face points of 128 threads (nine variables, one wavefront per matrix), every cell
+// of the grid came out wrong.  Variants that give a point or a cell several
+// threads come near it on grids that fit the GPU, so workgroups that do not fit in
+// x continue in y; kernels number them x + y gridDim.x (blk_x) and those past the
+// last one, fewer than the grid has rows, find no work.
 #pragma once
 
 namespace pypde {

@@ -125,6 +125,7 @@ def test_face_points_past_the_limit_of_one_row(monkeypatch):
     threads.  The field repeats every 1024 cells, so each period equals a run
     of one."""
     monkeypatch.setenv("PYPDE_TUNE", "0")
+    monkeypatch.setenv("PYPDE_WIDE", "1")    # the form with 128 threads per face point
     period, n = 1024, 2 ** 25
     x = (np.arange(period) + 0.5) / period
     tile = np.stack([1.0 + 0.2 * np.sin(2 * np.pi * (x + 0.1 * v)) for v in range(9)], axis=1)
