@@ -118,8 +118,8 @@ int weno_solver_noalloc(pypde_ctx *c, double *ret, const double *u, const int *n
 pypde_ctx *pypde_create(const char *src, bool useF, bool useB, bool useS, int *nX, int ndim,
                         double *dX, double CFL, int *boundaryTypes, bool STIFF, int FLUX, int N,
                         int V, bool secondOrder, const pypde_options *opts, int *rc);
-int pypde_set_state(pypde_ctx *c, const double *u);          /* host, row-major */
-int pypde_get_state(pypde_ctx *c, double *u);                /* host, row-major */
+int pypde_set_state(pypde_ctx *c, const double *u);          /* row-major; host, pinned or device */
+int pypde_get_state(pypde_ctx *c, double *u);                /* the same */
 /* Advance from t = 0 until tf or max_steps; ndt snapshot rows into ret (may be
  * NULL when ndt == 0).  Device state stays resident between calls. */
 int pypde_run(pypde_ctx *c, double tf, long max_steps, int ndt, double *ret, pypde_stats *stats);
@@ -226,7 +226,9 @@ void pypde_release_idle(void);
 int pypde_device_count(void);
 
 /* Compile (or fetch from the code-object cache) without touching a GPU; FLUX and
- * secondOrder as in pde_solver_hip. */
+ * secondOrder as in pde_solver_hip.  Above eight variables small and large grids
+ * run code objects of their own (wide_matrices in csrc/tune.h): this compiles the
+ * small ones', and with PYPDE_WIDE=0 in the environment the large ones'. */
 int pypde_hip_compile(const char *src, bool useF, bool useB, bool useS, int ndim, int N, int V,
                       bool STIFF, int FLUX, bool secondOrder, const pypde_options *opts);
 /* The same for the code object of ensemble members, which also holds the batched

@@ -711,7 +711,7 @@ DEV void predictor_static_body(PredLDS<MODE == 1 ? NTF_COLD : NTF>& sm, const do
   // from the plain guess, whose iterate is constant in time (the wave-uniform
   // q = w), so the right-hand side needs F, S and the derivatives once.  It is
   // peeled off the loop so that the loop holds one right-hand side only
-  // (the stiff cold pass, 141 registers for the reactive channel, needed 26
+  // (the stiff cold pass, 139 registers for the reactive channel, needed 26
   // more with both).
   auto iterate = [&](auto firstc) {
     constexpr bool FIRST = decltype(firstc)::value;

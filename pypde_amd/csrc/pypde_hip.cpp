@@ -353,7 +353,7 @@ const char* kernel_names[K_COUNT] = {"k_weno",   "k_dt",
 // mappings (one thread per cell and all variables, or one variable and R
 // x-rows per thread), predictor schedules (0 one kernel; for the stiff
 // predictor with the plain guess 2, 3 the cold/hot split, its cold pass built
-// for two or for three wavefronts per SIMD; 1 is not used).
+// for two or for three wavefronts per SIMD).
 constexpr int N_WENO_V = 4, N_FLUX_V = 3, N_UPD_V = 5, N_PRED_V = 4;
 const int WENO_TILE[N_WENO_V][2] = {{8, 32}, {4, 64}, {16, 16}, {16, 32}};
 // Cells per workgroup of the 1D reconstruction (the kernels' WENO1_W).
