@@ -187,15 +187,16 @@ DEV void callS(double* out, const double* q) {
 // (V = 5, order 4: 370 instead of 248; order 6: 253 spills instead of none),
 // us a step, 512 x 256 reactive channel, one at a time against all at once:
 // order 4 811 / 954, order 5 (256 x 128) 635 / 679, order 6 1473 / 1813; eight
-// coupled variables with B at order 4 1103 / 1274.  At N V <= 16 the two lie
-// within 3 % of each other, for the most part in favour of all at once.
+// coupled variables with B at order 4 1103 / 1274.  At N V <= 16, and in 1D up to
+// V = 8, the two lie within 4 % of each other, for the most part in favour of all
+// at once; 1D above V = 8 (lane form) 12 variables with B at order 4 7951 / 8680.
 //
 // The split's cold pass, which is there for its few registers (139, 233 with
 // all at once) and its wavefronts, stages one at a time, in LDS of its own size
 // (channel: 8,136 bytes, 15,696 with all at once, which held 10 of the 12
 // wavefronts per compute unit that its registers admit).
 constexpr int NTF =
-    PDE_SECOND || (PDE_STIFF && !PDE_GUESS && (D == 1 || N * V <= 16)) ? N : 1;
+    PDE_SECOND || (PDE_STIFF && !PDE_GUESS && ((D == 1 && V <= 8) || N * V <= 16)) ? N : 1;
 constexpr int NTF_COLD = PDE_SECOND ? N : 1;
 template <int TF>
 struct PredLDS {
